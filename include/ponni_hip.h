@@ -417,6 +417,10 @@ int64_t ponni_plan_program_source(ponni_plan plan, char* buf, int64_t len);
 /* Compile a FUSED plan's kernel with hipRTC now (no device needed; the result
  * is cached in-process and under $PONNI_JIT_CACHE or ~/.cache/ponni_hip) so the
  * first ponni_forward does not pay for it.  A no-op for the other paths.
+ * A FUSED plan's second kernel, for batches too small to fill the chip with
+ * the first, is compiled (and cached alike) by the first ponni_forward of
+ * such a batch on a stream that is not being captured; until then, and in
+ * ponni_forward_no_alloc, every batch runs on the first kernel.
  * Stands in for the compile step of building a reference model, which
  * happens when the application is compiled. */
 int ponni_plan_compile(ponni_plan plan);

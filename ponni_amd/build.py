@@ -36,7 +36,7 @@ SOURCES = [
 ]
 
 # Headers embedded in the library for the run-time (hipRTC) compiler.
-JIT_HEADERS = ["program.h", "pointwise.h", "fused_f32.h", "fused_f16.h", "narrow_jit.h"]
+JIT_HEADERS = ["program.h", "pointwise.h", "fused_f32.h", "fused_f16.h", "fused_split.h", "narrow_jit.h"]
 
 COMMON = [
     "-O3",

@@ -296,14 +296,61 @@ std::string narrow_source_of(ponni_plan_s const& p, FusedConfig& cfg);
 
 namespace {
 std::string fused_source_once(ponni_plan_s const& p, FusedConfig& cfg, bool allow_vec_staging);
+
+// Waves per workgroup and column tiles of the small-batch kernel.  Four waves
+// (one per SIMD) and one column tile: more waves repeat the operations that
+// every wave runs, more columns make the batch's tiles fewer (fp32 32-128-16
+// residual chain, 10,000 columns: 43 us; eight waves 49, two column tiles 53).
+// 16-bit contractions take a fragment per 16 cycles of MFMAs, more than L2
+// delivers, so chains of wide layers share each between two column tiles
+// (fp16 64-256-256-256-64, 21,600 columns: 15.5 against 22.6 us), unless they
+// hold operations that every wave repeats (256-wide with LayerNorm: 47.6 us
+// with one tile, 47.8 with two, and 26.4 against 31.1 at 10,000); beyond 512
+// features with eight waves (1024: 86 against 141 us).
+void split_shape(ponni_plan_s const& p, FusedConfig& cfg) {
+  bool const half = p.dtype == PONNI_F16 || p.dtype == PONNI_BF16;
+  bool repeated = false;
+  for (Op const& op : p.ops) repeated = repeated || (op.code != OP_DENSE && op.code != OP_SAVE && op.code != OP_LOAD);
+  cfg.split_waves = half && p.max_width > 512 ? 8 : 4;
+  cfg.split_nt = half && p.max_width > 176 && !repeated ? 2 : 1;
+  cfg.split_wps = cfg.split_waves / 4;
+}
+
+// The small-batch kernel's time per column over the main kernel's where both
+// fill the chip, from their cycles per SIMD and 16-column tile: its
+// contractions take as long as the wave with the most output tiles, and
+// what is not a contraction runs in all four waves.  (1.1: measured on
+// balanced chains, fp32 64-256-256-256-64 at 262,144 columns 786 against 686 us.)
+double split_cost_ratio(ponni_plan_s const& p) {
+  bool const half = p.dtype == PONNI_F16 || p.dtype == PONNI_BF16;
+  double const mfma = p.dtype == PONNI_F64 ? 256 : half ? 8 : 128;  // per input and output tile
+  double main = 0, split = 0;
+  for (Op const& op : p.ops) {
+    int const to = tiles(op.n_out), ti = tiles(op.code == OP_PROJ_ADD ? op.aux : op.n_in);
+    if (op.code == OP_DENSE || op.code == OP_PROJ_ADD) {
+      double const per_tile = ti * mfma + 100;  // (100: its share of the epilogue)
+      main += to * per_tile;
+      split += (to + 3) / 4 * 4 * per_tile;
+    } else if (op.code != OP_SAVE && op.code != OP_LOAD && op.code != OP_CONCAT) {
+      main += std::max(ti, to) * 80;
+      split += std::max(ti, to) * 80 * 4;
+    }
+  }
+  return main > 0 ? 1.1 * split / main : 0;
+}
 }  // namespace
 
 // A staged 16-bit plan whose per-feature vectors would not fit next to the
 // staging slots and input rows keeps them in global memory (L2).
 std::string fused_source(ponni_plan_s const& p, FusedConfig& cfg) {
   FusedConfig first = cfg;
+  if (first.split) split_shape(p, first);
   std::string src = fused_source_once(p, first, true);
-  if (first.lds_total > kFusedLdsBytes && first.vec_bytes > 0) return fused_source_once(p, cfg, false);
+  if (first.lds_total > kFusedLdsBytes && first.vec_bytes > 0) {
+    first = cfg;
+    if (first.split) split_shape(p, first);
+    src = fused_source_once(p, first, false);
+  }
   cfg = first;
   return src;
 }
@@ -323,7 +370,7 @@ std::string fused_source_once(ponni_plan_s const& p, FusedConfig& cfg, bool allo
   // run two waves per SIMD with A fragments staged through LDS (fused_f16.h
   // dense_hs), or one when the widest layer's two states do not fit in
   // half the registers.
-  int const NT = fused_nt(p);
+  int const NT = cfg.split ? cfg.split_nt : fused_nt(p);
   // 16-bit plans: two waves per SIMD (one eight-wave workgroup per CU), the
   // compile permitting (fused_compile).
   int const half_wps = 2;
@@ -406,6 +453,13 @@ std::string fused_source_once(ponni_plan_s const& p, FusedConfig& cfg, bool allo
   // waves share the staged A fragments and the activation table.
   if (half) cfg.waves = 4 * std::min(cfg.waves_per_simd, half_wps);
   cfg.columns_per_block = cfg.waves * 16 * NT;
+  if (cfg.split) {
+    cfg.waves = cfg.split_waves;
+    cfg.waves_per_simd = cfg.split_wps;
+    cfg.columns_per_block = 16 * NT;
+    cfg.lds_bytes = 0;
+    cfg.params_in_registers = cfg.saved_in_lds = false;
+  }
 
   std::ostringstream o;
   std::string const IO = half ? E : dbl ? std::string("double") : std::string("float");
@@ -415,7 +469,7 @@ std::string fused_source_once(ponni_plan_s const& p, FusedConfig& cfg, bool allo
   // and c5 2.8 / 3.5 % faster).  Plans streaming parameters from L2 keep the
   // compiler's order: measured neutral at their occupancy (c3), and the
   // registers it frees would move c3 to two waves per SIMD, 8 % slower.
-  int const epi_interleave = (!half && !dbl && (cfg.lds_bytes > 0 || cfg.params_in_registers)) ? 16 : 0;
+  int const epi_interleave = (!cfg.split && !half && !dbl && (cfg.lds_bytes > 0 || cfg.params_in_registers)) ? 16 : 0;
 
   if (dbl) o << "#define PONNI_REAL double\n";
   if (NT != 2) o << "#define PONNI_NT " << NT << "\n";
@@ -423,12 +477,13 @@ std::string fused_source_once(ponni_plan_s const& p, FusedConfig& cfg, bool allo
   // steps ahead (fused_f16.h kFragPipe; 64x512x512x64 3.28 against 3.38 ms,
   // 320 / 384 features 5-7 % faster; at one wave per SIMD, and with two
   // column tiles per wave (c4), reading ahead measured slower).
-  if (half && NT == 1 && cfg.waves_per_simd >= 2) o << "#define PONNI_PIPE 2\n";
+  if (!cfg.split && half && NT == 1 && cfg.waves_per_simd >= 2) o << "#define PONNI_PIPE 2\n";
   o << "#include \"" << (half ? "fused_f16.h" : "fused_f32.h") << "\"\n";
+  if (cfg.split) o << (half ? "#define PONNI_SPLIT_HALF\n" : "") << "#include \"fused_split.h\"\n";
   o << "using namespace ponni_hip;\nusing namespace ponni_hip::fused;\n";
   if (half) o << "typedef " << E << " E;\n";
   o << "extern \"C\" __global__ __launch_bounds__(" << 64 * cfg.waves << ", " << cfg.waves_per_simd << ") void "
-    << fused_kernel_name(p)
+    << fused_kernel_name(p) << (cfg.split ? "_split" : "")
     << "(" << F << " const* __restrict__ gparams, " << IO << " const* __restrict__ x, int64_t ldx, " << IO
     << "* __restrict__ y, int64_t ldy, int64_t batch) {\n";
   if (cfg.lds_bytes > 0) {
@@ -448,7 +503,7 @@ std::string fused_source_once(ponni_plan_s const& p, FusedConfig& cfg, bool allo
   for (Op const& op : p.ops)
     if (op.code == OP_DENSE) dense_seq.push_back(DenseRef{op.woff, (tiles(op.n_in) + 1) / 2, tiles(op.n_out)});
   int const slot_frags = 32, slots = 3;
-  if (half && !dense_seq.empty()) {
+  if (half && !cfg.split && !dense_seq.empty()) {
     std::ostringstream tab;
     int chunks = 0;
     for (DenseRef const& d : dense_seq) {
@@ -480,7 +535,8 @@ std::string fused_source_once(ponni_plan_s const& p, FusedConfig& cfg, bool allo
   // fragments (a late global load would wait behind them: vmcnt is in order).
   // (Measured: c4 unchanged, c3 slower as a persistent fp32 kernel, so only
   // 16-bit plans, which are persistent anyway, stage them by default.)
-  bool const stage_vecs = allow_vec_staging && half && cfg.lds_bytes == 0 && !cfg.params_in_registers;
+  bool const stage_vecs =
+      allow_vec_staging && (half || cfg.split) && cfg.lds_bytes == 0 && !cfg.params_in_registers;
   std::map<int, std::pair<int, int>> vec_lds;  // packed offset -> (LDS offset, length)
   int vec_total = 0;
   auto vec = [&](int off, int n) -> std::string {
@@ -513,8 +569,8 @@ std::string fused_source_once(ponni_plan_s const& p, FusedConfig& cfg, bool allo
   int const n_in0 = p.layers.front().n_in;
   int const in_rows_elems = tiles(n_in0) * 16 * 16 * NT;  // per wave, row-major 16-bit
   int const in_dma_bytes = cfg.waves * in_rows_elems * 2;
-  int const stage_bytes = half && !dense_seq.empty() ? slots * slot_frags * 1024 : 0;
-  bool const in_dma = half && NT % 2 == 0 && in_dma_bytes <= 64 * 1024 &&
+  int const stage_bytes = half && !cfg.split && !dense_seq.empty() ? slots * slot_frags * 1024 : 0;
+  bool const in_dma = half && !cfg.split && NT % 2 == 0 && in_dma_bytes <= 64 * 1024 &&
                       in_dma_bytes + stage_bytes + 16 * 1024 <= kFusedLdsBytes;
   std::string const WCOLS = std::to_string(16 * NT), NW = std::to_string(cfg.waves);
   // The next tile's rows are requested inside the second dense layer, right
@@ -554,8 +610,12 @@ std::string fused_source_once(ponni_plan_s const& p, FusedConfig& cfg, bool allo
     // the next one (requested during the tile, so long landed).
     o << "  wait_vmem();\n";
   }
-  o << "  for (int64_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {\n";
-  o << "    L.col0 = (tile * " << cfg.waves << " + wave_id()) * " << 16 * NT << ";\n";
+  // (the small-batch kernel runs one tile per workgroup: its exchange buffers
+  // alternate within a tile only)
+  if (cfg.split) o << "  if (int64_t const tile = blockIdx.x; tile < tiles) {\n";
+  else o << "  for (int64_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {\n";
+  if (cfg.split) o << "    L.col0 = tile * " << 16 * NT << ";\n";
+  else o << "    L.col0 = (tile * " << cfg.waves << " + wave_id()) * " << 16 * NT << ";\n";
   // Register-resident parameters may be hoisted out of the tile loop; otherwise
   // pin() hides the pointer's loop invariance so they are re-read per tile.
   o << "    " << F << " const* __restrict__ P = " << (cfg.params_in_registers ? "P0;\n" : "pin(P0);\n");
@@ -603,6 +663,43 @@ std::string fused_source_once(ponni_plan_s const& p, FusedConfig& cfg, bool allo
     }
     if (pad && n % 16) o << "    zero_pad<" << n << ", " << tiles(n) << ">(" << v << ", L);\n";
   };
+  // Small-batch kernel (fused_split.h): the contractions in program order,
+  // each with its fragments' type; the first fragments of the next one are
+  // requested (begin_next) before the exchange that ends the last.
+  struct Contraction {
+    int woff, ti, to;
+  };
+  std::vector<Contraction> contractions;
+  size_t next_begin = 0, at = 0;
+  int exchange_tiles = 0;
+  int parity = 0;
+  std::string const SW = std::to_string(cfg.waves);
+  auto begin_next = [&]() {
+    if (next_begin >= contractions.size()) return;
+    Contraction const& c = contractions[next_begin];
+    std::string const k = std::to_string(next_begin++);
+    o << "    " << (half ? "FragsH<E, " : "FragsR<") << c.ti << ", " << c.to << ", " << SW << "> fr" << k << ";\n";
+    o << "    fr" << k << ".begin(reinterpret_cast<" << (half ? "Vec<E>::x8" : F4) << " const*>(P + " << c.woff
+      << "), wv, L.lane);\n";
+  };
+  auto exchange = [&](std::string const& own, std::string const& nv, int n) {
+    std::string const buf = "xbuf[" + std::to_string(parity) + "]";
+    parity ^= 1;
+    o << "    split_put<" << tiles(n) << ", " << SW << ">(" << buf << ", " << own << ", wv, L);\n";
+    begin_next();
+    o << "    exchange_barrier();\n";
+    o << "    auto " << nv << " = " << (half ? "split_get_h<" : "split_get<") << tiles(n) << (half ? ", E" : "") << ", "
+      << NT << ">(" << buf << ", L);\n";
+  };
+  if (cfg.split) {
+    for (Op const& op : p.ops) {
+      if (op.code == OP_DENSE) contractions.push_back({op.woff, tiles(op.n_in), tiles(op.n_out)});
+      if (op.code == OP_PROJ_ADD) contractions.push_back({op.woff, tiles(op.aux), tiles(op.n_out)});
+      if (op.code == OP_DENSE || op.code == OP_PROJ_ADD) exchange_tiles = std::max(exchange_tiles, tiles(op.n_out));
+    }
+    begin_next();
+  }
+  bool stored = false;     // the last contraction wrote y itself
   std::string dense_hook;  // closes a dense_hs call that takes the prefetch hook
   bool pad_ok = true;      // false for a transposed tile
   for (Op const& op : p.ops) {
@@ -618,7 +715,27 @@ std::string fused_source_once(ponni_plan_s const& p, FusedConfig& cfg, bool allo
         // 16-bit rounding, and the add then costs no VALU op).
         bool const lead_bias = op.epi_count > 0 && p.steps[op.epi_begin].act == ACT_BIAS;
         bool const seed = lead_bias && (half || (op.aux & DENSE_BIAS_FIRST));
-        if (half) {
+        std::string const own = "own" + std::to_string(at);
+        if (cfg.split) {
+          bool const tr = half && out_transposed && &op == &p.ops.back();
+          std::string init = half ? "SeedZero{}" : "[&](int) { return " + F4 + "{0, 0, 0, 0}; }";
+          if (seed && half)
+            init = tr ? "SeedRowsT{" + vec(p.steps[op.epi_begin].off, n) + ", L.c}"
+                      : "SeedRows{" + vec(p.steps[op.epi_begin].off, n) + ", L.g}";
+          else if (seed)
+            init = "[&](int mo) { return ld4(" + vec(p.steps[op.epi_begin].off, n) + " + 16 * mo + 4 * L.g); }";
+          std::string const ks = k_steps(op.woff, op.n_in);
+          o << "    auto " << own << " = ";
+          if (half) {
+            o << "split_dense_h<" << tiles(n) << ", " << SW << ", " << (tr ? "true" : "false") << ">(" << cur << ", fr"
+              << at << ", " << init << ", [&](int mo, floatx4 (&t)[" << NT << "], Vec<E>::x4 (&o)[" << NT << "]) {\n";
+          } else {
+            o << "split_dense<" << tiles(n) << ", " << SW << (ks.empty() ? ", " + std::to_string(4 * tiles(op.n_in)) : ks)
+              << ">(" << cur << ", fr" << at << ", " << init << ", [&](int mo, " << F4 << " (&t)[" << NT << "]) {\n";
+          }
+          if (tr) pad_ok = false;
+          at++;
+        } else if (half) {
           bool const tr = out_transposed && &op == &p.ops.back();
           bool const hook = static_cast<int>(dense_index) == hook_dense;
           std::string const init = !seed ? "SeedZero{}"
@@ -662,6 +779,16 @@ std::string fused_source_once(ponni_plan_s const& p, FusedConfig& cfg, bool allo
         if (half) o << "      tile_round<E>(t, o);\n";
         o << (dense_hook.empty() ? "    });\n" : dense_hook);
         dense_hook.clear();
+        if (cfg.split && &op == &p.ops.back()) {
+          if (half)
+            o << "    split_store_h<" << n << ", " << tiles(n) << ", " << SW << ", " << (pad_ok ? "false" : "true") << ">("
+              << own << ", y, ldy, wv, L, " << (out_transposed ? "yvec" : "false") << ");\n";
+          else
+            o << "    split_store<" << n << ", " << tiles(n) << ", " << SW << ">(" << own << ", y, ldy, wv, L);\n";
+          stored = true;
+        } else if (cfg.split) {
+          exchange(own, nv, n);
+        }
         pad_ok = true;
         cur = nv;
         cur_n = n;
@@ -744,7 +871,26 @@ std::string fused_source_once(ponni_plan_s const& p, FusedConfig& cfg, bool allo
       case OP_PROJ_ADD: {
         // proj = b + W^T saved (bias first, ponni_Binop_Projection_Add.h:91-92); out = in + proj.
         auto const& sv = saved[op.slot];
-        if (half) {
+        if (cfg.split) {
+          std::string const nv = fresh(), own = "own" + std::to_string(at);
+          std::string const bias = vec(op.boff, cur_n);
+          std::string const pad = cur_n % 16 ? " if (mo == " + std::to_string(tiles(cur_n) - 1) + ") tile_zero_pad<" +
+                                                   std::to_string(cur_n) + ">(t, mo, L);"
+                                             : std::string();
+          std::string const ks = k_steps(op.woff, sv.second);
+          if (half)
+            o << "    auto " << own << " = split_dense_h<" << tiles(cur_n) << ", " << SW << ", false>(" << sv.first << ", fr"
+              << at << ", SeedRows{" << bias << ", L.g}, [&](int mo, floatx4 (&t)[" << NT << "], Vec<E>::x4 (&o)[" << NT
+              << "]) { tile_add_state_at_h(t, " << cur << ", mo);" << pad << " tile_round<E>(t, o); });\n";
+          else
+            o << "    auto " << own << " = split_dense<" << tiles(cur_n) << ", " << SW
+              << (ks.empty() ? ", " + std::to_string(4 * tiles(sv.second)) : ks) << ">(" << sv.first << ", fr" << at
+              << ", [&](int mo) { return ld4(" << bias << " + 16 * mo + 4 * L.g); }, [&](int mo, " << F4 << " (&t)[" << NT
+              << "]) { tile_add_state_at(t, " << cur << ", mo);" << pad << " });\n";
+          at++;
+          exchange(own, nv, cur_n);
+          cur = nv;
+        } else if (half) {
           o << "    proj_add_h<" << tiles(sv.second) << ", " << tiles(cur_n) << ", " << cur_n << ">(" << cur << ", " << sv.first
             << ", reinterpret_cast<E const*>(P + " << op.woff << "), " << vec(op.boff, cur_n) << ", L);\n";
         } else {
@@ -840,20 +986,34 @@ std::string fused_source_once(ponni_plan_s const& p, FusedConfig& cfg, bool allo
   // and the rows were requested before it).
   if (half && in_dma)
     o << (stage_bytes > 0 ? "    wait_vmem_n<chunk_requests<" + NW + ">()>();\n" : std::string("    wait_vmem();\n"));
-  if (out_transposed) o << "    store_rows_ht<" << cur_n << ">(" << cur << ", y, ldy, L, yvec);\n";
+  // (one wave's share of the stores where every wave holds the output)
+  if (stored) {
+  } else if (cfg.split) {
+    o << "    if (wv == 0) " << (half ? "store_rows_h<" : "store_rows<") << cur_n << ">(" << cur << ", y, ldy, L);\n";
+  } else if (out_transposed) o << "    store_rows_ht<" << cur_n << ">(" << cur << ", y, ldy, L, yvec);\n";
   else if (half) o << "    store_rows_h<" << cur_n << ">(" << cur << ", y, ldy, L);\n";
   else o << "    store_rows<" << cur_n << ">(" << cur << ", y, ldy, L);\n";
   o << "  }\n}\n";
   if (!vec_lds.empty()) {
-    head << "  __shared__ floatx4 lds_vec[" << vec_total / 4 << "];\n";
+    head << "  __shared__ " << F4 << " lds_vec[" << vec_total / 4 << "];\n";
     for (auto const& kv : vec_lds)
       head << "  stage_vec(lds_vec + " << kv.second.first / 4 << ", gparams + " << kv.first << ", "
            << kv.second.second / 4 << ");\n";
     head << "  __syncthreads();\n";
-    head << "  float const* __restrict__ VP = reinterpret_cast<float const*>(lds_vec);\n";
+    head << "  " << F << " const* __restrict__ VP = reinterpret_cast<" << F << " const*>(lds_vec);\n";
   }
-  cfg.vec_bytes = vec_total * 4;
-  cfg.lds_total = stage_bytes + (in_dma ? in_dma_bytes : 0) + cfg.vec_bytes + static_cast<int>(cfg.lds_bytes);
+  int exchange_bytes = 0;
+  if (cfg.split) {
+    // (16-bit states exchange tiles in pairs)
+    int const units = half ? (exchange_tiles + 1) / 2 * 2 * NT * 64 : exchange_tiles * NT * 64;
+    exchange_bytes = 2 * units * (half ? 8 : 4 * es);
+    head << "  __shared__ " << (half ? "Vec<E>::x8" : F4) << " xlds[2][" << (half ? units / 2 : units) << "];\n";
+    head << "  " << (half ? "Vec<E>::x4" : F4) << "* const xbuf[2] = {reinterpret_cast<" << (half ? "Vec<E>::x4" : F4)
+         << "*>(xlds[0]), reinterpret_cast<" << (half ? "Vec<E>::x4" : F4) << "*>(xlds[1])};\n";
+    head << "  int const wv = wave_id();\n";
+  }
+  cfg.vec_bytes = vec_total * es;
+  cfg.lds_total = exchange_bytes + stage_bytes + (in_dma ? in_dma_bytes : 0) + cfg.vec_bytes + static_cast<int>(cfg.lds_bytes);
   return head.str() + o.str();
 }
 }  // namespace
@@ -1084,8 +1244,12 @@ std::string cache_key(std::string const& src, bool contract) {
   if (hiprtcVersion(&major, &minor) == HIPRTC_SUCCESS)
     opts += "hiprtc " + std::to_string(major) + "." + std::to_string(minor) + " ";
   opts += compiler_identity() + " ";
-  std::string hdrs;
-  for (int i = 0; i < kJitHeaderCount; i++) hdrs += kJitHeaderTexts[i];
+  // (the headers are constant: hashed once)
+  static std::string const hdrs = [] {
+    std::string all;
+    for (int i = 0; i < kJitHeaderCount; i++) all += kJitHeaderTexts[i];
+    return std::to_string(fnv(all));
+  }();
   char buf[32];
   std::snprintf(buf, sizeof(buf), "%016llx", static_cast<unsigned long long>(fnv(src + opts + hdrs)));
   return buf;
@@ -1116,7 +1280,7 @@ int metadata_int(std::vector<char> const& code, char const* key) {
   return -1;
 }
 
-int compile_cached(ponni_plan_s const& p, std::string& key, std::vector<char>& code, std::string& error);
+int compile_cached(ponni_plan_s const& p, bool split, std::string& key, std::vector<char>& code, std::string& error);
 
 }  // namespace
 
@@ -1131,7 +1295,7 @@ int fused_compile(ponni_plan_s& p, std::string& key, std::vector<char>& code, st
     int wps = est.waves_per_simd;
     auto spills_regs = [&](int w, int& spills, int& regs) -> int {
       p.fused_wps = w;
-      int const st = compile_cached(p, key, code, error);
+      int const st = compile_cached(p, false, key, code, error);
       if (st != PONNI_OK) return st;
       spills = metadata_int(code, ".vgpr_spill_count");
       int const v = metadata_int(code, ".vgpr_count"), a = metadata_int(code, ".agpr_count");
@@ -1166,13 +1330,14 @@ int fused_compile(ponni_plan_s& p, std::string& key, std::vector<char>& code, st
     }
     p.fused_wps = wps;
   }
-  return compile_cached(p, key, code, error);
+  return compile_cached(p, false, key, code, error);
 }
 
 namespace {
 
-int compile_cached(ponni_plan_s const& p, std::string& key, std::vector<char>& code, std::string& error) {
+int compile_cached(ponni_plan_s const& p, bool split, std::string& key, std::vector<char>& code, std::string& error) {
   FusedConfig cfg;
+  cfg.split = split;
   std::string const src = fused_source(p, cfg);
   key = cache_key(src, contract_on(p));
   std::lock_guard<std::mutex> lock(g_code_mutex);
@@ -1210,50 +1375,115 @@ int compile_cached(ponni_plan_s const& p, std::string& key, std::vector<char>& c
 
 }  // namespace
 
-int fused_prepare(ponni_plan_s& p, std::string& error) {
-  std::string key;
-  std::vector<char> code;
-  int const st = fused_compile(p, key, code, error);
-  if (st != PONNI_OK) return st;
-  FusedConfig cfg;
-  (void)fused_source(p, cfg);
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) {
+namespace {
+
+// The compiled kernel's module on the current device (loaded once per device
+// and distinct kernel).
+int load_module(std::string const& key, std::vector<char> const& code, std::string const& name, int threads,
+                std::shared_ptr<Module>& out, int& device, std::string& error) {
+  if (hipGetDevice(&device) != hipSuccess) {
     error = "no HIP device";
     return PONNI_ERR_DEVICE;
   }
   std::lock_guard<std::mutex> lock(g_mutex);
-  auto it = g_modules.find({dev, key});
+  auto it = g_modules.find({device, key});
   if (it == g_modules.end()) {
     auto m = std::make_shared<Module>();
     hipError_t e = hipModuleLoadData(&m->module, code.data());
-    if (e == hipSuccess) e = hipModuleGetFunction(&m->fn, m->module, fused_kernel_name(p).c_str());
-    if (e == hipSuccess)
-      e = hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&m->blocks_per_cu, m->fn, cfg.waves * 64, 0);
+    if (e == hipSuccess) e = hipModuleGetFunction(&m->fn, m->module, name.c_str());
+    if (e == hipSuccess) e = hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&m->blocks_per_cu, m->fn, threads, 0);
     if (e != hipSuccess) {
       error = std::string("loading the fused kernel failed: ") + hipGetErrorString(e);
       return PONNI_ERR_DEVICE;
     }
-    it = g_modules.emplace(std::make_pair(dev, key), m).first;
+    it = g_modules.emplace(std::make_pair(device, key), m).first;
   }
-  p.fused_fn = it->second->fn;
-  p.fused_blocks_per_cu = it->second->blocks_per_cu > 0 ? it->second->blocks_per_cu : 1;
+  out = it->second;
+  return PONNI_OK;
+}
+
+}  // namespace
+
+int fused_prepare(ponni_plan_s& p, std::string& error) {
+  std::string key;
+  std::vector<char> code;
+  int st = fused_compile(p, key, code, error);
+  if (st != PONNI_OK) return st;
+  FusedConfig cfg;
+  (void)fused_source(p, cfg);
+  int dev = 0;
+  std::shared_ptr<Module> m;
+  st = load_module(key, code, fused_kernel_name(p), cfg.waves * 64, m, dev, error);
+  if (st != PONNI_OK) return st;
   // The persistent grid's size, looked up once rather than at every launch.
   if (hipDeviceGetAttribute(&p.fused_cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
       p.fused_cus <= 0) {
     error = "no compute units";
     return PONNI_ERR_DEVICE;
   }
+  p.fused_blocks_per_cu = m->blocks_per_cu > 0 ? m->blocks_per_cu : 1;
   p.fused_persistent = cfg.lds_bytes > 0 || cfg.vec_bytes > 0 || cfg.params_in_registers || cfg.persistent_loop;
   p.fused_columns_per_block = cfg.columns_per_block;
   p.fused_waves = cfg.waves;
+  p.fused_fn = m->fn;
+  if (p.path == PONNI_PATH_FUSED) {
+    bool const half = p.dtype == PONNI_F16 || p.dtype == PONNI_BF16;
+    int widest = 0;
+    for (Op const& op : p.ops)
+      if (op.code == OP_DENSE || op.code == OP_PROJ_ADD) widest = std::max(widest, tiles(op.n_out));
+    // (fp32 and 16-bit models of at most two tiles run at the launch floor either way)
+    p.split_ratio = widest >= (p.dtype == PONNI_F64 ? 2 : 3) ? split_cost_ratio(p) : 0;
+    // The main kernel with spilled states, or with one column tile per wave
+    // and one wave per SIMD, is the slower one at every batch (262,144 columns:
+    // fp32 40-256-20 residual, 151 registers spilled, 2908 against 1435 us;
+    // fp32 24-384-384-12 1519 against 809; fp16 64-1024-1024-64, 259 spilled,
+    // 1028 against 791); 16-bit plans that spill few are not (62: 455 against 489).
+    int const spills = metadata_int(code, ".vgpr_spill_count");
+    p.split_always = half ? fused_nt(p) == 1 && spills >= 100
+                          : spills > 0 || (fused_nt(p) == 1 && cfg.waves_per_simd == 1);
+  }
   return PONNI_OK;
 }
 
+int fused_prepare_split(ponni_plan_s& p, std::string& error) {
+  std::string key;
+  std::vector<char> code;
+  int st = compile_cached(p, true, key, code, error);
+  if (st != PONNI_OK) return st;
+  FusedConfig cfg;
+  cfg.split = true;
+  (void)fused_source(p, cfg);
+  int dev = 0;
+  std::shared_ptr<Module> m;
+  st = load_module(key, code, fused_kernel_name(p) + "_split", cfg.waves * 64, m, dev, error);
+  if (st != PONNI_OK) return st;
+  p.split_columns_per_block = cfg.columns_per_block;
+  p.split_waves = cfg.waves;
+  p.split_fn = m->fn;
+  return PONNI_OK;
+}
+
+// A round of the main kernel (one workgroup per CU) takes a wave's whole pass
+// however few columns the batch has, and a batch just over a round takes two;
+// the small-batch kernel's time grows with the batch from about a quarter of
+// a round (measured 0.15-0.25 over the models below).  Measured at 10,000 /
+// 21,600 / 32,769 columns, main against small-batch: fp32 32-128-16 residual
+// 82 / 85 / 165 against 43 / 82 / 116 us; fp16 64-256-256-256-64 24 / 25 / 30
+// against 11 / 16 / 25; fp64 16-64-64-64-8 12.6 / 13.2 / 22.4 against 8.4 /
+// 13.2 / 17.4.  Beyond two rounds the main kernel's workgroups balance.
+bool fused_wants_split(ponni_plan_s const& p, int64_t batch) {
+  if (p.path != PONNI_PATH_FUSED || p.split_ratio <= 0) return false;
+  if (p.split_always) return true;
+  double const rounds = double(batch) / (double(p.fused_cus) * p.fused_columns_per_block);
+  return rounds <= 2 && 0.25 + p.split_ratio * rounds < (rounds <= 1 ? 1 : 2);
+}
+
 hipError_t fused_launch(ponni_plan_s const& p, LaunchArgs const& a, hipStream_t stream) {
-  int64_t const blocks = (a.batch + p.fused_columns_per_block - 1) / p.fused_columns_per_block;
+  bool const split = p.split_fn != nullptr && fused_wants_split(p, a.batch);
+  int const columns = split ? p.split_columns_per_block : p.fused_columns_per_block;
+  int64_t const blocks = (a.batch + columns - 1) / columns;
   int64_t grid = blocks;
-  if (p.fused_persistent) {
+  if (p.fused_persistent && !split) {
     int64_t const resident = int64_t(p.fused_cus) * p.fused_blocks_per_cu;
     grid = blocks < resident ? blocks : resident;
   }
@@ -1262,19 +1492,20 @@ hipError_t fused_launch(ponni_plan_s const& p, LaunchArgs const& a, hipStream_t 
   void* y = a.y;
   int64_t ldx = a.ld_x, ldy = a.ld_y, batch = a.batch;
   void* args[] = {&params, &x, &ldx, &y, &ldy, &batch};
-  unsigned const threads = 64u * unsigned(p.fused_waves);
+  hipFunction_t const fn = split ? p.split_fn : p.fused_fn;
+  unsigned const threads = 64u * unsigned(split ? p.split_waves : p.fused_waves);
   bool const timed = a.ev_start != nullptr || a.ev_stop != nullptr;
   // The extended launch takes the global work size in 32 bits; a grid
   // beyond that is timed by events recorded around an ordinary launch.
   if (timed && uint64_t(grid) * threads <= UINT32_MAX)
-    return hipExtModuleLaunchKernel(p.fused_fn, static_cast<uint32_t>(uint64_t(grid) * threads), 1, 1, threads, 1, 1,
+    return hipExtModuleLaunchKernel(fn, static_cast<uint32_t>(uint64_t(grid) * threads), 1, 1, threads, 1, 1,
                                     0, stream, args, nullptr, a.ev_start, a.ev_stop, 0);
   if (timed && a.ev_start != nullptr) {
     hipError_t const e = hipEventRecord(a.ev_start, stream);
     if (e != hipSuccess) return e;
   }
   hipError_t const e =
-      hipModuleLaunchKernel(p.fused_fn, static_cast<unsigned>(grid), 1, 1, threads, 1, 1, 0, stream, args, nullptr);
+      hipModuleLaunchKernel(fn, static_cast<unsigned>(grid), 1, 1, threads, 1, 1, 0, stream, args, nullptr);
   if (e != hipSuccess || !timed || a.ev_stop == nullptr) return e;
   return hipEventRecord(a.ev_stop, stream);
 }

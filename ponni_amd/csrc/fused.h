@@ -23,6 +23,10 @@ struct FusedConfig {
   bool persistent_loop = false;      // staged 16-bit plans: one workgroup per CU loops over tiles
   int columns_per_block = 128;
   int lds_total = 0;                 // bytes of LDS the kernel declares
+  // The small-batch kernel (fused_split.h): a workgroup's waves share one
+  // tile of columns and split each contraction's output tiles.
+  bool split = false;
+  int split_waves = 8, split_nt = 1, split_wps = 2;
 };
 
 // Widest state a FUSED kernel of this dtype keeps on chip.
@@ -37,6 +41,10 @@ std::string fused_source(ponni_plan_s const& p, FusedConfig& cfg);
 int fused_compile(ponni_plan_s& p, std::string& key, std::vector<char>& code, std::string& error);
 // Compile if needed and load the module on the current device.
 int fused_prepare(ponni_plan_s& p, std::string& error);
+// The small-batch kernel of a FUSED plan: does a batch run on it, and
+// compile if needed and load it (after fused_prepare).
+bool fused_wants_split(ponni_plan_s const& p, int64_t batch);
+int fused_prepare_split(ponni_plan_s& p, std::string& error);
 hipError_t fused_launch(ponni_plan_s const& p, LaunchArgs const& a, hipStream_t stream);
 
 }  // namespace ponni_hip

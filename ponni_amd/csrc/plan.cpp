@@ -1438,6 +1438,16 @@ int forward_impl(ponni_plan plan, const void* x, int64_t ld_in, void* y, int64_t
     HIP_TRY(hipGetDevice(&dev));
     if (dev != plan->device) return fail(PONNI_ERR_DEVICE, "plan was first used on another device");
   }
+  // (A captured stream cannot load a module: a plan whose small-batch kernel
+  // is not there yet then runs its other kernel, which takes any batch.)
+  if (plan->split_fn == nullptr && !no_alloc && fused_wants_split(*plan, batch)) {
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &capturing) == hipSuccess && capturing == hipStreamCaptureStatusNone) {
+      std::string error;
+      int const st = fused_prepare_split(*plan, error);
+      if (st != PONNI_OK) return fail(st, error);
+    }
+  }
   void* scratch[3] = {};  // tmp1, tmp2, the saved-slot area
   int64_t scratch_ld = 0;
   if (no_alloc) {

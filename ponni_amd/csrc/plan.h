@@ -197,6 +197,13 @@ struct ponni_plan_s {
   int fused_columns_per_block = 128;
   int fused_waves = 4;  // waves per workgroup
   int fused_wps = 0;    // waves per SIMD the kernel is compiled for (0: not settled yet)
+  // Its small-batch kernel (fused_split.h), loaded by the first forward of a
+  // batch that runs on it; until then every batch runs on fused_fn.
+  hipFunction_t split_fn = nullptr;
+  int split_columns_per_block = 16;
+  int split_waves = 4;
+  double split_ratio = 0;     // its time per column over fused_fn's (0: the plan has none)
+  bool split_always = false;  // it is the faster one at every batch
 
   // Parameter segments shared with caller-owned arrays (two per layer at
   // most), and the gather map that refreshes the device-shared ones.

@@ -1,0 +1,99 @@
+"""The small-batch kernels of FUSED plans (fused_split.h: a workgroup's waves
+share one tile of columns) against the CPU oracle, and the kernels that large
+batches run on the same small batches: tile counts that do and do not divide
+among the waves, padded widths, projections, barriers, saved states, a
+transposed output, one and two column tiles, ragged column edges.
+
+A plan put on the device by ponni_plan_device_params has only its main
+kernel loaded, and the allocation-free forward loads nothing, so that pair
+runs the main kernel at any batch; ponni_forward chooses by the batch.
+Bars: those of test_gpu_parity.py (fp64 1e-12 relative to the largest value)."""
+import ctypes
+
+import numpy as np
+import pytest
+
+import oracle
+import ponni_amd as P
+from tests.test_gpu_parity import ORACLE_MODE, TORCH_DT, check_f32, check_half
+
+pytestmark = pytest.mark.gpu
+
+
+def _w(r, a, b):
+    return r.uniform(-1, 1, (a, b)) * np.sqrt(6.0 / (a + b))
+
+
+def _mlp(r, widths, act):
+    layers = []
+    for i, (a, b) in enumerate(zip(widths, widths[1:])):
+        layers += [P.Matvec(_w(r, a, b)), P.Bias(r.uniform(-0.1, 0.1, b))]
+        if i < len(widths) - 2:
+            layers.append(act(b))
+    return layers
+
+
+def _residual(r, n, w, out, blocks):
+    layers = [P.Matvec(_w(r, n, w))]
+    for _ in range(blocks):
+        layers += [P.Save_State(0, w), P.LayerNorm(r.uniform(0.8, 1.2, w), r.uniform(-0.1, 0.1, w)),
+                   P.Matvec(_w(r, w, w)), P.Gelu(w, True), P.Matvec(_w(r, w, w)), P.Bias(r.uniform(-0.1, 0.1, w)),
+                   P.Binop_Add(0, w)]
+    return layers + [P.Matvec(_w(r, w, out)), P.Softmax(out)]
+
+
+def _projection(r, n, w):
+    return [P.Save_State(1, n), P.Matvec(_w(r, n, w)), P.Sigmoid(w),
+            P.Binop_Projection_Add(1, _w(r, n, w), r.uniform(-0.1, 0.1, w)), P.Binop_Concatenate(1, w, w + n, True),
+            P.Matvec(_w(r, w + n, w)), P.Binop_Projection_Add(1, _w(r, n, w), r.uniform(-0.1, 0.1, w))]
+
+
+CHAINS = {
+    "odd_tiles": lambda r: _mlp(r, [20, 70, 130, 33], P.Tanh),       # 5, 9, 3 output tiles
+    "few_tiles": lambda r: _mlp(r, [5, 40, 16, 40, 3], P.Relu),      # 3, 1, 3, 1
+    "wide": lambda r: _mlp(r, [64, 250, 200, 64], P.Tanh),           # 16-bit: two column tiles
+    "widest": lambda r: _mlp(r, [33, 520, 31], P.Silu),              # 16-bit: eight waves
+    "residual": lambda r: _residual(r, 19, 70, 7, 2),
+    "projection": lambda r: _projection(r, 21, 45),
+}
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _oracle_built():
+    oracle.build()
+
+
+@pytest.mark.parametrize("dtype", ["f32", "f16", "bf16", "f64"])
+@pytest.mark.parametrize("chain", sorted(CHAINS))
+def test_small_batch_and_main_kernels(cuda, chain, dtype):
+    import torch
+
+    if chain == "widest" and dtype in ("f32", "f64"):
+        pytest.skip("wider than these types' fused kernels")
+    layers = CHAINS[chain](np.random.default_rng(77))
+    tdt = getattr(torch, TORCH_DT[dtype])
+    small = P.create_inference_model(*layers, dtype=dtype, path="fused")
+    main = P.create_inference_model(*layers, dtype=dtype, path="fused")
+    A = P._abi
+    A.check(A.lib().ponni_plan_device_params(main._plan, ctypes.byref(ctypes.c_void_p())))
+    n_in, n_out = small.get_num_inputs(), small.get_num_outputs()
+    for B, pad in [(1, 0), (16, 3), (33, 0), (64, 8), (515, 0)]:
+        x = np.random.default_rng(B).standard_normal((n_in, B))
+        xs = torch.zeros((n_in, B + pad), dtype=tdt, device="cuda:0")
+        xs[:, :B] = torch.from_numpy(x).to(tdt)
+        want = oracle.forward(layers, xs[:, :B].double().cpu().numpy(), ORACLE_MODE[dtype])
+        for name in ("small", "main"):
+            print(f"small batch: chain={chain} dtype={dtype} B={B} kernel={name}", flush=True)
+            ys = torch.full((n_out, B + pad), float("nan"), dtype=tdt, device="cuda:0")
+            stream = torch.cuda.current_stream().cuda_stream
+            args = (xs.data_ptr(), xs.stride(0), ys.data_ptr(), ys.stride(0), B, stream)
+            (small.forward_raw if name == "small" else main.forward_raw_no_alloc)(*args)
+            torch.cuda.synchronize()
+            assert torch.isnan(ys[:, B:].float()).all(), "kernel wrote past the batch"
+            got = ys[:, :B].double().cpu().numpy()
+            if dtype == "f32":
+                check_f32(got, want)
+            elif dtype == "f64":
+                assert np.abs(got - want).max() <= 1e-12 * max(1.0, np.abs(want).max())
+            else:
+                check_half(got, want)
