@@ -22,6 +22,7 @@ SOURCES = [
     "plan.cpp",
     "file_abi.cpp",
     "kernels_generic.hip",
+    "kernels_layered.hip",
     "kernels_narrow.hip",
     "kernels_mfma_dispatch.cpp",
     "kernels_mfma_f32_mt2.hip",

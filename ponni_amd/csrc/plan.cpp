@@ -326,9 +326,15 @@ Step make_step(ponni_layer_desc const& d) {
 
 int round_up(int v, int m) { return (v + m - 1) / m * m; }
 
-// GENERIC and LAYERED plans share the op list, the reference parameter
-// layout and the HBM scratch.
-bool generic_layout(ponni_plan_s const& p) { return p.path == PONNI_PATH_GENERIC || p.path == PONNI_PATH_LAYERED; }
+// GENERIC and LAYERED plans share the op list and the HBM scratch.
+bool has_scratch(ponni_plan_s const& p) { return p.path == PONNI_PATH_GENERIC || p.path == PONNI_PATH_LAYERED; }
+
+// 16-bit FUSED and LAYERED plans hold their dense weights as 16-bit operands
+// (and everything else as fp32 words); other plans hold the compute type.
+bool half_words(ponni_plan_s const& p) {
+  return (p.path == PONNI_PATH_FUSED || p.path == PONNI_PATH_LAYERED) &&
+         (p.dtype == PONNI_F16 || p.dtype == PONNI_BF16);
+}
 
 // Rows of the saved-slot area (generic_ops.h Bufs): slot s after slots
 // 0 .. s-1, each get_saved_state_size<s>() rows high.
@@ -380,7 +386,9 @@ std::vector<int32_t> contractions_over_input(ponni_plan_s const& p) {
 
 // Per-path packed size and layout of one layer's parameters.
 // GENERIC: reference layout.  NARROW: padded to the width class W.
-// MFMA: dense weights in A-fragment order, vectors padded to 16.
+// MFMA / FUSED: dense weights in A-fragment order, vectors padded to 16.
+// LAYERED: the same, but a projection's weights (read by the GENERIC op) in
+// the reference layout.
 int64_t packed_size(ponni_plan_s const& p, ponni_layer_desc const& d) {
   int const W = p.width_class;
   switch (p.path) {
@@ -396,9 +404,12 @@ int64_t packed_size(ponni_plan_s const& p, ponni_layer_desc const& d) {
         default: return 0;
       }
     case PONNI_PATH_MFMA:
+    case PONNI_PATH_LAYERED:
     case PONNI_PATH_FUSED: {
       auto tiles = [](int n) { return (n + 15) / 16; };
-      if (p.path == PONNI_PATH_FUSED && (p.dtype == PONNI_F16 || p.dtype == PONNI_BF16)) {
+      if (p.path == PONNI_PATH_LAYERED && d.kind == PONNI_LAYER_BINOP_PROJECTION_ADD)
+        return (int64_t(d.n_aux) * d.n_in + 15) / 16 * 16 + round_up(d.n_in, 16);
+      if (half_words(p)) {
         // Dense blocks: one 1 KB fragment (256 four-byte units) per output tile
         // and 32-feature step; vectors stay fp32.
         auto steps = [&](int n) { return (tiles(n) + 1) / 2; };
@@ -438,8 +449,7 @@ int64_t packed_size(ponni_plan_s const& p, ponni_layer_desc const& d) {
 // Packed length of a per-feature vector of n features in the path's layout.
 int64_t vec_size(ponni_plan_s const& p, int n) {
   switch (p.path) {
-    case PONNI_PATH_GENERIC:
-    case PONNI_PATH_LAYERED: return n;
+    case PONNI_PATH_GENERIC: return n;
     case PONNI_PATH_NARROW: return p.width_class;
     default: return round_up(n, 16);
   }
@@ -663,7 +673,7 @@ bool mfma_supports(ponni_plan_s const& p) {
 //               rounded to the plan's 16-bit type, stored as fp32
 template <class Emit>
 void visit_param_slots(ponni_plan_s const& p, Emit&& emit) {
-  bool const half_fused = p.path == PONNI_PATH_FUSED && (p.dtype == PONNI_F16 || p.dtype == PONNI_BF16);
+  bool const half_fused = half_words(p);
   int const vec_kind = half_fused ? SLOT_WORD : SLOT_VALUE;
   int const L = static_cast<int>(p.layers.size());
   int const W = p.width_class;
@@ -677,7 +687,11 @@ void visit_param_slots(ponni_plan_s const& p, Emit&& emit) {
     // transposed source holds W^T [N, K] (generated Dense, "output_input").
     auto dense = [&](int64_t src0, int K, int N, bool transposed) {
       auto idx = [&](int k, int n) { return src0 + (transposed ? int64_t(n) * K + k : int64_t(k) * N + n); };
-      if (half_fused) {
+      if (p.path == PONNI_PATH_GENERIC ||
+          (p.path == PONNI_PATH_LAYERED && d.kind == PONNI_LAYER_BINOP_PROJECTION_ADD)) {
+        for (int k = 0; k < K; k++)
+          for (int n = 0; n < N; n++) emit(base + int64_t(k) * N + n, vec_kind, i, idx(k, n));
+      } else if (half_fused) {
         int64_t const hb = 2 * base;  // 16-bit index of the layer's first word
         // v_mfma_f32_16x16x32 A fragment of output tile mo and 32-feature
         // step t: lane l, element j holds W[16(2t + j/4) + 4(l/16) + j%4][16 mo + l%16].
@@ -690,9 +704,6 @@ void visit_param_slots(ponni_plan_s const& p, Emit&& emit) {
                 int const n = 16 * mo + (l & 15);
                 if (k < K && n < N) emit(hb + ((int64_t(mo) * TS + t) * 64 + l) * 8 + j, SLOT_HALF, i, idx(k, n));
               }
-      } else if (generic_layout(p)) {
-        for (int k = 0; k < K; k++)
-          for (int n = 0; n < N; n++) emit(base + int64_t(k) * N + n, SLOT_VALUE, i, idx(k, n));
       } else if (p.path == PONNI_PATH_NARROW) {
         for (int k = 0; k < K; k++)
           for (int n = 0; n < N; n++) emit(base + int64_t(k) * W + n, SLOT_VALUE, i, idx(k, n));
@@ -706,10 +717,12 @@ void visit_param_slots(ponni_plan_s const& p, Emit&& emit) {
         // that transposed order and the result lands in the fp32 tile layout.
         bool const rows_t = p.dtype == PONNI_F64;
         int const TK = (K + 15) / 16, TN = (N + 15) / 16;
+        // (four values of 16 lanes at a time: 16 neighbours of a source row)
         for (int mo = 0; mo < TN; mo++)
           for (int m = 0; m < TK; m++)
-            for (int l = 0; l < 64; l++)
-              for (int v = 0; v < 4; v++) {
+            for (int gv = 0; gv < 16; gv++)
+              for (int c = 0; c < 16; c++) {
+                int const l = gv / 4 * 16 + c, v = gv % 4;
                 int const k = k_in ? 4 * (4 * m + v) + (l >> 4) : 16 * m + 4 * (l >> 4) + v;
                 int const r = l & 15;
                 int const n = 16 * mo + (rows_t ? (r & 3) * 4 + (r >> 2) : r);
@@ -751,14 +764,18 @@ void visit_param_slots(ponni_plan_s const& p, Emit&& emit) {
   }
 }
 
-void pack_params(ponni_plan_s const& p, std::vector<double>& out) {
-  out.assign(static_cast<size_t>(p.packed_elements), 0.0);
-  visit_param_slots(p, [&](int64_t slot, int, int layer, int64_t idx) {
-    out[slot] = round_to_dtype(p.params[layer][idx], p.dtype);
+// Parameters in the compute type T (every value exact in it once rounded to
+// the plan's type).
+template <class T>
+void pack_params(ponni_plan_s const& p, std::vector<T>& out) {
+  out.assign(static_cast<size_t>(p.packed_elements), T(0));
+  visit_param_slots(p, [&, dst = out.data(), dtype = p.dtype](int64_t slot, int, int layer, int64_t idx) {
+    double const v = p.params[layer][idx];
+    dst[slot] = dtype == PONNI_F32 ? static_cast<T>(static_cast<float>(v)) : static_cast<T>(round_to_dtype(v, dtype));
   });
 }
 
-// Parameters of FUSED fp16 / bf16 plans as 32-bit words: dense blocks hold
+// Parameters of FUSED and LAYERED fp16 / bf16 plans as 32-bit words: dense blocks hold
 // pairs of 16-bit operands in the v_mfma_f32_16x16x32 A-fragment order (see
 // fused_f16.h), vectors hold fp32 values already rounded to the operand type.
 void pack_words_half(ponni_plan_s const& p, std::vector<uint32_t>& out) {
@@ -978,12 +995,21 @@ int upload(ponni_plan_s& p) {
   if (!p.steps.empty())
     HIP_TRY(hipMemcpy(p.d_steps, p.steps.data(), sizeof(Step) * p.steps.size(), hipMemcpyHostToDevice));
   HIP_TRY(hipMemcpy(p.d_slot_rows, p.slot_rows.data(), sizeof(int32_t) * p.slot_rows.size(), hipMemcpyHostToDevice));
-  std::vector<double> packed;
+  std::vector<double> packed64;
+  std::vector<float> packed32;
   std::vector<uint32_t> words;
-  bool const half_fused = p.path == PONNI_PATH_FUSED && (p.dtype == PONNI_F16 || p.dtype == PONNI_BF16);
-  if (half_fused) pack_words_half(p, words);
-  else pack_params(p, packed);
-  size_t const count = half_fused ? words.size() : packed.size();
+  void const* packed = nullptr;
+  if (half_words(p)) {
+    pack_words_half(p, words);
+    packed = words.data();
+  } else if (p.dtype == PONNI_F64) {
+    pack_params(p, packed64);
+    packed = packed64.data();
+  } else {
+    pack_params(p, packed32);
+    packed = packed32.data();
+  }
+  size_t const count = static_cast<size_t>(p.packed_elements);
   // Rounded up so vector reads of the last packed block stay inside the allocation.
   size_t const bytes = std::max<size_t>((count * param_element_size(p) + 255) / 256 * 256, 256);
   if (bytes > p.d_params_bytes) {
@@ -992,16 +1018,7 @@ int upload(ponni_plan_s& p) {
     HIP_TRY(hipMalloc(&p.d_params, bytes));
     p.d_params_bytes = bytes;
   }
-  if (half_fused) {
-    if (!words.empty()) HIP_TRY(hipMemcpy(p.d_params, words.data(), words.size() * 4, hipMemcpyHostToDevice));
-  } else if (!packed.empty()) {
-    if (p.dtype == PONNI_F64) {
-      HIP_TRY(hipMemcpy(p.d_params, packed.data(), packed.size() * 8, hipMemcpyHostToDevice));
-    } else {
-      std::vector<float> f(packed.begin(), packed.end());
-      HIP_TRY(hipMemcpy(p.d_params, f.data(), f.size() * 4, hipMemcpyHostToDevice));
-    }
-  }
+  if (count > 0) HIP_TRY(hipMemcpy(p.d_params, packed, count * param_element_size(p), hipMemcpyHostToDevice));
   if ((p.path == PONNI_PATH_FUSED || p.narrow_jit) && p.fused_fn == nullptr) {
     std::string error;
     int const st = fused_prepare(p, error);
@@ -1013,7 +1030,7 @@ int upload(ponni_plan_s& p) {
   // the fixed per-device scratch; its address is looked up here, where
   // loading the code object that holds it may allocate, so that
   // ponni_forward_no_alloc never does that lookup first.
-  if (generic_layout(p)) {
+  if (has_scratch(p)) {
     void* base = nullptr;
     HIP_TRY(static_scratch(dev, &base));
   }
@@ -1028,17 +1045,24 @@ void release_scratch(ponni_plan_s& p) {
   }
 }
 
+// Row stride of the state buffers for `batch` columns: LAYERED reads and
+// writes whole 16-byte pieces of aligned rows.
+int64_t scratch_stride(ponni_plan_s const& p, int64_t batch) {
+  return p.path == PONNI_PATH_LAYERED ? (batch + 15) / 16 * 16 : batch;
+}
+
 int reallocate_scratch(ponni_plan_s& p, int64_t batch) {
   HIP_TRY(hipDeviceSynchronize());
   release_scratch(p);
   p.capacity = batch;
-  if (!generic_layout(p) || batch == 0) return PONNI_OK;
+  p.scratch_ld = scratch_stride(p, batch);
+  if (!has_scratch(p) || batch == 0) return PONNI_OK;
   size_t const es = element_size(p.dtype);
   for (int b = 0; b < 2; b++) {
     if (p.tmp_features[b] > 0)
-      HIP_TRY(hipMalloc(&p.d_scratch[b], es * size_t(p.tmp_features[b]) * size_t(batch)));
+      HIP_TRY(hipMalloc(&p.d_scratch[b], es * size_t(p.tmp_features[b]) * size_t(p.scratch_ld)));
   }
-  if (p.saved_total > 0) HIP_TRY(hipMalloc(&p.d_scratch[2], es * size_t(p.saved_total) * size_t(batch)));
+  if (p.saved_total > 0) HIP_TRY(hipMalloc(&p.d_scratch[2], es * size_t(p.saved_total) * size_t(p.scratch_ld)));
   return PONNI_OK;
 }
 
@@ -1451,9 +1475,12 @@ int forward_impl(ponni_plan plan, const void* x, int64_t ld_in, void* y, int64_t
   void* scratch[3] = {};  // tmp1, tmp2, the saved-slot area
   int64_t scratch_ld = 0;
   if (no_alloc) {
-    if (generic_layout(*plan)) {
+    if (has_scratch(*plan)) {
       int64_t offset[3];
-      size_t const need = carved_scratch_bytes(*plan, batch, offset);
+      // (aligned rows where they fit)
+      scratch_ld = scratch_stride(*plan, batch);
+      if (carved_scratch_bytes(*plan, scratch_ld, offset) > kStaticScratchBytes) scratch_ld = batch;
+      size_t const need = carved_scratch_bytes(*plan, scratch_ld, offset);
       if (need > kStaticScratchBytes)
         return fail(PONNI_ERR_SHAPE, "ponni_forward_no_alloc: batch " + std::to_string(batch) + " needs " +
                                          std::to_string(need) + " bytes of state buffers; the fixed scratch holds " +
@@ -1462,17 +1489,16 @@ int forward_impl(ponni_plan plan, const void* x, int64_t ld_in, void* y, int64_t
       if (need > 0) HIP_TRY(static_scratch(plan->device, &base));
       for (int b = 0; b < 3; b++)
         if (offset[b] >= 0) scratch[b] = static_cast<char*>(base) + offset[b];
-      scratch_ld = batch;
     }
   } else {
-    if (generic_layout(*plan) && batch > plan->capacity) {
+    if (has_scratch(*plan) && batch > plan->capacity) {
       int const st = reallocate_scratch(*plan, batch);
       if (st != PONNI_OK) return st;
     } else if (batch > plan->capacity) {
       plan->capacity = batch;  // register paths keep no batch scratch
     }
     for (int b = 0; b < 3; b++) scratch[b] = plan->d_scratch[b];
-    scratch_ld = plan->capacity;
+    scratch_ld = plan->scratch_ld;
   }
   LaunchArgs a{};
   a.ops = plan->d_ops;
@@ -1696,11 +1722,9 @@ int host_twin(ponni_plan_s& plan, ponni_plan_s*& twin) {
   int const st = pull_shared(plan, plan.num_shared_device > 0);
   if (st != PONNI_OK) return st;
   if (plan.host_version != plan.params_version) {
-    std::vector<double> packed;
     twin->params = plan.params;
-    pack_params(*twin, packed);
-    if (twin->dtype == PONNI_F64) twin->host_params_f64 = std::move(packed);
-    else twin->host_params_f32.assign(packed.begin(), packed.end());
+    if (twin->dtype == PONNI_F64) pack_params(*twin, twin->host_params_f64);
+    else pack_params(*twin, twin->host_params_f32);
     plan.host_version = plan.params_version;
   }
   return PONNI_OK;

@@ -90,9 +90,9 @@ constexpr size_t kStaticScratchBytes = size_t(PONNI_NO_ALLOC_SCRATCH_BYTES);
 hipError_t static_scratch(int device, void** out);
 
 hipError_t launch_generic(int dtype, LaunchArgs const& args, hipStream_t stream);
-// One dense op of a LAYERED plan (kernels_generic.hip layered_dense): in and
-// out are the op's state buffers, params the plan's packed parameters in the
-// compute type (GENERIC packing: W [n_in][n_out] at woff).
+// One dense op of a LAYERED plan (kernels_layered.hip layered_dense): in and
+// out are the op's state buffers, params the plan's packed parameters (W in
+// A-fragment order at woff, 4-byte or fp64 units; vectors in the compute type).
 struct DenseArgs {
   const void* x;
   int64_t ldx;
@@ -176,6 +176,7 @@ struct ponni_plan_s {
   size_t d_params_bytes = 0;
   void* d_scratch[3] = {};  // tmp1, tmp2, the saved-slot area
   int64_t capacity = 0;
+  int64_t scratch_ld = 0;  // row stride of d_scratch (at least capacity)
 
   // GENERIC twin of this plan for ponni_plan_device_model (created on first
   // use), and the parameter version it last uploaded.

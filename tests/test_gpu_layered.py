@@ -1,0 +1,80 @@
+"""The LAYERED contraction (kernels_layered.hip) against the CPU oracle where
+it can go wrong: input widths that end inside a contraction step (with
+infinities, which the zero rows past the input must not meet), output widths
+that end inside a tile, rows at every alignment (16-byte pieces, 4-byte
+pieces, elements), the small and the large workgroup tile, epilogues on the
+accumulators and in the loop over the finished tile, a bias that seeds the
+sum.  Bars: those of test_gpu_parity.py (fp64 1e-12 relative to the largest
+value)."""
+import numpy as np
+import pytest
+
+import oracle
+import ponni_amd as P
+from ponni_amd import graph as G
+from tests.test_gpu_parity import ORACLE_MODE, check_f32, check_half, check_non_finite, gpu_run
+from tests.test_graph import lowered_with_params
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _oracle_built():
+    oracle.build()
+
+
+def _w(r, a, b):
+    return r.uniform(-1, 1, (a, b)) * np.sqrt(6.0 / (a + b))
+
+
+def _generated(r, n_in, w):
+    g = G.GraphBuilder(n_in)
+    h = g.unary("Tanh", g.dense(g.input, _w(r, w, n_in), r.uniform(-0.2, 0.2, w), name="a"))
+    return lowered_with_params(g.finish(g.unary("Abs", g.dense(h, _w(r, 5, w), r.uniform(-0.2, 0.2, 5), name="b"))))
+
+
+CHAINS = {
+    # usual steps, then steps of the loop (two with parameters), then usual ones in the loop
+    "epilogues": lambda r: [P.Matvec(_w(r, 37, 150)), P.Bias(r.uniform(-0.1, 0.1, 150)), P.Silu(150), P.Mish(150),
+                            P.Bias(r.uniform(-0.1, 0.1, 150)), P.Tanh(150), P.Matvec(_w(r, 150, 70)), P.Gelu(70),
+                            P.Matvec(_w(r, 70, 3)), P.Bias(r.uniform(-0.1, 0.1, 3)), P.LeakyRelu(3, 0.2)],
+    "one_step": lambda r: [P.Matvec(_w(r, 3, 65)), P.Sigmoid(65), P.LayerNorm(65), P.Matvec(_w(r, 65, 129))],
+    "generated": lambda r: _generated(r, 50, 200),
+    "projection": lambda r: [P.Save_State(0, 9), P.Matvec(_w(r, 9, 33)), P.Relu(33),
+                             P.Binop_Projection_Add(0, _w(r, 9, 33), r.uniform(-0.1, 0.1, 33)),
+                             P.Matvec(_w(r, 33, 17)), P.Gelu(17, True)],
+}
+
+
+@pytest.mark.parametrize("dtype", ["f32", "f16", "bf16", "f64"])
+@pytest.mark.parametrize("chain", sorted(CHAINS))
+def test_layered_edges(cuda, chain, dtype):
+    layers = CHAINS[chain](np.random.default_rng(31))
+    # the last batch has enough columns for the large tile (512 of them)
+    for B, pad in [(1, 0), (127, 0), (130, 6), (257, 3), (33_003, 5), (40_000, 0)]:
+        x = np.random.default_rng(B).standard_normal((layers[0].n_in, B))
+        print(f"layered: chain={chain} dtype={dtype} B={B}", flush=True)
+        got, xg, m = gpu_run(layers, x, dtype=dtype, path="layered", pad=pad)
+        assert m.path == "layered"
+        want = oracle.forward(layers, xg, ORACLE_MODE[dtype])
+        if dtype == "f32":
+            check_f32(got, want)
+        elif dtype == "f64":
+            assert np.abs(got - want).max() <= 1e-12 * max(1.0, np.abs(want).max())
+        else:
+            check_half(got, want)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "f16", "bf16", "f64"])
+@pytest.mark.parametrize("n_in", [5, 16, 33])
+def test_layered_infinite_inputs(cuda, n_in, dtype):
+    r = np.random.default_rng(n_in)
+    layers = [P.Matvec(_w(r, n_in, 70)), P.Tanh(70), P.Matvec(_w(r, 70, 21)), P.Bias(r.uniform(-0.1, 0.1, 21))]
+    x = r.standard_normal((n_in, 515))
+    x[r.integers(n_in, size=200), np.arange(0, 400, 2)] = np.where(np.arange(200) % 2, np.inf, -np.inf)
+    print(f"layered infinities: n_in={n_in} dtype={dtype}", flush=True)
+    for pad in (0, 5):
+        got, xg, _ = gpu_run(layers, x, dtype=dtype, path="layered", pad=pad)
+        want = oracle.forward(layers, xg, ORACLE_MODE[dtype])
+        assert np.isfinite(want[:, 0:400:2]).mean() > 0.5
+        check_non_finite(got, want, dtype)
