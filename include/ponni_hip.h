@@ -348,6 +348,16 @@ int ponni_plan_reallocate_internal_state(ponni_plan plan, int64_t batch);
 int ponni_forward(ponni_plan plan, const void* x, int64_t ld_in, void* y,
                   int64_t ld_out, int64_t batch, hipStream_t stream);
 
+/* ponni_forward of an F16 / BF16 plan on fp32 rows: x is rounded to the
+ * plan's type as it is read and y holds its values as floats, bit for bit
+ * what converting the arrays around ponni_forward gives, without the passes
+ * over memory (the generated infer_batch_half2 on Scalar views,
+ * kokkos_nn/emitter.py:1551-1573).  FUSED and generated NARROW plans; others,
+ * and a plan whose kernel for it would have to be loaded while the stream is
+ * captured, give PONNI_ERR_UNSUPPORTED.  x and y must not overlap. */
+int ponni_forward_fp32_rows(ponni_plan plan, const float* x, int64_t ld_in, float* y,
+                            int64_t ld_out, int64_t batch, hipStream_t stream);
+
 /* ponni_forward for callers that cannot allocate device memory: code under
  * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc.
  * It has no counterpart in the reference.  It calls no hipMalloc, hipFree or

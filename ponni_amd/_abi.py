@@ -175,6 +175,8 @@ def lib() -> ctypes.CDLL:
     L.ponni_forward.argtypes = [vp, vp, i64, vp, i64, i64, vp]
     L.ponni_forward_no_alloc.restype = ctypes.c_int
     L.ponni_forward_no_alloc.argtypes = [vp, vp, i64, vp, i64, i64, vp]
+    L.ponni_forward_fp32_rows.restype = ctypes.c_int
+    L.ponni_forward_fp32_rows.argtypes = [vp, vp, i64, vp, i64, i64, vp]
     L.ponni_forward_timed.restype = ctypes.c_int
     L.ponni_forward_timed.argtypes = [vp, vp, i64, vp, i64, i64, vp, vp, vp]
     L.ponni_forward_steps.restype = ctypes.c_int

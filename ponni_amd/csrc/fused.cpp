@@ -462,7 +462,8 @@ std::string fused_source_once(ponni_plan_s const& p, FusedConfig& cfg, bool allo
   }
 
   std::ostringstream o;
-  std::string const IO = half ? E : dbl ? std::string("double") : std::string("float");
+  std::string const IO = half && !cfg.io32 ? E : dbl ? std::string("double") : std::string("float");
+  int const io_bytes = half && !cfg.io32 ? 2 : es;
   o << "// generated by libponni_hip for one plan\n";
   // fp32 plans whose parameters sit in LDS or registers keep each dense
   // tile's epilogue among the next tile's MFMAs (fused_f32.h dense_ep; c2
@@ -483,7 +484,7 @@ std::string fused_source_once(ponni_plan_s const& p, FusedConfig& cfg, bool allo
   o << "using namespace ponni_hip;\nusing namespace ponni_hip::fused;\n";
   if (half) o << "typedef " << E << " E;\n";
   o << "extern \"C\" __global__ __launch_bounds__(" << 64 * cfg.waves << ", " << cfg.waves_per_simd << ") void "
-    << fused_kernel_name(p) << (cfg.split ? "_split" : "")
+    << fused_kernel_name(p) << cfg.suffix()
     << "(" << F << " const* __restrict__ gparams, " << IO << " const* __restrict__ x, int64_t ldx, " << IO
     << "* __restrict__ y, int64_t ldy, int64_t batch) {\n";
   if (cfg.lds_bytes > 0) {
@@ -568,7 +569,7 @@ std::string fused_source_once(ponni_plan_s const& p, FusedConfig& cfg, bool allo
   // A fragments (3 slots of 32 KB) and vectors.
   int const n_in0 = p.layers.front().n_in;
   int const in_rows_elems = tiles(n_in0) * 16 * 16 * NT;  // per wave, row-major 16-bit
-  int const in_dma_bytes = cfg.waves * in_rows_elems * 2;
+  int const in_dma_bytes = cfg.waves * in_rows_elems * io_bytes;
   int const stage_bytes = half && !cfg.split && !dense_seq.empty() ? slots * slot_frags * 1024 : 0;
   bool const in_dma = half && !cfg.split && NT % 2 == 0 && in_dma_bytes <= 64 * 1024 &&
                       in_dma_bytes + stage_bytes + 16 * 1024 <= kFusedLdsBytes;
@@ -595,12 +596,13 @@ std::string fused_source_once(ponni_plan_s const& p, FusedConfig& cfg, bool allo
     }
   }
   if (out_transposed)
-    o << "  bool const yvec = ((reinterpret_cast<uint64_t>(y) | uint64_t(ldy) * 2) & 7) == 0;\n";
+    o << "  bool const yvec = ((reinterpret_cast<uint64_t>(y) | uint64_t(ldy) * " << io_bytes << ") & " << 4 * io_bytes - 1
+      << ") == 0;\n";
   if (in_dma) {
-    o << "  __shared__ unsigned short in_buf[" << cfg.waves << "][" << in_rows_elems << "];\n";
+    o << "  __shared__ __attribute__((aligned(16))) " << IO << " in_buf[" << cfg.waves << "][" << in_rows_elems << "];\n";
     // Whole tiles of a 16-byte aligned x with a row stride of a multiple of
-    // 8 elements go through LDS; others (the batch's last tile) load directly.
-    o << "  bool const xvec = ((reinterpret_cast<uint64_t>(x) | uint64_t(ldx) * 2) & 15) == 0;\n";
+    // 16 bytes go through LDS; others (the batch's last tile) load directly.
+    o << "  bool const xvec = ((reinterpret_cast<uint64_t>(x) | uint64_t(ldx) * " << io_bytes << ") & 15) == 0;\n";
     o << "  L.col0 = (int64_t(blockIdx.x) * " << NW << " + wave_id()) * " << WCOLS << ";\n";
     o << "  if (blockIdx.x < tiles && xvec && L.col0 + " << WCOLS << " <= batch) prefetch_rows_lds16<" << n_in0 << ", "
       << NT << ">(x, ldx, L, in_buf[wave_id()]);\n";
@@ -625,12 +627,12 @@ std::string fused_source_once(ponni_plan_s const& p, FusedConfig& cfg, bool allo
   int cur_n = p.layers.front().n_in;
   if (in_dma) {
     o << "    auto " << cur << " = xvec && L.col0 + " << WCOLS << " <= batch ? load_rows_lds16<" << cur_n << ", " << NT
-      << ", E>(in_buf[wave_id()], L) : load_rows_h<" << cur_n << ", " << NT << ">(x, ldx, L);\n";
+      << ", E>(in_buf[wave_id()], L) : load_rows_h<" << cur_n << ", " << NT << ", E>(x, ldx, L);\n";
     o << "    wait_lds();\n";
     o << "    Lane Ln = L;\n    Ln.col0 = ((tile + gridDim.x) * " << NW << " + wave_id()) * " << WCOLS << ";\n";
     o << "    bool const pre_next = tile + gridDim.x < tiles && xvec && Ln.col0 + " << WCOLS << " <= batch;\n";
     if (hook_dense < 0) o << "    " << prefetch_next << "\n";
-  } else if (half) o << "    auto " << cur << " = load_rows_h<" << cur_n << ", " << NT << ">(x, ldx, L);\n";
+  } else if (half) o << "    auto " << cur << " = load_rows_h<" << cur_n << ", " << NT << ", E>(x, ldx, L);\n";
   else o << "    auto " << cur << " = " << (in_k.empty() ? "load_rows<" : "load_rows_k<") << cur_n << ">(x, ldx, L);\n";
   std::map<int, std::pair<std::string, int>> saved;  // slot -> (expression, width)
   // The logistic family runs on the hardware transcendentals (pointwise.h),
@@ -1041,7 +1043,9 @@ std::string narrow_source(ponni_plan_s const& p, FusedConfig& cfg) {
   // U groups of V samples per lane, 256 * V samples apart, so that all of a
   // lane's input rows are in flight before its first FMA.
   int const U = 1;
+  bool const io32 = cfg.io32;
   cfg = FusedConfig{};
+  cfg.io32 = io32;
   cfg.waves = 4;
   cfg.waves_per_simd = 4;
   cfg.columns_per_block = 256 * V * U;
@@ -1159,11 +1163,12 @@ std::string narrow_source(ponni_plan_s const& p, FusedConfig& cfg) {
     cur_n = op.n_out;
   }
   o << "}\n";
-  o << "extern \"C\" __global__ __launch_bounds__(256) void " << fused_kernel_name(p)
-    << "(real const* __restrict__ P, S const* __restrict__ x, int64_t ldx, S* __restrict__ y, int64_t ldy, "
+  o << "typedef " << (io32 ? "float" : "S") << " IO;\n";
+  o << "extern \"C\" __global__ __launch_bounds__(256) void " << fused_kernel_name(p) << cfg.suffix()
+    << "(real const* __restrict__ P, IO const* __restrict__ x, int64_t ldx, IO* __restrict__ y, int64_t ldy, "
        "int64_t batch) {\n";
   o << "  constexpr int U = " << U << ", V = " << V << ";\n";
-  o << "  bool const aligned = vec_ok<S, V>(x, ldx) && vec_ok<S, V>(y, ldy);\n";
+  o << "  bool const aligned = vec_ok<IO, V>(x, ldx) && vec_ok<IO, V>(y, ldy);\n";
   // Workgroups wholly inside the batch (all but the last) with vector-aligned
   // views take a path with no per-lane predicate, so every load is issued
   // before the first wait.
@@ -1280,7 +1285,8 @@ int metadata_int(std::vector<char> const& code, char const* key) {
   return -1;
 }
 
-int compile_cached(ponni_plan_s const& p, bool split, std::string& key, std::vector<char>& code, std::string& error);
+int compile_cached(ponni_plan_s const& p, FusedConfig cfg, std::string& key, std::vector<char>& code,
+                   std::string& error);
 
 }  // namespace
 
@@ -1295,7 +1301,7 @@ int fused_compile(ponni_plan_s& p, std::string& key, std::vector<char>& code, st
     int wps = est.waves_per_simd;
     auto spills_regs = [&](int w, int& spills, int& regs) -> int {
       p.fused_wps = w;
-      int const st = compile_cached(p, false, key, code, error);
+      int const st = compile_cached(p, FusedConfig{}, key, code, error);
       if (st != PONNI_OK) return st;
       spills = metadata_int(code, ".vgpr_spill_count");
       int const v = metadata_int(code, ".vgpr_count"), a = metadata_int(code, ".agpr_count");
@@ -1330,14 +1336,13 @@ int fused_compile(ponni_plan_s& p, std::string& key, std::vector<char>& code, st
     }
     p.fused_wps = wps;
   }
-  return compile_cached(p, false, key, code, error);
+  return compile_cached(p, FusedConfig{}, key, code, error);
 }
 
 namespace {
 
-int compile_cached(ponni_plan_s const& p, bool split, std::string& key, std::vector<char>& code, std::string& error) {
-  FusedConfig cfg;
-  cfg.split = split;
+int compile_cached(ponni_plan_s const& p, FusedConfig cfg, std::string& key, std::vector<char>& code,
+                   std::string& error) {
   std::string const src = fused_source(p, cfg);
   key = cache_key(src, contract_on(p));
   std::lock_guard<std::mutex> lock(g_code_mutex);
@@ -1404,16 +1409,19 @@ int load_module(std::string const& key, std::vector<char> const& code, std::stri
 
 }  // namespace
 
-int fused_prepare(ponni_plan_s& p, std::string& error) {
+int fused_prepare(ponni_plan_s& p, bool io32, bool split, std::string& error) {
   std::string key;
   std::vector<char> code;
-  int st = fused_compile(p, key, code, error);
-  if (st != PONNI_OK) return st;
   FusedConfig cfg;
+  cfg.io32 = io32;
+  cfg.split = split;
+  bool const main = !io32 && !split;  // (settles the plan's occupancy)
+  int st = main ? fused_compile(p, key, code, error) : compile_cached(p, cfg, key, code, error);
+  if (st != PONNI_OK) return st;
   (void)fused_source(p, cfg);
   int dev = 0;
   std::shared_ptr<Module> m;
-  st = load_module(key, code, fused_kernel_name(p), cfg.waves * 64, m, dev, error);
+  st = load_module(key, code, fused_kernel_name(p) + cfg.suffix(), cfg.waves * 64, m, dev, error);
   if (st != PONNI_OK) return st;
   // The persistent grid's size, looked up once rather than at every launch.
   if (hipDeviceGetAttribute(&p.fused_cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
@@ -1421,12 +1429,14 @@ int fused_prepare(ponni_plan_s& p, std::string& error) {
     error = "no compute units";
     return PONNI_ERR_DEVICE;
   }
-  p.fused_blocks_per_cu = m->blocks_per_cu > 0 ? m->blocks_per_cu : 1;
-  p.fused_persistent = cfg.lds_bytes > 0 || cfg.vec_bytes > 0 || cfg.params_in_registers || cfg.persistent_loop;
-  p.fused_columns_per_block = cfg.columns_per_block;
-  p.fused_waves = cfg.waves;
-  p.fused_fn = m->fn;
-  if (p.path == PONNI_PATH_FUSED) {
+  FusedKernel& k = p.kernels[io32][split];
+  k.columns_per_block = cfg.columns_per_block;
+  k.waves = cfg.waves;
+  k.resident = 0;
+  if (!split && (cfg.lds_bytes > 0 || cfg.vec_bytes > 0 || cfg.params_in_registers || cfg.persistent_loop))
+    k.resident = int64_t(p.fused_cus) * (m->blocks_per_cu > 0 ? m->blocks_per_cu : 1);
+  k.fn = m->fn;
+  if (main && p.path == PONNI_PATH_FUSED) {
     bool const half = p.dtype == PONNI_F16 || p.dtype == PONNI_BF16;
     int widest = 0;
     for (Op const& op : p.ops)
@@ -1445,24 +1455,6 @@ int fused_prepare(ponni_plan_s& p, std::string& error) {
   return PONNI_OK;
 }
 
-int fused_prepare_split(ponni_plan_s& p, std::string& error) {
-  std::string key;
-  std::vector<char> code;
-  int st = compile_cached(p, true, key, code, error);
-  if (st != PONNI_OK) return st;
-  FusedConfig cfg;
-  cfg.split = true;
-  (void)fused_source(p, cfg);
-  int dev = 0;
-  std::shared_ptr<Module> m;
-  st = load_module(key, code, fused_kernel_name(p) + "_split", cfg.waves * 64, m, dev, error);
-  if (st != PONNI_OK) return st;
-  p.split_columns_per_block = cfg.columns_per_block;
-  p.split_waves = cfg.waves;
-  p.split_fn = m->fn;
-  return PONNI_OK;
-}
-
 // A round of the main kernel (one workgroup per CU) takes a wave's whole pass
 // however few columns the batch has, and a batch just over a round takes two;
 // the small-batch kernel's time grows with the batch from about a quarter of
@@ -1474,26 +1466,22 @@ int fused_prepare_split(ponni_plan_s& p, std::string& error) {
 bool fused_wants_split(ponni_plan_s const& p, int64_t batch) {
   if (p.path != PONNI_PATH_FUSED || p.split_ratio <= 0) return false;
   if (p.split_always) return true;
-  double const rounds = double(batch) / (double(p.fused_cus) * p.fused_columns_per_block);
+  double const rounds = double(batch) / (double(p.fused_cus) * p.kernels[0][0].columns_per_block);
   return rounds <= 2 && 0.25 + p.split_ratio * rounds < (rounds <= 1 ? 1 : 2);
 }
 
-hipError_t fused_launch(ponni_plan_s const& p, LaunchArgs const& a, hipStream_t stream) {
-  bool const split = p.split_fn != nullptr && fused_wants_split(p, a.batch);
-  int const columns = split ? p.split_columns_per_block : p.fused_columns_per_block;
-  int64_t const blocks = (a.batch + columns - 1) / columns;
-  int64_t grid = blocks;
-  if (p.fused_persistent && !split) {
-    int64_t const resident = int64_t(p.fused_cus) * p.fused_blocks_per_cu;
-    grid = blocks < resident ? blocks : resident;
-  }
+hipError_t fused_launch(ponni_plan_s const& p, LaunchArgs const& a, bool io32, hipStream_t stream) {
+  bool const split = p.kernels[io32][1].fn != nullptr && fused_wants_split(p, a.batch);
+  FusedKernel const& k = p.kernels[io32][split];
+  int64_t grid = (a.batch + k.columns_per_block - 1) / k.columns_per_block;
+  if (k.resident > 0 && grid > k.resident) grid = k.resident;
   void const* params = a.params;
   void const* x = a.x;
   void* y = a.y;
   int64_t ldx = a.ld_x, ldy = a.ld_y, batch = a.batch;
   void* args[] = {&params, &x, &ldx, &y, &ldy, &batch};
-  hipFunction_t const fn = split ? p.split_fn : p.fused_fn;
-  unsigned const threads = 64u * unsigned(split ? p.split_waves : p.fused_waves);
+  hipFunction_t const fn = k.fn;
+  unsigned const threads = 64u * unsigned(k.waves);
   bool const timed = a.ev_start != nullptr || a.ev_stop != nullptr;
   // The extended launch takes the global work size in 32 bits; a grid
   // beyond that is timed by events recorded around an ordinary launch.

@@ -26,7 +26,9 @@ struct FusedConfig {
   // The small-batch kernel (fused_split.h): a workgroup's waves share one
   // tile of columns and split each contraction's output tiles.
   bool split = false;
+  bool io32 = false;  // a 16-bit plan's kernel on fp32 input and output rows
   int split_waves = 8, split_nt = 1, split_wps = 2;
+  std::string suffix() const { return std::string(io32 ? "_io32" : "") + (split ? "_split" : ""); }
 };
 
 // Widest state a FUSED kernel of this dtype keeps on chip.
@@ -39,12 +41,11 @@ std::string fused_source(ponni_plan_s const& p, FusedConfig& cfg);
 // Compile (or fetch from cache) the plan's kernel; needs no device.  The
 // first call settles the plan's occupancy (ponni_plan_s::fused_wps).
 int fused_compile(ponni_plan_s& p, std::string& key, std::vector<char>& code, std::string& error);
-// Compile if needed and load the module on the current device.
-int fused_prepare(ponni_plan_s& p, std::string& error);
-// The small-batch kernel of a FUSED plan: does a batch run on it, and
-// compile if needed and load it (after fused_prepare).
+// Compile if needed one of the plan's kernels (ponni_plan_s::kernels) and load
+// it on the current device; the main one first.
+int fused_prepare(ponni_plan_s& p, bool io32, bool split, std::string& error);
+// Does a batch run on the small-batch kernel (once the main one is loaded)?
 bool fused_wants_split(ponni_plan_s const& p, int64_t batch);
-int fused_prepare_split(ponni_plan_s& p, std::string& error);
-hipError_t fused_launch(ponni_plan_s const& p, LaunchArgs const& a, hipStream_t stream);
+hipError_t fused_launch(ponni_plan_s const& p, LaunchArgs const& a, bool io32, hipStream_t stream);
 
 }  // namespace ponni_hip

@@ -59,14 +59,14 @@ __device__ inline E* lane_ptr(E* p, int64_t ld, Lane const& L) {
   return p + off;
 }
 
-// x [N, batch] (row stride ld) -> tile; rows >= N and columns >= batch read 0.
-// Waves whose columns are all inside the batch (all but the last) load
+// x [N, batch] (row stride ld, of E or of float values, which are rounded to
+// E) -> tile; rows >= N and columns >= batch read 0.  Waves whose columns are all inside the batch (all but the last) load
 // without per-element predication.
-template <int N, int NT, class E>
-__device__ inline H<(N + 15) / 16, NT, E> load_rows_h(E const* __restrict__ x, int64_t ld, Lane const& L) {
+template <int N, int NT, class E, class X>
+__device__ inline H<(N + 15) / 16, NT, E> load_rows_h(X const* __restrict__ x, int64_t ld, Lane const& L) {
   constexpr int T = (N + 15) / 16;
   H<T, NT, E> s;
-  E const* __restrict__ xl = lane_ptr(x, ld, L);
+  X const* __restrict__ xl = lane_ptr(x, ld, L);
   if (L.col0 + 16 * NT <= L.batch) {
 #pragma unroll
     for (int m = 0; m < T; m++)
@@ -75,7 +75,7 @@ __device__ inline H<(N + 15) / 16, NT, E> load_rows_h(E const* __restrict__ x, i
 #pragma unroll
         for (int e = 0; e < 4; e++) {
           int const f = 16 * m + 4 * L.g + e;
-          s.v[m][n][e] = (N % 16 == 0 || f < N) ? xl[int64_t(16 * m + e) * ld + 16 * n] : E(0.0f);
+          s.v[m][n][e] = (N % 16 == 0 || f < N) ? static_cast<E>(xl[int64_t(16 * m + e) * ld + 16 * n]) : E(0.0f);
         }
     return s;
   }
@@ -87,7 +87,7 @@ __device__ inline H<(N + 15) / 16, NT, E> load_rows_h(E const* __restrict__ x, i
 #pragma unroll
       for (int e = 0; e < 4; e++) {
         int const f = 16 * m + 4 * L.g + e;
-        s.v[m][n][e] = (f < N && col_ok) ? xl[int64_t(16 * m + e) * ld + 16 * n] : E(0.0f);
+        s.v[m][n][e] = (f < N && col_ok) ? static_cast<E>(xl[int64_t(16 * m + e) * ld + 16 * n]) : E(0.0f);
       }
     }
   return s;
@@ -95,14 +95,15 @@ __device__ inline H<(N + 15) / 16, NT, E> load_rows_h(E const* __restrict__ x, i
 
 // ---- input rows prefetched into LDS one tile ahead ----------------------
 // A wave's input tile (rows 0..16T-1, columns col0 .. col0 + 16 NT - 1) is
-// requested with global_load_lds_dwordx4: piece p = 64 i + l of instruction
-// i fills row slot s = p / (2 NT), columns 8 (p % (2 NT)) .. +7, landing at
-// buf + 8 p, so buf holds 16 NT columns per slot.  Within each block of 16
+// requested with global_load_lds_dwordx4: with 16-bit rows, piece p = 64 i +
+// l of instruction i fills row slot s = p / (2 NT), columns 8 (p % (2 NT)) ..
+// +7, landing at byte 16 p of buf, so buf holds 16 NT columns per slot (fp32
+// rows: twice the pieces of 4 columns, rounded to E when read).  Within each block of 16
 // slots, slot 4a + b holds row 4b + a (a 4 x 4 transpose): the tile's
 // reader takes rows 4g + e in lane group g, which then sit in slots 4e + g,
 // 16 NT elements apart instead of 4 x that, in four different LDS banks
 // (row-major, all four groups read one bank).  Only whole tiles
-// of a 16-byte aligned x with a row stride of a multiple of 8 elements are
+// of a 16-byte aligned x with a row stride of whole 16-byte pieces are
 // requested this way (the caller checks); rows >= N issue nothing.  The
 // loads are asynchronous: the caller waits (vmcnt) before reading buf.
 typedef __attribute__((address_space(3))) void* lds_ptr;
@@ -127,11 +128,12 @@ __device__ inline void dma16(void const* g, void* lds) {
   asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "{m0}"(m0) : "memory");
 }
 
-template <int N, int NT, class E>
-__device__ inline void prefetch_rows_lds16(E const* __restrict__ x, int64_t ld, Lane const& L,
-                                           unsigned short* __restrict__ buf) {
+template <int N, int NT, class X>
+__device__ inline void prefetch_rows_lds16(X const* __restrict__ x, int64_t ld, Lane const& L,
+                                           X* __restrict__ buf) {
   constexpr int T = (N + 15) / 16;
-  constexpr int PR = 2 * NT;  // 16-byte pieces per row
+  constexpr int PE = 16 / int(sizeof(X));  // columns per piece
+  constexpr int PR = 16 * NT / PE;         // 16-byte pieces per row
   static_assert(16 * PR % 64 == 0, "whole instructions per tile");
 #pragma unroll
   for (int i = 0; i < T * 16 * PR / 64; i++) {
@@ -139,14 +141,14 @@ __device__ inline void prefetch_rows_lds16(E const* __restrict__ x, int64_t ld, 
     int const slot = piece / PR, k = piece % PR;
     int const r = (slot & ~15) | ((slot & 3) << 2) | ((slot >> 2) & 3);
     if (N % 16 == 0 || r < N)
-      dma16(x + int64_t(r) * ld + L.col0 + 8 * k, buf + 64 * 8 * i);
+      dma16(x + int64_t(r) * ld + L.col0 + PE * k, buf + 64 * PE * i);
   }
 }
 
 // The lane's tile elements from a prefetched buf (row f = 16m + 4g + e in
 // slot 16m + 4e + g); rows >= N read 0.
-template <int N, int NT, class E>
-__device__ inline H<(N + 15) / 16, NT, E> load_rows_lds16(unsigned short const* __restrict__ buf, Lane const& L) {
+template <int N, int NT, class E, class X>
+__device__ inline H<(N + 15) / 16, NT, E> load_rows_lds16(X const* __restrict__ buf, Lane const& L) {
   constexpr int T = (N + 15) / 16;
   H<T, NT, E> s;
 #pragma unroll
@@ -156,8 +158,8 @@ __device__ inline H<(N + 15) / 16, NT, E> load_rows_lds16(unsigned short const* 
 #pragma unroll
       for (int e = 0; e < 4; e++) {
         int const f = 16 * m + 4 * L.g + e;
-        unsigned short const bits = buf[(16 * m + 4 * e + L.g) * (16 * NT) + 16 * n + L.c];
-        s.v[m][n][e] = (N % 16 == 0 || f < N) ? __builtin_bit_cast(E, bits) : E(0.0f);
+        E const v = static_cast<E>(buf[(16 * m + 4 * e + L.g) * (16 * NT) + 16 * n + L.c]);
+        s.v[m][n][e] = (N % 16 == 0 || f < N) ? v : E(0.0f);
       }
   return s;
 }
@@ -167,9 +169,9 @@ __device__ inline H<(N + 15) / 16, NT, E> load_rows_lds16(unsigned short const* 
 __device__ inline void wait_vmem() { __builtin_amdgcn_s_waitcnt(0x0F70); }
 __device__ inline void wait_lds() { __builtin_amdgcn_s_waitcnt(0xC07F); }
 
-template <int N, int T, int NT, class E>
-__device__ inline void store_rows_h(H<T, NT, E> const& s, E* __restrict__ y, int64_t ld, Lane const& L) {
-  E* __restrict__ yl = lane_ptr(y, ld, L);
+template <int N, int T, int NT, class E, class Y>
+__device__ inline void store_rows_h(H<T, NT, E> const& s, Y* __restrict__ y, int64_t ld, Lane const& L) {
+  Y* __restrict__ yl = lane_ptr(y, ld, L);
   bool const full = L.col0 + 16 * NT <= L.batch;
 #pragma unroll
   for (int m = 0; m < T; m++)
@@ -179,7 +181,7 @@ __device__ inline void store_rows_h(H<T, NT, E> const& s, E* __restrict__ y, int
 #pragma unroll
       for (int e = 0; e < 4; e++) {
         int const f = 16 * m + 4 * L.g + e;
-        if ((N % 16 == 0 || f < N) && col_ok) yl[int64_t(16 * m + e) * ld + 16 * n] = s.v[m][n][e];
+        if ((N % 16 == 0 || f < N) && col_ok) yl[int64_t(16 * m + e) * ld + 16 * n] = static_cast<Y>(s.v[m][n][e]);
       }
     }
 }
@@ -187,26 +189,29 @@ __device__ inline void store_rows_h(H<T, NT, E> const& s, E* __restrict__ y, int
 // Transposed tile (a dense layer run with its MFMA operands swapped, fused
 // dense_hs<..., TR = true>): lane l, element e <-> feature 16m + c, column
 // col0 + 16n + 4g + e, so each lane's 4 elements are consecutive columns of
-// one output row.  Whole tiles of an 8-byte aligned y with a row stride of a
-// multiple of 4 elements (vec_ok) store them as one 8-byte write; otherwise
+// one output row.  Whole tiles of a y aligned to 4 elements with a row stride
+// of a multiple of 4 elements (vec_ok) store them as one write; otherwise
 // element by element inside the batch.  Rows >= N are not written.
-template <int N, int T, int NT, class E>
-__device__ inline void store_rows_ht(H<T, NT, E> const& s, E* __restrict__ y, int64_t ld, Lane const& L,
+template <class Y> struct Vec4Of { typedef Y type __attribute__((ext_vector_type(4))); };
+template <int N, int T, int NT, class E, class Y>
+__device__ inline void store_rows_ht(H<T, NT, E> const& s, Y* __restrict__ y, int64_t ld, Lane const& L,
                                      bool vec_ok) {
+  using Y4 = typename Vec4Of<Y>::type;
   bool const full = vec_ok && L.col0 + 16 * NT <= L.batch;
 #pragma unroll
   for (int m = 0; m < T; m++) {
     int const f = 16 * m + L.c;
     if (N % 16 != 0 && f >= N) continue;
-    E* __restrict__ yr = y + int64_t(f) * ld + L.col0 + 4 * L.g;
+    Y* __restrict__ yr = y + int64_t(f) * ld + L.col0 + 4 * L.g;
 #pragma unroll
     for (int n = 0; n < NT; n++) {
+      Y4 const o = __builtin_convertvector(s.v[m][n], Y4);
       if (full) {
-        *reinterpret_cast<typename Vec<E>::x4*>(yr + 16 * n) = s.v[m][n];
+        *reinterpret_cast<Y4*>(yr + 16 * n) = o;
       } else {
 #pragma unroll
         for (int e = 0; e < 4; e++)
-          if (L.col0 + 16 * n + 4 * L.g + e < L.batch) yr[16 * n + e] = s.v[m][n][e];
+          if (L.col0 + 16 * n + 4 * L.g + e < L.batch) yr[16 * n + e] = o[e];
       }
     }
   }

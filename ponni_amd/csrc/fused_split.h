@@ -231,9 +231,10 @@ __device__ inline H<TO, NT, E> split_get_h(typename Vec<E>::x4 const* __restrict
 }
 
 // Own tiles of the output: row-major tiles, or transposed ones (TR).
-template <int N, int TO, int W, bool TR, int OWN, int NT, class E>
-__device__ inline void split_store_h(H<OWN, NT, E> const& own, E* __restrict__ y, int64_t ld, int wave, Lane const& L,
+template <int N, int TO, int W, bool TR, int OWN, int NT, class E, class Y>
+__device__ inline void split_store_h(H<OWN, NT, E> const& own, Y* __restrict__ y, int64_t ld, int wave, Lane const& L,
                                      bool vec_ok) {
+  using Y4 = typename Vec4Of<Y>::type;
 #pragma unroll
   for (int o = 0; o < OWN; o++) {
     int const mo = wave + W * o;
@@ -241,25 +242,26 @@ __device__ inline void split_store_h(H<OWN, NT, E> const& own, E* __restrict__ y
     if (TR) {
       int const f = 16 * mo + L.c;
       if (N % 16 != 0 && f >= N) continue;
-      E* __restrict__ yr = y + int64_t(f) * ld + L.col0 + 4 * L.g;
+      Y* __restrict__ yr = y + int64_t(f) * ld + L.col0 + 4 * L.g;
       bool const full = vec_ok && L.col0 + 16 * NT <= L.batch;
 #pragma unroll
       for (int n = 0; n < NT; n++) {
+        Y4 const v = __builtin_convertvector(own.v[o][n], Y4);
         if (full) {
-          *reinterpret_cast<typename Vec<E>::x4*>(yr + 16 * n) = own.v[o][n];
+          *reinterpret_cast<Y4*>(yr + 16 * n) = v;
         } else {
 #pragma unroll
           for (int e = 0; e < 4; e++)
-            if (L.col0 + 16 * n + 4 * L.g + e < L.batch) yr[16 * n + e] = own.v[o][n][e];
+            if (L.col0 + 16 * n + 4 * L.g + e < L.batch) yr[16 * n + e] = v[e];
         }
       }
     } else {
-      E* __restrict__ yl = y + (int64_t(16 * mo + 4 * L.g) * ld + L.col0 + L.c);
+      Y* __restrict__ yl = y + (int64_t(16 * mo + 4 * L.g) * ld + L.col0 + L.c);
 #pragma unroll
       for (int n = 0; n < NT; n++)
 #pragma unroll
         for (int e = 0; e < 4; e++)
-          if (16 * mo + 4 * L.g + e < N && L.col0 + 16 * n + L.c < L.batch) yl[int64_t(e) * ld + 16 * n] = own.v[o][n][e];
+          if (16 * mo + 4 * L.g + e < N && L.col0 + 16 * n + L.c < L.batch) yl[int64_t(e) * ld + 16 * n] = static_cast<Y>(own.v[o][n][e]);
     }
   }
 }

@@ -48,10 +48,11 @@ __device__ inline bool vec_ok(void const* p, int64_t ld) {
   return (reinterpret_cast<unsigned long long>(p) % (sizeof(S) * V)) == 0 && ld % V == 0;
 }
 
-// s[f][v] = x(f, b0 + v) for f < N; rows >= N and samples >= batch are 0.
-template <class S, int V, int N, int W, class C>
-__device__ inline void load(C (&s)[W][V], S const* __restrict__ x, int64_t ld, int64_t b0, int64_t batch, bool vec) {
-  typedef typename VecOf<S, V>::type SV;
+// s[f][v] = x(f, b0 + v) rounded to S for f < N; rows >= N and samples >=
+// batch are 0.  (x and y of a 16-bit plan may hold floats.)
+template <class S, int V, int N, int W, class C, class X>
+__device__ inline void load(C (&s)[W][V], X const* __restrict__ x, int64_t ld, int64_t b0, int64_t batch, bool vec) {
+  typedef typename VecOf<X, V>::type SV;
 #pragma unroll
   for (int f = 0; f < W; f++)
 #pragma unroll
@@ -61,26 +62,26 @@ __device__ inline void load(C (&s)[W][V], S const* __restrict__ x, int64_t ld, i
     for (int f = 0; f < N; f++) {
       SV const r = *reinterpret_cast<SV const*>(x + int64_t(f) * ld + b0);
 #pragma unroll
-      for (int v = 0; v < V; v++) s[f][v] = static_cast<C>(r[v]);
+      for (int v = 0; v < V; v++) s[f][v] = static_cast<C>(static_cast<S>(r[v]));
     }
   } else {
 #pragma unroll
     for (int f = 0; f < N; f++)
 #pragma unroll
       for (int v = 0; v < V; v++)
-        if (b0 + v < batch) s[f][v] = static_cast<C>(x[int64_t(f) * ld + b0 + v]);
+        if (b0 + v < batch) s[f][v] = static_cast<C>(static_cast<S>(x[int64_t(f) * ld + b0 + v]));
   }
 }
 
-template <class S, int V, int N, int W, class C>
-__device__ inline void store(C const (&s)[W][V], S* __restrict__ y, int64_t ld, int64_t b0, int64_t batch, bool vec) {
-  typedef typename VecOf<S, V>::type SV;
+template <class S, int V, int N, int W, class C, class Y>
+__device__ inline void store(C const (&s)[W][V], Y* __restrict__ y, int64_t ld, int64_t b0, int64_t batch, bool vec) {
+  typedef typename VecOf<Y, V>::type SV;
   if (vec) {
 #pragma unroll
     for (int f = 0; f < N; f++) {
       SV r;
 #pragma unroll
-      for (int v = 0; v < V; v++) r[v] = static_cast<S>(s[f][v]);
+      for (int v = 0; v < V; v++) r[v] = static_cast<Y>(static_cast<S>(s[f][v]));
       *reinterpret_cast<SV*>(y + int64_t(f) * ld + b0) = r;
     }
   } else {
@@ -88,7 +89,7 @@ __device__ inline void store(C const (&s)[W][V], S* __restrict__ y, int64_t ld, 
     for (int f = 0; f < N; f++)
 #pragma unroll
       for (int v = 0; v < V; v++)
-        if (b0 + v < batch) y[int64_t(f) * ld + b0 + v] = static_cast<S>(s[f][v]);
+        if (b0 + v < batch) y[int64_t(f) * ld + b0 + v] = static_cast<Y>(static_cast<S>(s[f][v]));
   }
 }
 

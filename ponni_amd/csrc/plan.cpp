@@ -1019,9 +1019,9 @@ int upload(ponni_plan_s& p) {
     p.d_params_bytes = bytes;
   }
   if (count > 0) HIP_TRY(hipMemcpy(p.d_params, packed, count * param_element_size(p), hipMemcpyHostToDevice));
-  if ((p.path == PONNI_PATH_FUSED || p.narrow_jit) && p.fused_fn == nullptr) {
+  if ((p.path == PONNI_PATH_FUSED || p.narrow_jit) && p.kernels[0][0].fn == nullptr) {
     std::string error;
-    int const st = fused_prepare(p, error);
+    int const st = fused_prepare(p, false, false, error);
     if (st != PONNI_OK) return fail(st, error);
   }
   int const st = build_gather(p);
@@ -1431,7 +1431,7 @@ hipError_t layered_forward(ponni_plan_s const& p, LaunchArgs a, hipStream_t stre
 }
 
 int forward_impl(ponni_plan plan, const void* x, int64_t ld_in, void* y, int64_t ld_out, int64_t batch,
-                 hipStream_t stream, hipEvent_t ev_start, hipEvent_t ev_stop, bool no_alloc) {
+                 hipStream_t stream, hipEvent_t ev_start, hipEvent_t ev_stop, bool no_alloc, bool io32) {
   if (plan == nullptr) return fail(PONNI_ERR_INVALID_ARGUMENT, "plan is null");
   if (plan->external)
     return fail(PONNI_ERR_UNSUPPORTED, "the plan holds external (custom) layers: run it through ponni_plan_device_model");
@@ -1462,13 +1462,24 @@ int forward_impl(ponni_plan plan, const void* x, int64_t ld_in, void* y, int64_t
     HIP_TRY(hipGetDevice(&dev));
     if (dev != plan->device) return fail(PONNI_ERR_DEVICE, "plan was first used on another device");
   }
-  // (A captured stream cannot load a module: a plan whose small-batch kernel
-  // is not there yet then runs its other kernel, which takes any batch.)
-  if (plan->split_fn == nullptr && !no_alloc && fused_wants_split(*plan, batch)) {
+  // The kernels of this call that are not loaded yet.  (A captured stream
+  // cannot load a module: a plan whose small-batch kernel is not there yet
+  // then runs its other kernel, which takes any batch.)
+  bool const need_rows = io32 && plan->kernels[1][0].fn == nullptr;
+  bool const need_split = !no_alloc && plan->kernels[io32][1].fn == nullptr && fused_wants_split(*plan, batch);
+  if (need_rows || need_split) {
     hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(stream, &capturing) == hipSuccess && capturing == hipStreamCaptureStatusNone) {
-      std::string error;
-      int const st = fused_prepare_split(*plan, error);
+    bool const can_load =
+        hipStreamIsCapturing(stream, &capturing) == hipSuccess && capturing == hipStreamCaptureStatusNone;
+    if (need_rows && !can_load)
+      return fail(PONNI_ERR_UNSUPPORTED, "fp32 rows: the kernel is not loaded yet, and the stream is being captured");
+    std::string error;
+    if (need_rows) {
+      int const st = fused_prepare(*plan, true, false, error);
+      if (st != PONNI_OK) return fail(st, error);
+    }
+    if (need_split && can_load) {
+      int const st = fused_prepare(*plan, io32, true, error);
       if (st != PONNI_OK) return fail(st, error);
     }
   }
@@ -1532,11 +1543,11 @@ int forward_impl(ponni_plan plan, const void* x, int64_t ld_in, void* y, int64_t
   }
   switch (plan->path) {
     case PONNI_PATH_NARROW:
-      err = plan->narrow_jit ? fused_launch(*plan, a, stream)
+      err = plan->narrow_jit ? fused_launch(*plan, a, io32, stream)
                              : launch_narrow(plan->dtype, plan->width_class, plan->num_slots, a, stream);
       break;
     case PONNI_PATH_MFMA: err = launch_mfma(plan->dtype, plan->width_class, plan->num_slots, a, stream); break;
-    case PONNI_PATH_FUSED: err = fused_launch(*plan, a, stream); break;
+    case PONNI_PATH_FUSED: err = fused_launch(*plan, a, io32, stream); break;
     case PONNI_PATH_LAYERED: err = layered_forward(*plan, a, stream); break;
     default: err = launch_generic(plan->dtype, a, stream); break;
   }
@@ -1548,18 +1559,27 @@ int forward_impl(ponni_plan plan, const void* x, int64_t ld_in, void* y, int64_t
 
 int ponni_forward(ponni_plan plan, const void* x, int64_t ld_in, void* y, int64_t ld_out, int64_t batch,
                   hipStream_t stream) {
-  return forward_impl(plan, x, ld_in, y, ld_out, batch, stream, nullptr, nullptr, false);
+  return forward_impl(plan, x, ld_in, y, ld_out, batch, stream, nullptr, nullptr, false, false);
 }
 
 int ponni_forward_no_alloc(ponni_plan plan, const void* x, int64_t ld_in, void* y, int64_t ld_out, int64_t batch,
                            hipStream_t stream) {
-  return forward_impl(plan, x, ld_in, y, ld_out, batch, stream, nullptr, nullptr, true);
+  return forward_impl(plan, x, ld_in, y, ld_out, batch, stream, nullptr, nullptr, true, false);
 }
 
 int ponni_forward_timed(ponni_plan plan, const void* x, int64_t ld_in, void* y, int64_t ld_out, int64_t batch,
                         hipStream_t stream, hipEvent_t start, hipEvent_t stop) {
   if (start == nullptr || stop == nullptr) return fail(PONNI_ERR_INVALID_ARGUMENT, "timing events are null");
-  return forward_impl(plan, x, ld_in, y, ld_out, batch, stream, start, stop, false);
+  return forward_impl(plan, x, ld_in, y, ld_out, batch, stream, start, stop, false, false);
+}
+
+int ponni_forward_fp32_rows(ponni_plan plan, const float* x, int64_t ld_in, float* y, int64_t ld_out, int64_t batch,
+                            hipStream_t stream) {
+  if (plan == nullptr) return fail(PONNI_ERR_INVALID_ARGUMENT, "plan is null");
+  bool const half = plan->dtype == PONNI_F16 || plan->dtype == PONNI_BF16;
+  if (!half || !(plan->path == PONNI_PATH_FUSED || plan->narrow_jit))
+    return fail(PONNI_ERR_UNSUPPORTED, "fp32 rows: a 16-bit plan on FUSED or generated NARROW");
+  return forward_impl(plan, x, ld_in, y, ld_out, batch, stream, nullptr, nullptr, false, true);
 }
 
 int ponni_forward_steps(ponni_plan plan, const void* const* x, int64_t ld_in, void* const* y, int64_t ld_out,

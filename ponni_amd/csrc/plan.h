@@ -54,6 +54,14 @@ inline void launch_kernel(F kernel, dim3 grid, dim3 block, uint32_t shmem, hipSt
     (void)hipLaunchKernel(fn, grid, block, argv, shmem, stream);
 }
 
+// A generated kernel on the device.
+struct FusedKernel {
+  hipFunction_t fn = nullptr;
+  int columns_per_block = 128;
+  int waves = 4;         // per workgroup
+  int64_t resident = 0;  // a persistent grid's workgroups (0: one per column block)
+};
+
 // Kinds of packed parameter slots (plan.cpp visit_param_slots).
 enum SlotKind { SLOT_VALUE = 0, SLOT_HALF = 1, SLOT_WORD = 2 };
 
@@ -190,21 +198,18 @@ struct ponni_plan_s {
   uint64_t host_version = 0;
   // NARROW plans run a generated kernel (narrow_jit.h) unless JIT is off.
   bool narrow_jit = false;
-  // FUSED path (and generated NARROW): the plan's generated kernel (compiled on first forward).
-  hipFunction_t fused_fn = nullptr;
-  int fused_blocks_per_cu = 1;
-  int fused_cus = 0;              // compute units of the plan's device
-  bool fused_persistent = false;  // grid sized to the resident workgroups
-  int fused_columns_per_block = 128;
-  int fused_waves = 4;  // waves per workgroup
-  int fused_wps = 0;    // waves per SIMD the kernel is compiled for (0: not settled yet)
-  // Its small-batch kernel (fused_split.h), loaded by the first forward of a
-  // batch that runs on it; until then every batch runs on fused_fn.
-  hipFunction_t split_fn = nullptr;
-  int split_columns_per_block = 16;
-  int split_waves = 4;
-  double split_ratio = 0;     // its time per column over fused_fn's (0: the plan has none)
-  bool split_always = false;  // it is the faster one at every batch
+  // FUSED path (and generated NARROW): the plan's generated kernels,
+  // kernels[fp32 rows][small batch].  kernels[0][0], the main one, is loaded when
+  // the plan is put on the device; the small-batch kernels (fused_split.h) and
+  // those of a 16-bit plan on fp32 rows by the first forward that runs on
+  // them.
+  ponni_hip::FusedKernel kernels[2][2];
+  int fused_cus = 0;  // compute units of the plan's device
+  int fused_wps = 0;  // waves per SIMD the main kernel is compiled for (0: not settled yet)
+  // The small-batch kernel's time per column over the main one's (0: the plan
+  // has none), and whether it is the faster one at every batch.
+  double split_ratio = 0;
+  bool split_always = false;
 
   // Parameter segments shared with caller-owned arrays (two per layer at
   // most), and the gather map that refreshes the device-shared ones.

@@ -1211,6 +1211,8 @@ class GeneratedModel:
         import torch
 
         self._check(x, y)
+        if self.plan("f16").forward_fp32_rows(x, y):
+            return
         xh = x.to(torch.float16)
         yh = torch.empty((self.num_outputs, x.shape[1]), dtype=torch.float16, device=x.device)
         self.plan("f16").forward_batch_parallel(xh, yh)

@@ -319,6 +319,28 @@ class Inference:
         from the library's fixed per-GPU scratch (ponni_forward_no_alloc)."""
         A.check(A.lib().ponni_forward_no_alloc(self._plan, x_ptr, ld_in, y_ptr, ld_out, batch, stream))
 
+    def forward_fp32_rows(self, x, y) -> bool:
+        """forward_batch_parallel of a 16-bit plan on fp32 GPU tensors
+        (ponni_forward_fp32_rows); False, with nothing done, where the plan or
+        the tensors do not allow it."""
+        import torch
+
+        if not (x.dtype == y.dtype == torch.float32 and x.is_cuda and x.device == y.device):
+            return False
+        B = x.shape[1]
+        sx, sy = x.stride(), y.stride()
+        if sx[1] != 1 or sy[1] != 1 or sx[0] < B or sy[0] < B:
+            return False
+        px, py = x.data_ptr(), y.data_ptr()
+        if px < py + 4 * ((y.shape[0] - 1) * sy[0] + B) and py < px + 4 * ((x.shape[0] - 1) * sx[0] + B):
+            return False  # overlapping views
+        st = A.lib().ponni_forward_fp32_rows(self._plan, px, sx[0], py, sy[0], B,
+                                             torch.cuda.current_stream(x.device).cuda_stream)
+        if st == A.PONNI_ERR_UNSUPPORTED:
+            return False
+        A.check(st)
+        return True
+
     def forward_raw_timed(self, x_ptr: int, ld_in: int, y_ptr: int, ld_out: int, batch: int, stream: int,
                           start_event: int, stop_event: int) -> None:
         """forward_raw whose kernel dispatch stamps two caller-created HIP events

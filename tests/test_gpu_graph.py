@@ -166,3 +166,47 @@ def test_generated_graphs_f64_fused(cuda, case):
     want = oracle.forward(layers, x, oracle.MODE_F64)
     got = y.cpu().numpy()
     assert np.allclose(got, want, rtol=1e-11, atol=1e-11 * max(1.0, np.abs(want).max())), np.abs(got - want).max()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", ["c5", "wide_in", "narrow"])
+def test_half2_on_fp32_rows_is_the_converted_call(cuda, shape):
+    """infer_batch_half2 reads and writes the fp32 views in the kernel: the
+    same bits as converting them around the fp16 plan's forward pass, for
+    small and large batches and rows at any alignment; overlapping views are
+    left to the conversion."""
+    import torch
+
+    if shape == "c5":
+        gr = C.c5_graph(True)
+    else:
+        n, w, o = (70, 40, 33) if shape == "wide_in" else (5, 7, 3)
+        r = np.random.default_rng(8)
+        g = G.GraphBuilder(n)
+        h = g.unary("Tanh", g.dense(g.input, r.uniform(-0.3, 0.3, (w, n)), r.uniform(-0.2, 0.2, w), name="a"))
+        gr = g.finish(g.dense(h, r.uniform(-0.3, 0.3, (o, w)), r.uniform(-0.2, 0.2, o), name="b"))
+    gm = G.GeneratedModel(gr)
+    plan = gm.plan("f16")
+    for B, pad, off in [(1, 0, 0), (33, 0, 0), (4096, 4, 0), (70_001, 0, 0), (200_000, 8, 1), (200_000, 8, 4)]:
+        print(f"half2 rows: {shape} B={B} pad={pad} off={off}", flush=True)
+        xs = torch.randn((gm.num_inputs, B + pad + off), device="cuda:0",
+                         generator=torch.Generator("cuda:0").manual_seed(B))
+        x = xs[:, off:off + B]
+        ys = torch.full((gm.num_outputs, B + pad + off), float("nan"), device="cuda:0")
+        y = ys[:, off:off + B]
+        gm.infer_batch_half2(x, y)
+        want = plan.forward_batch_parallel(x.to(torch.float16).contiguous()).float()
+        torch.cuda.synchronize()
+        assert torch.equal(y, want)
+        assert torch.isnan(ys[:, :off]).all() and torch.isnan(ys[:, off + B:]).all()
+    xt = torch.randn((4096, gm.num_inputs), device="cuda:0").t()  # column stride
+    y = torch.empty((gm.num_outputs, 4096), device="cuda:0")
+    assert not plan.forward_fp32_rows(xt, y)
+    with pytest.raises(AssertionError):  # refused, as by infer_batch
+        gm.infer_batch_half2(xt, y)
+    both = torch.randn((gm.num_inputs + gm.num_outputs, 4096), device="cuda:0")
+    x, y = both[:gm.num_inputs], both[:gm.num_outputs]
+    want = plan.forward_batch_parallel(x.to(torch.float16)).float()
+    assert not plan.forward_fp32_rows(x, y)
+    gm.infer_batch_half2(x, y)
+    assert torch.equal(y, want)
