@@ -426,8 +426,12 @@ std::string fused_source_once(ponni_plan_s const& p, FusedConfig& cfg, bool allo
     }
   }
   cfg.waves_per_simd = regs <= 128 ? 4 : regs <= 168 ? 3 : regs <= 256 ? 2 : 1;
+  bool const want_resident = cfg.resident && half && !cfg.split && NT == 2;
+  cfg.resident = false;
   if (half) cfg.waves_per_simd = half_wps;
-  if (p.fused_wps > 0) cfg.waves_per_simd = p.fused_wps;  // measured by fused_compile
+  // (measured by fused_compile)
+  if (want_resident && p.resident_wps > 0) cfg.waves_per_simd = p.resident_wps;
+  if (!want_resident && p.fused_wps > 0) cfg.waves_per_simd = p.fused_wps;
 
   // Waves per workgroup: LDS-staged parameters are copied once per
   // workgroup, so when copies would cap the resident workgroups below the
@@ -452,6 +456,36 @@ std::string fused_source_once(ponni_plan_s const& p, FusedConfig& cfg, bool allo
   // A workgroup of 16-bit plans is one wave per SIMD per occupancy level: its
   // waves share the staged A fragments and the activation table.
   if (half) cfg.waves = 4 * std::min(cfg.waves_per_simd, half_wps);
+  // 16-bit plans whose A fragments fit in LDS beside the vectors and input
+  // rows keep them there for the kernel's life: no staging requests and no
+  // barriers in the tile loop, and as many waves as the registers allow (the
+  // smallest workgroup that reaches them).
+  int64_t frag_bytes = 0;
+  int64_t vec_bytes = 0;  // (at most)
+  for (Op const& op : p.ops) {
+    if (op.code == OP_DENSE) frag_bytes += int64_t((tiles(op.n_in) + 1) / 2) * tiles(op.n_out) * 1024;
+    if (op.code == OP_PROJ_ADD) frag_bytes += int64_t((tiles(op.aux) + 1) / 2) * tiles(op.n_out) * 1024;
+    vec_bytes += int64_t(4 + op.epi_count) * 64 * std::max(tiles(op.n_in), tiles(op.n_out));
+  }
+  if (want_resident && frag_bytes > 0) {
+    int64_t const rows_per_wave = int64_t(tiles(p.layers.front().n_in)) * 16 * 16 * NT * (cfg.io32 ? 4 : 2);
+    int best = 0;
+    for (int w = 4; w <= 4 * cfg.waves_per_simd; w += 4) {
+      int64_t const lds = frag_bytes + vec_bytes + w * rows_per_wave;
+      int const by_lds = static_cast<int>(kFusedLdsBytes / lds);
+      int const waves = std::min(by_lds, 4 * cfg.waves_per_simd / w) * w;
+      if (waves > best) {
+        best = waves;
+        cfg.waves = w;
+      }
+    }
+    // (at least the staged form's two waves per SIMD)
+    cfg.resident = best >= 4 * std::min(cfg.waves_per_simd, half_wps);
+  }
+  if (want_resident && !cfg.resident) {
+    cfg.waves_per_simd = p.fused_wps > 0 ? p.fused_wps : half_wps;
+    cfg.waves = 4 * std::min(cfg.waves_per_simd, half_wps);
+  }
   cfg.columns_per_block = cfg.waves * 16 * NT;
   if (cfg.split) {
     cfg.waves = cfg.split_waves;
@@ -504,7 +538,20 @@ std::string fused_source_once(ponni_plan_s const& p, FusedConfig& cfg, bool allo
   for (Op const& op : p.ops)
     if (op.code == OP_DENSE) dense_seq.push_back(DenseRef{op.woff, (tiles(op.n_in) + 1) / 2, tiles(op.n_out)});
   int const slot_frags = 32, slots = 3;
-  if (half && !cfg.split && !dense_seq.empty()) {
+  std::map<int, int> frag_at;  // resident: packed offset of a layer's weights -> its first fragment in LDS
+  if (cfg.resident) {
+    int frags = 0;
+    std::ostringstream copies;
+    for (Op const& op : p.ops) {
+      if (op.code != OP_DENSE && op.code != OP_PROJ_ADD) continue;
+      int const n = (tiles(op.code == OP_DENSE ? op.n_in : op.aux) + 1) / 2 * tiles(op.n_out);
+      if (!frag_at.emplace(op.woff, frags).second) continue;
+      copies << "  stage_frags<E>(a_all + " << frags * 64 << ", gparams + " << op.woff << ", " << n << ");\n";
+      frags += n;
+    }
+    o << "  __shared__ Vec<E>::x8 a_all[" << frags * 64 << "];\n" << copies.str() << "  wait_vmem();\n  __syncthreads();\n";
+    cfg.persistent_loop = true;
+  } else if (half && !cfg.split && !dense_seq.empty()) {
     std::ostringstream tab;
     int chunks = 0;
     for (DenseRef const& d : dense_seq) {
@@ -563,16 +610,35 @@ std::string fused_source_once(ponni_plan_s const& p, FusedConfig& cfg, bool allo
   head << o.str();
   o.str("");
   o << "  Lane L;\n  L.lane = threadIdx.x & 63;\n  L.g = L.lane >> 4;\n  L.c = L.lane & 15;\n  L.batch = batch;\n";
-  o << "  int64_t const tiles = (batch + " << cfg.columns_per_block - 1 << ") / " << cfg.columns_per_block << ";\n";
+  // Persistent kernels with no barrier in the tile loop deal tiles of one wave's
+  // columns to the waves, wave 0 of every workgroup first, so that a batch
+  // spreads over all CUs and SIMDs whatever its size (whole workgroups of 12
+  // waves in turn: fp32 24-96-48-10 graph, 262,144 columns, a last round on 171 of
+  // 256 CUs, 61.5 us; this way 56).  16-bit rows: pairs of waves take
+  // neighbouring tiles, the two halves of a cache line.
+  cfg.by_wave = cfg.resident || (!half && !cfg.split && (cfg.lds_bytes > 0 || cfg.params_in_registers));
+  int const tile_columns = cfg.by_wave ? 16 * NT : cfg.columns_per_block;
+  o << "  int64_t const tiles = (batch + " << tile_columns - 1 << ") / " << tile_columns << ";\n";
+  std::string const first_tile = !cfg.by_wave ? "blockIdx.x"
+                                 : half       ? "(int64_t(wave_id() >> 1) * gridDim.x + blockIdx.x) * 2 + (wave_id() & 1)"
+                                              : "int64_t(wave_id()) * gridDim.x + blockIdx.x";
+  std::string const tile_step = cfg.by_wave ? "int64_t(gridDim.x) * " + std::to_string(cfg.waves) : "gridDim.x";
+  auto column_of = [&](std::string const& tile) {
+    std::string const c = std::to_string(16 * NT);
+    if (cfg.by_wave || cfg.split) return "(" + tile + ") * " + c;
+    return "((" + tile + ") * " + std::to_string(cfg.waves) + " + wave_id()) * " + c;
+  };
   // 16-bit plans request each tile's input rows into LDS one tile ahead
   // (fused_f16.h prefetch_rows_lds16) when the buffer fits next to the staged
   // A fragments (3 slots of 32 KB) and vectors.
   int const n_in0 = p.layers.front().n_in;
   int const in_rows_elems = tiles(n_in0) * 16 * 16 * NT;  // per wave, row-major 16-bit
   int const in_dma_bytes = cfg.waves * in_rows_elems * io_bytes;
-  int const stage_bytes = half && !cfg.split && !dense_seq.empty() ? slots * slot_frags * 1024 : 0;
-  bool const in_dma = half && !cfg.split && NT % 2 == 0 && in_dma_bytes <= 64 * 1024 &&
-                      in_dma_bytes + stage_bytes + 16 * 1024 <= kFusedLdsBytes;
+  int const stage_bytes = cfg.resident ? static_cast<int>(frag_bytes)
+                          : half && !cfg.split && !dense_seq.empty() ? slots * slot_frags * 1024 : 0;
+  bool const in_dma = half && !cfg.split && NT % 2 == 0 &&
+                      (cfg.resident || (in_dma_bytes <= 64 * 1024 &&
+                                        in_dma_bytes + stage_bytes + 16 * 1024 <= kFusedLdsBytes));
   std::string const WCOLS = std::to_string(16 * NT), NW = std::to_string(cfg.waves);
   // The next tile's rows are requested inside the second dense layer, right
   // after its first chunk's weight loads (fused_f16.h dense_hs hook): waits
@@ -603,8 +669,8 @@ std::string fused_source_once(ponni_plan_s const& p, FusedConfig& cfg, bool allo
     // Whole tiles of a 16-byte aligned x with a row stride of a multiple of
     // 16 bytes go through LDS; others (the batch's last tile) load directly.
     o << "  bool const xvec = ((reinterpret_cast<uint64_t>(x) | uint64_t(ldx) * " << io_bytes << ") & 15) == 0;\n";
-    o << "  L.col0 = (int64_t(blockIdx.x) * " << NW << " + wave_id()) * " << WCOLS << ";\n";
-    o << "  if (blockIdx.x < tiles && xvec && L.col0 + " << WCOLS << " <= batch) prefetch_rows_lds16<" << n_in0 << ", "
+    o << "  int64_t const tile0 = " << first_tile << ";\n  L.col0 = " << column_of("tile0") << ";\n";
+    o << "  if (tile0 < tiles && xvec && L.col0 + " << WCOLS << " <= batch) prefetch_rows_lds16<" << n_in0 << ", "
       << NT << ">(x, ldx, L, in_buf[wave_id()]);\n";
     // The LDS writes of these loads complete with vmcnt, which the compiler
     // does not track (fused_f16.h dma16): each tile's rows are waited for
@@ -615,12 +681,12 @@ std::string fused_source_once(ponni_plan_s const& p, FusedConfig& cfg, bool allo
   // (the small-batch kernel runs one tile per workgroup: its exchange buffers
   // alternate within a tile only)
   if (cfg.split) o << "  if (int64_t const tile = blockIdx.x; tile < tiles) {\n";
-  else o << "  for (int64_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {\n";
-  if (cfg.split) o << "    L.col0 = tile * " << 16 * NT << ";\n";
-  else o << "    L.col0 = (tile * " << cfg.waves << " + wave_id()) * " << 16 * NT << ";\n";
+  else o << "  for (int64_t tile = " << (in_dma ? "tile0" : first_tile) << "; tile < tiles; tile += " << tile_step << ") {\n";
+  o << "    L.col0 = " << column_of("tile") << ";\n";
   // Register-resident parameters may be hoisted out of the tile loop; otherwise
   // pin() hides the pointer's loop invariance so they are re-read per tile.
   o << "    " << F << " const* __restrict__ P = " << (cfg.params_in_registers ? "P0;\n" : "pin(P0);\n");
+  if (cfg.resident) o << "    Vec<E>::x8 const* __restrict__ AL = pin(a_all);\n";
   int var = 0;
   auto fresh = [&]() { return "s" + std::to_string(var++); };
   std::string cur = fresh();
@@ -629,8 +695,8 @@ std::string fused_source_once(ponni_plan_s const& p, FusedConfig& cfg, bool allo
     o << "    auto " << cur << " = xvec && L.col0 + " << WCOLS << " <= batch ? load_rows_lds16<" << cur_n << ", " << NT
       << ", E>(in_buf[wave_id()], L) : load_rows_h<" << cur_n << ", " << NT << ", E>(x, ldx, L);\n";
     o << "    wait_lds();\n";
-    o << "    Lane Ln = L;\n    Ln.col0 = ((tile + gridDim.x) * " << NW << " + wave_id()) * " << WCOLS << ";\n";
-    o << "    bool const pre_next = tile + gridDim.x < tiles && xvec && Ln.col0 + " << WCOLS << " <= batch;\n";
+    o << "    Lane Ln = L;\n    Ln.col0 = " << column_of("tile + " + tile_step) << ";\n";
+    o << "    bool const pre_next = tile + " << tile_step << " < tiles && xvec && Ln.col0 + " << WCOLS << " <= batch;\n";
     if (hook_dense < 0) o << "    " << prefetch_next << "\n";
   } else if (half) o << "    auto " << cur << " = load_rows_h<" << cur_n << ", " << NT << ", E>(x, ldx, L);\n";
   else o << "    auto " << cur << " = " << (in_k.empty() ? "load_rows<" : "load_rows_k<") << cur_n << ">(x, ldx, L);\n";
@@ -744,11 +810,18 @@ std::string fused_source_once(ponni_plan_s const& p, FusedConfig& cfg, bool allo
                                    : tr  ? "SeedRowsT{" + vec(p.steps[op.epi_begin].off, n) + ", L.c}"
                                          : "SeedRows{" + vec(p.steps[op.epi_begin].off, n) + ", L.g}";
           dense_index++;
-          o << "    auto " << nv << " = dense_hs<" << tiles(op.n_in) << ", " << tiles(n) << ", " << NT << ", "
-            << cfg.waves << (tr || hook ? tr ? ", true" : ", false" : "") << (hook ? ", 0" : "") << ">(" << cur
-            << ", st, L, " << init << ", [&](int mo, floatx4 (&t)[" << NT << "], Vec<E>::x4 (&o)[" << NT
+          if (cfg.resident) {
+            if (hook) o << "    " << prefetch_next << "\n";
+            o << "    auto " << nv << " = dense_hr<" << tiles(op.n_in) << ", " << tiles(n) << ", " << NT
+              << (tr ? ", true" : "") << ">(" << cur << ", AL + " << frag_at[op.woff] * 64;
+          } else {
+            o << "    auto " << nv << " = dense_hs<" << tiles(op.n_in) << ", " << tiles(n) << ", " << NT << ", "
+              << cfg.waves << (tr || hook ? tr ? ", true" : ", false" : "") << (hook ? ", 0" : "") << ">(" << cur
+              << ", st";
+          }
+          o << ", L, " << init << ", [&](int mo, floatx4 (&t)[" << NT << "], Vec<E>::x4 (&o)[" << NT
             << "]) {\n";
-          if (hook) dense_hook = "    }, [&] { " + prefetch_next + " });\n";
+          if (hook && !cfg.resident) dense_hook = "    }, [&] { " + prefetch_next + " });\n";
           if (tr) pad_ok = false;
         } else {
           std::string const init = seed ? "bias_rows<" + std::to_string(tiles(n)) + ">(" + vec(p.steps[op.epi_begin].off, n) + ", L)"
@@ -894,7 +967,10 @@ std::string fused_source_once(ponni_plan_s const& p, FusedConfig& cfg, bool allo
           cur = nv;
         } else if (half) {
           o << "    proj_add_h<" << tiles(sv.second) << ", " << tiles(cur_n) << ", " << cur_n << ">(" << cur << ", " << sv.first
-            << ", reinterpret_cast<E const*>(P + " << op.woff << "), " << vec(op.boff, cur_n) << ", L);\n";
+            << ", reinterpret_cast<E const*>(";
+          if (cfg.resident) o << "AL + " << frag_at[op.woff] * 64;
+          else o << "P + " << op.woff;
+          o << "), " << vec(op.boff, cur_n) << ", L);\n";
         } else {
           // The bias seeds the accumulators; each finished tile adds the
           // state's tile (proj + in, the same sum as in + proj).
@@ -987,7 +1063,7 @@ std::string fused_source_once(ponni_plan_s const& p, FusedConfig& cfg, bool allo
   // have landed (with staging, every request but the last chunk's is done,
   // and the rows were requested before it).
   if (half && in_dma)
-    o << (stage_bytes > 0 ? "    wait_vmem_n<chunk_requests<" + NW + ">()>();\n" : std::string("    wait_vmem();\n"));
+    o << (stage_bytes > 0 && !cfg.resident ? "    wait_vmem_n<chunk_requests<" + NW + ">()>();\n" : std::string("    wait_vmem();\n"));
   // (one wave's share of the stores where every wave holds the output)
   if (stored) {
   } else if (cfg.split) {
@@ -1294,14 +1370,25 @@ int compile_cached(ponni_plan_s const& p, FusedConfig cfg, std::string& key, std
 // estimated waves per SIMD; with register spills it is recompiled for one
 // wave fewer, and when it fits the next occupancy's register budget (512 /
 // waves, a multiple of 8) without spills it moves up one.
-int fused_compile(ponni_plan_s& p, std::string& key, std::vector<char>& code, std::string& error) {
-  if (p.path == PONNI_PATH_FUSED && p.fused_wps == 0) {
-    FusedConfig est;
+int fused_compile(ponni_plan_s& p, bool resident, std::string& key, std::vector<char>& code, std::string& error) {
+  FusedConfig est;
+  if (resident) {
+    est.resident = true;
     (void)fused_source(p, est);
+    resident = est.resident;
+  }
+  FusedConfig request;
+  request.resident = resident;
+  int& settled = resident ? p.resident_wps : p.fused_wps;
+  if (p.path == PONNI_PATH_FUSED && settled == 0) {
+    if (!resident) {
+      est = FusedConfig{};
+      (void)fused_source(p, est);
+    }
     int wps = est.waves_per_simd;
     auto spills_regs = [&](int w, int& spills, int& regs) -> int {
-      p.fused_wps = w;
-      int const st = compile_cached(p, FusedConfig{}, key, code, error);
+      settled = w;
+      int const st = compile_cached(p, request, key, code, error);
       if (st != PONNI_OK) return st;
       spills = metadata_int(code, ".vgpr_spill_count");
       int const v = metadata_int(code, ".vgpr_count"), a = metadata_int(code, ".agpr_count");
@@ -1322,6 +1409,12 @@ int fused_compile(ponni_plan_s& p, std::string& key, std::vector<char>& code, st
     int spills = 0, regs = 0;
     int st = spills_regs(wps, spills, regs);
     if (st != PONNI_OK) return st;
+    // Resident 16-bit plans: straight to the occupancy their registers allow.
+    if (resident && spills == 0 && regs <= 168) {
+      wps = regs <= 128 ? 4 : 3;
+      st = spills_regs(wps, spills, regs);
+      if (st != PONNI_OK) return st;
+    }
     while (spills > tolerated(wps) && wps > 1) {
       wps--;
       st = spills_regs(wps, spills, regs);
@@ -1334,9 +1427,9 @@ int fused_compile(ponni_plan_s& p, std::string& key, std::vector<char>& code, st
       if (st != PONNI_OK) return st;
       if (up_spills == 0) wps = wps + 1;
     }
-    p.fused_wps = wps;
+    settled = wps;
   }
-  return compile_cached(p, FusedConfig{}, key, code, error);
+  return compile_cached(p, request, key, code, error);
 }
 
 namespace {
@@ -1415,8 +1508,9 @@ int fused_prepare(ponni_plan_s& p, bool io32, bool split, std::string& error) {
   FusedConfig cfg;
   cfg.io32 = io32;
   cfg.split = split;
+  cfg.resident = !split;
   bool const main = !io32 && !split;  // (settles the plan's occupancy)
-  int st = main ? fused_compile(p, key, code, error) : compile_cached(p, cfg, key, code, error);
+  int st = main ? fused_compile(p, true, key, code, error) : compile_cached(p, cfg, key, code, error);
   if (st != PONNI_OK) return st;
   (void)fused_source(p, cfg);
   int dev = 0;
@@ -1432,6 +1526,7 @@ int fused_prepare(ponni_plan_s& p, bool io32, bool split, std::string& error) {
   FusedKernel& k = p.kernels[io32][split];
   k.columns_per_block = cfg.columns_per_block;
   k.waves = cfg.waves;
+  k.wave_columns = cfg.by_wave ? cfg.columns_per_block / cfg.waves : 0;
   k.resident = 0;
   if (!split && (cfg.lds_bytes > 0 || cfg.vec_bytes > 0 || cfg.params_in_registers || cfg.persistent_loop))
     k.resident = int64_t(p.fused_cus) * (m->blocks_per_cu > 0 ? m->blocks_per_cu : 1);
@@ -1466,14 +1561,20 @@ int fused_prepare(ponni_plan_s& p, bool io32, bool split, std::string& error) {
 bool fused_wants_split(ponni_plan_s const& p, int64_t batch) {
   if (p.path != PONNI_PATH_FUSED || p.split_ratio <= 0) return false;
   if (p.split_always) return true;
-  double const rounds = double(batch) / (double(p.fused_cus) * p.kernels[0][0].columns_per_block);
-  return rounds <= 2 && 0.25 + p.split_ratio * rounds < (rounds <= 1 ? 1 : 2);
+  FusedKernel const& main = p.kernels[0][0];
+  // (tiles dealt to waves: one wave per SIMD everywhere is the flat part; more
+  // waves then share the SIMDs instead of taking a second round)
+  int const columns = main.wave_columns > 0 ? 4 * main.wave_columns : main.columns_per_block;
+  double const rounds = double(batch) / (double(p.fused_cus) * columns);
+  return rounds <= (main.wave_columns > 0 ? 1 : 2) && 0.25 + p.split_ratio * rounds < (rounds <= 1 ? 1 : 2);
 }
 
 hipError_t fused_launch(ponni_plan_s const& p, LaunchArgs const& a, bool io32, hipStream_t stream) {
   bool const split = p.kernels[io32][1].fn != nullptr && fused_wants_split(p, a.batch);
   FusedKernel const& k = p.kernels[io32][split];
-  int64_t grid = (a.batch + k.columns_per_block - 1) / k.columns_per_block;
+  // (a persistent grid whose tiles go to waves takes every CU it has tiles for)
+  int64_t const columns = k.wave_columns > 0 ? k.wave_columns : k.columns_per_block;
+  int64_t grid = (a.batch + columns - 1) / columns;
   if (k.resident > 0 && grid > k.resident) grid = k.resident;
   void const* params = a.params;
   void const* x = a.x;

@@ -20,6 +20,11 @@ struct FusedConfig {
   int waves_per_simd = 2;     // occupancy the kernel is compiled for
   bool params_in_registers = false;  // parameters loaded once per wave, kept in VGPRs
   bool saved_in_lds = false;         // Save_State slots kept in LDS, not registers
+  // 16-bit plans: every A fragment stays in LDS.  In: where that is possible
+  // (the kernels that forward passes run; kernel sources handed out keep the
+  // staged form); out: that it is.
+  bool resident = false;
+  bool by_wave = false;  // persistent kernels: tiles go to waves, not to workgroups
   bool persistent_loop = false;      // staged 16-bit plans: one workgroup per CU loops over tiles
   int columns_per_block = 128;
   int lds_total = 0;                 // bytes of LDS the kernel declares
@@ -38,9 +43,10 @@ bool fused_supports(ponni_plan_s const& p);
 bool narrow_jit_supports(ponni_plan_s const& p);
 std::string fused_kernel_name(ponni_plan_s const& p);
 std::string fused_source(ponni_plan_s const& p, FusedConfig& cfg);
-// Compile (or fetch from cache) the plan's kernel; needs no device.  The
-// first call settles the plan's occupancy (ponni_plan_s::fused_wps).
-int fused_compile(ponni_plan_s& p, std::string& key, std::vector<char>& code, std::string& error);
+// Compile (or fetch from cache) the plan's main kernel, a 16-bit plan's with
+// resident fragments if asked and possible; needs no device.  The first call
+// settles the kernel's occupancy (ponni_plan_s::fused_wps, resident_wps).
+int fused_compile(ponni_plan_s& p, bool resident, std::string& key, std::vector<char>& code, std::string& error);
 // Compile if needed one of the plan's kernels (ponni_plan_s::kernels) and load
 // it on the current device; the main one first.
 int fused_prepare(ponni_plan_s& p, bool io32, bool split, std::string& error);

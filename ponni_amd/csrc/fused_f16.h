@@ -432,6 +432,65 @@ __device__ inline H<TO, NT, E> dense_hs(H<TI, NT, E> const& in, Stage<E>& st, La
   return out;
 }
 
+// n fragments into LDS once per workgroup; the caller waits (wait_vmem) and
+// synchronizes before the first read.
+template <class E>
+__device__ inline void stage_frags(typename Vec<E>::x8* __restrict__ lds, float const* __restrict__ src, int n) {
+  for (int f = wave_id(); f < n; f += blockDim.x >> 6) dma16(src + f * 256 + (threadIdx.x & 63) * 4, lds + f * 64);
+}
+
+// The same for plans whose A fragments all stay in LDS (frags: the layer's,
+// 64 lanes each): no chunks, so no waits and no barriers, and the waves of a
+// workgroup run apart.
+template <int TI, int TO, int NT, bool TR = false, class E, class Init, class Epi>
+__device__ inline H<TO, NT, E> dense_hr(H<TI, NT, E> const& in, typename Vec<E>::x8 const* __restrict__ frags,
+                                        Lane const& L, Init init, Epi epi) {
+  using V8 = typename Vec<E>::x8;
+  using V4 = typename Vec<E>::x4;
+  constexpr int TS = (TI + 1) / 2;
+  constexpr int GT = TO % kTileGroup == 0 ? kTileGroup : 1;
+  V8 const* __restrict__ fl = frags + L.lane;
+  H<TO, NT, E> out;
+  floatx4 prev[GT][NT];
+#pragma unroll
+  for (int mo = 0; mo < TO; mo += GT) {
+    floatx4 acc[GT][NT];
+#pragma unroll
+    for (int q = 0; q < GT; q++) {
+      floatx4 const seed = init(mo + q);
+#pragma unroll
+      for (int n = 0; n < NT; n++) acc[q][n] = seed;
+    }
+    if (kSetPrio) __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int t = 0; t < TS; t++) {
+      V8 a[GT];
+#pragma unroll
+      for (int q = 0; q < GT; q++) a[q] = fl[((mo + q) * TS + t) * 64];
+#pragma unroll
+      for (int n = 0; n < NT; n++) {
+        V4 const lo = in.v[2 * t][n];
+        V4 const hi = (2 * t + 1 < TI) ? in.v[(2 * t + 1 < TI) ? 2 * t + 1 : 2 * t][n]
+                                       : V4{E(0.0f), E(0.0f), E(0.0f), E(0.0f)};
+        V8 const b = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+#pragma unroll
+        for (int q = 0; q < GT; q++) acc[q][n] = TR ? Vec<E>::mfma(b, a[q], acc[q][n]) : Vec<E>::mfma(a[q], b, acc[q][n]);
+      }
+    }
+    if (kSetPrio) __builtin_amdgcn_s_setprio(0);
+    if (mo > 0)
+#pragma unroll
+      for (int q = 0; q < GT; q++) epi(mo - GT + q, prev[q], out.v[mo - GT + q]);
+#pragma unroll
+    for (int q = 0; q < GT; q++)
+#pragma unroll
+      for (int n = 0; n < NT; n++) prev[q][n] = acc[q][n];
+  }
+#pragma unroll
+  for (int q = 0; q < GT; q++) epi(TO - GT + q, prev[q], out.v[TO - GT + q]);
+  return out;
+}
+
 // Accumulator seeds for dense_hs: zero, or the per-feature vector b.
 struct SeedZero {
   __device__ floatx4 operator()(int) const { return floatx4{0.0f, 0.0f, 0.0f, 0.0f}; }

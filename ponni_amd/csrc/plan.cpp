@@ -1681,7 +1681,7 @@ int ponni_plan_compile(ponni_plan plan) {
   if (plan->path != PONNI_PATH_FUSED && !plan->narrow_jit) return PONNI_OK;
   std::string key, error;
   std::vector<char> code;
-  int const st = fused_compile(*plan, key, code, error);
+  int const st = fused_compile(*plan, true, key, code, error);
   return st == PONNI_OK ? PONNI_OK : fail(st, error);
 }
 
@@ -1692,7 +1692,7 @@ int ponni_plan_kernel_config(ponni_plan plan, int32_t* threads, int32_t* columns
     return fail(PONNI_ERR_UNSUPPORTED, "only FUSED and generated NARROW plans have a generated kernel");
   std::string key, error;
   std::vector<char> code;
-  int const st = fused_compile(*plan, key, code, error);
+  int const st = fused_compile(*plan, false, key, code, error);
   if (st != PONNI_OK) return fail(st, error);
   FusedConfig cfg;
   (void)fused_source(*plan, cfg);

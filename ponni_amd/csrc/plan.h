@@ -60,6 +60,7 @@ struct FusedKernel {
   int columns_per_block = 128;
   int waves = 4;         // per workgroup
   int64_t resident = 0;  // a persistent grid's workgroups (0: one per column block)
+  int wave_columns = 0;  // columns of a tile where tiles go to waves (0: to workgroups)
 };
 
 // Kinds of packed parameter slots (plan.cpp visit_param_slots).
@@ -205,7 +206,10 @@ struct ponni_plan_s {
   // them.
   ponni_hip::FusedKernel kernels[2][2];
   int fused_cus = 0;  // compute units of the plan's device
-  int fused_wps = 0;  // waves per SIMD the main kernel is compiled for (0: not settled yet)
+  // Waves per SIMD the main kernel is compiled for, and its form with resident
+  // fragments (0: not settled yet).
+  int fused_wps = 0;
+  int resident_wps = 0;
   // The small-batch kernel's time per column over the main one's (0: the plan
   // has none), and whether it is the faster one at every batch.
   double split_ratio = 0;

@@ -97,3 +97,32 @@ def test_small_batch_and_main_kernels(cuda, chain, dtype):
                 assert np.abs(got - want).max() <= 1e-12 * max(1.0, np.abs(want).max())
             else:
                 check_half(got, want)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("chain", ["few_tiles", "projection"])
+def test_tiles_dealt_to_waves(cuda, chain, dtype):
+    """Persistent kernels whose tiles go to waves (fp32 parameters in LDS,
+    16-bit fragments in LDS): batches around one tile on every CU, around a
+    wave on every SIMD, and of several passes with a ragged end, aligned and
+    misaligned rows, on the main kernel."""
+    import torch
+
+    layers = CHAINS[chain](np.random.default_rng(78))
+    tdt = getattr(torch, TORCH_DT[dtype])
+    main = P.create_inference_model(*layers, dtype=dtype, path="fused")
+    A = P._abi
+    A.check(A.lib().ponni_plan_device_params(main._plan, ctypes.byref(ctypes.c_void_p())))
+    n_in, n_out = main.get_num_inputs(), main.get_num_outputs()
+    for B, pad in [(31, 1), (8_192, 0), (8_225, 7), (32_769, 7), (300_007, 1)]:
+        print(f"tiles dealt to waves: chain={chain} dtype={dtype} B={B}", flush=True)
+        x = np.random.default_rng(B).standard_normal((n_in, B))
+        xs = torch.zeros((n_in, B + pad), dtype=tdt, device="cuda:0")
+        xs[:, :B] = torch.from_numpy(x).to(tdt)
+        ys = torch.full((n_out, B + pad), float("nan"), dtype=tdt, device="cuda:0")
+        main.forward_raw_no_alloc(xs.data_ptr(), xs.stride(0), ys.data_ptr(), ys.stride(0), B,
+                                  torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        assert torch.isnan(ys[:, B:].float()).all(), "kernel wrote past the batch"
+        want = oracle.forward(layers, xs[:, :B].double().cpu().numpy(), ORACLE_MODE[dtype])
+        (check_f32 if dtype == "f32" else check_half)(ys[:, :B].double().cpu().numpy(), want)
