@@ -1244,11 +1244,9 @@ std::string narrow_source(ponni_plan_s const& p, FusedConfig& cfg) {
     << "(real const* __restrict__ P, IO const* __restrict__ x, int64_t ldx, IO* __restrict__ y, int64_t ldy, "
        "int64_t batch) {\n";
   o << "  constexpr int U = " << U << ", V = " << V << ";\n";
-  o << "  bool const aligned = vec_ok<IO, V>(x, ldx) && vec_ok<IO, V>(y, ldy);\n";
-  // Workgroups wholly inside the batch (all but the last) with vector-aligned
-  // views take a path with no per-lane predicate, so every load is issued
-  // before the first wait.
-  o << "  if (aligned && (int64_t(blockIdx.x) + 1) * (U * 256 * V) <= batch) {\n";
+  // Workgroups wholly inside the batch (all but the last) take a path with no
+  // per-lane predicate, so every load is issued before the first wait.
+  o << "  if ((int64_t(blockIdx.x) + 1) * (U * 256 * V) <= batch) {\n";
   o << "    real s[U][" << W << "][V];\n";
   o << "#pragma unroll\n    for (int u = 0; u < U; u++)\n      load<S, V, " << p.layers.front().n_in << WV
     << "(s[u], x, ldx, ((int64_t(blockIdx.x) * U + u) * 256 + threadIdx.x) * V, batch, true);\n";
@@ -1261,10 +1259,10 @@ std::string narrow_source(ponni_plan_s const& p, FusedConfig& cfg) {
   o << "#pragma unroll\n  for (int u = 0; u < U; u++) {\n";
   o << "    b0[u] = ((int64_t(blockIdx.x) * U + u) * 256 + threadIdx.x) * V;\n";
   o << "    if (b0[u] < batch) load<S, V, " << p.layers.front().n_in << WV
-    << "(s[u], x, ldx, b0[u], batch, aligned && b0[u] + V <= batch);\n  }\n";
+    << "(s[u], x, ldx, b0[u], batch, b0[u] + V <= batch);\n  }\n";
   o << "#pragma unroll\n  for (int u = 0; u < U; u++)\n    if (b0[u] < batch) chain(s[u], P);\n";
   o << "#pragma unroll\n  for (int u = 0; u < U; u++)\n    if (b0[u] < batch) store<S, V, " << p.layers.back().n_out
-    << WV << "(s[u], y, ldy, b0[u], batch, aligned && b0[u] + V <= batch);\n}\n";
+    << WV << "(s[u], y, ldy, b0[u], batch, b0[u] + V <= batch);\n}\n";
   return o.str();
 }
 

@@ -21,9 +21,12 @@
 namespace ponni_hip {
 namespace narrowj {
 
+// V elements at any element alignment: rows of an odd batch, or a column
+// subview, start anywhere, and gfx950 loads and stores 16 bytes at any
+// address.
 template <class S, int V>
 struct VecOf {
-  typedef S type __attribute__((ext_vector_type(V)));
+  typedef S type __attribute__((ext_vector_type(V), aligned(alignof(S))));
 };
 
 template <class A, class B>
@@ -40,12 +43,6 @@ template <class S, class C>
 __device__ inline C round_state(C v) {
   if constexpr (same_type<S, C>::value) return v;
   else return static_cast<C>(static_cast<S>(v));
-}
-
-// Can rows of this view be moved as aligned V-element vectors?
-template <class S, int V>
-__device__ inline bool vec_ok(void const* p, int64_t ld) {
-  return (reinterpret_cast<unsigned long long>(p) % (sizeof(S) * V)) == 0 && ld % V == 0;
 }
 
 // s[f][v] = x(f, b0 + v) rounded to S for f < N; rows >= N and samples >=
