@@ -468,7 +468,7 @@ std::string fused_source_once(ponni_plan_s const& p, FusedConfig& cfg, bool allo
     vec_bytes += int64_t(4 + op.epi_count) * 64 * std::max(tiles(op.n_in), tiles(op.n_out));
   }
   if (want_resident && frag_bytes > 0) {
-    int64_t const rows_per_wave = int64_t(tiles(p.layers.front().n_in)) * 16 * 16 * NT * (cfg.io32 ? 4 : 2);
+    int64_t const rows_per_wave = int64_t(tiles(p.layers.front().n_in)) * 16 * (16 * NT * (cfg.io32 ? 4 : 2) + (cfg.any_rows ? 16 : 0));
     int best = 0;
     for (int w = 4; w <= 4 * cfg.waves_per_simd; w += 4) {
       int64_t const lds = frag_bytes + vec_bytes + w * rows_per_wave;
@@ -632,8 +632,9 @@ std::string fused_source_once(ponni_plan_s const& p, FusedConfig& cfg, bool allo
   // (fused_f16.h prefetch_rows_lds16) when the buffer fits next to the staged
   // A fragments (3 slots of 32 KB) and vectors.
   int const n_in0 = p.layers.front().n_in;
-  int const in_rows_elems = tiles(n_in0) * 16 * 16 * NT;  // per wave, row-major 16-bit
-  int const in_dma_bytes = cfg.waves * in_rows_elems * io_bytes;
+  // (per wave; of misaligned rows the 16-byte blocks that hold them, one more a row)
+  int const in_rows_bytes = tiles(n_in0) * 16 * (16 * NT * io_bytes + (cfg.any_rows ? 16 : 0));
+  int const in_dma_bytes = cfg.waves * in_rows_bytes;
   int const stage_bytes = cfg.resident ? static_cast<int>(frag_bytes)
                           : half && !cfg.split && !dense_seq.empty() ? slots * slot_frags * 1024 : 0;
   bool const in_dma = half && !cfg.split && NT % 2 == 0 &&
@@ -646,8 +647,11 @@ std::string fused_source_once(ponni_plan_s const& p, FusedConfig& cfg, bool allo
   // them, the next one a chunk later.  With one dense layer: after this
   // tile's rows are read.
   int const hook_dense = half && in_dma && dense_seq.size() >= 2 ? 1 : -1;
-  std::string const prefetch_next = "if (pre_next) prefetch_rows_lds16<" + std::to_string(n_in0) + ", " +
-                                    std::to_string(NT) + ">(x, ldx, Ln, in_buf[wave_id()]);";
+  auto prefetch = [&](std::string const& lane) {
+    return std::string(cfg.any_rows ? "prefetch_rows_any<" : "prefetch_rows_lds16<") + std::to_string(n_in0) + ", " +
+           std::to_string(NT) + ">(x, ldx, " + lane + ", in_buf[wave_id()]);";
+  };
+  std::string const prefetch_next = "if (pre_next) " + prefetch("Ln");
   // The last op, a dense layer whose epilogue is its bias (the seed) and
   // activations without parameters, runs transposed and writes 8-byte runs
   // of output rows (fused_f16.h store_rows_ht).
@@ -661,17 +665,19 @@ std::string fused_source_once(ponni_plan_s const& p, FusedConfig& cfg, bool allo
       if (a == ACT_BIAS || act_has_param(a)) out_transposed = false;
     }
   }
-  if (out_transposed)
-    o << "  bool const yvec = ((reinterpret_cast<uint64_t>(y) | uint64_t(ldy) * " << io_bytes << ") & " << 4 * io_bytes - 1
-      << ") == 0;\n";
   if (in_dma) {
-    o << "  __shared__ __attribute__((aligned(16))) " << IO << " in_buf[" << cfg.waves << "][" << in_rows_elems << "];\n";
+    if (cfg.any_rows)
+      o << "  __shared__ __attribute__((aligned(16))) char in_buf[" << cfg.waves << "][" << in_rows_bytes << "];\n";
+    else
+      o << "  __shared__ __attribute__((aligned(16))) " << IO << " in_buf[" << cfg.waves << "][" << in_rows_bytes / io_bytes
+        << "];\n";
     // Whole tiles of a 16-byte aligned x with a row stride of a multiple of
-    // 16 bytes go through LDS; others (the batch's last tile) load directly.
-    o << "  bool const xvec = ((reinterpret_cast<uint64_t>(x) | uint64_t(ldx) * " << io_bytes << ") & 15) == 0;\n";
+    // 16 bytes go through LDS (or of any x, in the kernel for such rows);
+    // others (the batch's last tile) load directly.
+    if (cfg.any_rows) o << "  constexpr bool xvec = true;\n";
+    else o << "  bool const xvec = ((reinterpret_cast<uint64_t>(x) | uint64_t(ldx) * " << io_bytes << ") & 15) == 0;\n";
     o << "  int64_t const tile0 = " << first_tile << ";\n  L.col0 = " << column_of("tile0") << ";\n";
-    o << "  if (tile0 < tiles && xvec && L.col0 + " << WCOLS << " <= batch) prefetch_rows_lds16<" << n_in0 << ", "
-      << NT << ">(x, ldx, L, in_buf[wave_id()]);\n";
+    o << "  if (tile0 < tiles && xvec && L.col0 + " << WCOLS << " <= batch) " << prefetch("L") << "\n";
     // The LDS writes of these loads complete with vmcnt, which the compiler
     // does not track (fused_f16.h dma16): each tile's rows are waited for
     // explicitly, here for the first tile and before the output stores for
@@ -692,8 +698,10 @@ std::string fused_source_once(ponni_plan_s const& p, FusedConfig& cfg, bool allo
   std::string cur = fresh();
   int cur_n = p.layers.front().n_in;
   if (in_dma) {
-    o << "    auto " << cur << " = xvec && L.col0 + " << WCOLS << " <= batch ? load_rows_lds16<" << cur_n << ", " << NT
-      << ", E>(in_buf[wave_id()], L) : load_rows_h<" << cur_n << ", " << NT << ", E>(x, ldx, L);\n";
+    o << "    auto " << cur << " = xvec && L.col0 + " << WCOLS << " <= batch ? "
+      << (cfg.any_rows ? "load_rows_any<" : "load_rows_lds16<") << cur_n << ", " << NT << ", E>("
+      << (cfg.any_rows ? "x, ldx, " : "") << "in_buf[wave_id()], L) : load_rows_h<" << cur_n << ", " << NT
+      << ", E>(x, ldx, L);\n";
     o << "    wait_lds();\n";
     o << "    Lane Ln = L;\n    Ln.col0 = " << column_of("tile + " + tile_step) << ";\n";
     o << "    bool const pre_next = tile + " << tile_step << " < tiles && xvec && Ln.col0 + " << WCOLS << " <= batch;\n";
@@ -857,7 +865,7 @@ std::string fused_source_once(ponni_plan_s const& p, FusedConfig& cfg, bool allo
         if (cfg.split && &op == &p.ops.back()) {
           if (half)
             o << "    split_store_h<" << n << ", " << tiles(n) << ", " << SW << ", " << (pad_ok ? "false" : "true") << ">("
-              << own << ", y, ldy, wv, L, " << (out_transposed ? "yvec" : "false") << ");\n";
+              << own << ", y, ldy, wv, L);\n";
           else
             o << "    split_store<" << n << ", " << tiles(n) << ", " << SW << ">(" << own << ", y, ldy, wv, L);\n";
           stored = true;
@@ -1068,7 +1076,7 @@ std::string fused_source_once(ponni_plan_s const& p, FusedConfig& cfg, bool allo
   if (stored) {
   } else if (cfg.split) {
     o << "    if (wv == 0) " << (half ? "store_rows_h<" : "store_rows<") << cur_n << ">(" << cur << ", y, ldy, L);\n";
-  } else if (out_transposed) o << "    store_rows_ht<" << cur_n << ">(" << cur << ", y, ldy, L, yvec);\n";
+  } else if (out_transposed) o << "    store_rows_ht<" << cur_n << ">(" << cur << ", y, ldy, L);\n";
   else if (half) o << "    store_rows_h<" << cur_n << ">(" << cur << ", y, ldy, L);\n";
   else o << "    store_rows<" << cur_n << ">(" << cur << ", y, ldy, L);\n";
   o << "  }\n}\n";
@@ -1091,6 +1099,7 @@ std::string fused_source_once(ponni_plan_s const& p, FusedConfig& cfg, bool allo
     head << "  int const wv = wave_id();\n";
   }
   cfg.vec_bytes = vec_total * es;
+  cfg.rows_in_lds = in_dma;
   cfg.lds_total = exchange_bytes + stage_bytes + (in_dma ? in_dma_bytes : 0) + cfg.vec_bytes + static_cast<int>(cfg.lds_bytes);
   return head.str() + o.str();
 }
@@ -1500,14 +1509,16 @@ int load_module(std::string const& key, std::vector<char> const& code, std::stri
 
 }  // namespace
 
-int fused_prepare(ponni_plan_s& p, bool io32, bool split, std::string& error) {
+int fused_prepare(ponni_plan_s& p, bool io32, FusedForm form, std::string& error) {
+  bool const split = form == FUSED_SMALL;
   std::string key;
   std::vector<char> code;
   FusedConfig cfg;
   cfg.io32 = io32;
   cfg.split = split;
+  cfg.any_rows = form == FUSED_ANY_ROWS;
   cfg.resident = !split;
-  bool const main = !io32 && !split;  // (settles the plan's occupancy)
+  bool const main = !io32 && form == FUSED_MAIN;  // (settles the plan's occupancy)
   int st = main ? fused_compile(p, true, key, code, error) : compile_cached(p, cfg, key, code, error);
   if (st != PONNI_OK) return st;
   (void)fused_source(p, cfg);
@@ -1521,7 +1532,11 @@ int fused_prepare(ponni_plan_s& p, bool io32, bool split, std::string& error) {
     error = "no compute units";
     return PONNI_ERR_DEVICE;
   }
-  FusedKernel& k = p.kernels[io32][split];
+  FusedKernel& k = p.kernels[io32][form];
+  // (a kernel that spills registers already gains nothing from the form for
+  // misaligned rows, which needs a few more: fp16 32-128-16 residual, 15
+  // spilled, 1,000,003 columns 484 against 490 us)
+  k.rows_in_lds = cfg.rows_in_lds && metadata_int(code, ".vgpr_spill_count") <= 0;
   k.columns_per_block = cfg.columns_per_block;
   k.waves = cfg.waves;
   k.wave_columns = cfg.by_wave ? cfg.columns_per_block / cfg.waves : 0;
@@ -1556,8 +1571,8 @@ int fused_prepare(ponni_plan_s& p, bool io32, bool split, std::string& error) {
 // 82 / 85 / 165 against 43 / 82 / 116 us; fp16 64-256-256-256-64 24 / 25 / 30
 // against 11 / 16 / 25; fp64 16-64-64-64-8 12.6 / 13.2 / 22.4 against 8.4 /
 // 13.2 / 17.4.  Beyond two rounds the main kernel's workgroups balance.
-bool fused_wants_split(ponni_plan_s const& p, int64_t batch) {
-  if (p.path != PONNI_PATH_FUSED || p.split_ratio <= 0) return false;
+static bool fused_wants_split(ponni_plan_s const& p, int64_t batch) {
+  if (p.split_ratio <= 0) return false;
   if (p.split_always) return true;
   FusedKernel const& main = p.kernels[0][0];
   // (tiles dealt to waves: one wave per SIMD everywhere is the flat part; more
@@ -1567,9 +1582,21 @@ bool fused_wants_split(ponni_plan_s const& p, int64_t batch) {
   return rounds <= (main.wave_columns > 0 ? 1 : 2) && 0.25 + p.split_ratio * rounds < (rounds <= 1 ? 1 : 2);
 }
 
+FusedForm fused_wanted_form(ponni_plan_s const& p, void const* x, int64_t ld_in, int64_t batch, bool io32) {
+  if (p.path != PONNI_PATH_FUSED) return FUSED_MAIN;
+  if (fused_wants_split(p, batch)) return FUSED_SMALL;
+  // Rows that do not start on 16 bytes, where aligned ones go through LDS a
+  // tile ahead: element loads instead took half again the time (fp16
+  // 64-256-256-256-64, 262,145 columns: 166 us, aligned 110).
+  int const es = io32 ? 4 : 2;
+  bool const aligned = ((reinterpret_cast<uint64_t>(x) | uint64_t(ld_in) * es) & 15) == 0;
+  return p.kernels[io32][FUSED_MAIN].rows_in_lds && !aligned ? FUSED_ANY_ROWS : FUSED_MAIN;
+}
+
 hipError_t fused_launch(ponni_plan_s const& p, LaunchArgs const& a, bool io32, hipStream_t stream) {
-  bool const split = p.kernels[io32][1].fn != nullptr && fused_wants_split(p, a.batch);
-  FusedKernel const& k = p.kernels[io32][split];
+  FusedForm form = fused_wanted_form(p, a.x, a.ld_x, a.batch, io32);
+  if (p.kernels[io32][form].fn == nullptr) form = FUSED_MAIN;
+  FusedKernel const& k = p.kernels[io32][form];
   // (a persistent grid whose tiles go to waves takes every CU it has tiles for)
   int64_t const columns = k.wave_columns > 0 ? k.wave_columns : k.columns_per_block;
   int64_t grid = (a.batch + columns - 1) / columns;

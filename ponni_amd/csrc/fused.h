@@ -31,9 +31,11 @@ struct FusedConfig {
   // The small-batch kernel (fused_split.h): a workgroup's waves share one
   // tile of columns and split each contraction's output tiles.
   bool split = false;
+  bool any_rows = false;     // 16-bit: input rows at any alignment through LDS
+  bool rows_in_lds = false;  // input rows go through LDS a tile ahead
   bool io32 = false;  // a 16-bit plan's kernel on fp32 input and output rows
   int split_waves = 8, split_nt = 1, split_wps = 2;
-  std::string suffix() const { return std::string(io32 ? "_io32" : "") + (split ? "_split" : ""); }
+  std::string suffix() const { return std::string(io32 ? "_io32" : "") + (split ? "_split" : any_rows ? "_any" : ""); }
 };
 
 // Widest state a FUSED kernel of this dtype keeps on chip.
@@ -49,9 +51,10 @@ std::string fused_source(ponni_plan_s const& p, FusedConfig& cfg);
 int fused_compile(ponni_plan_s& p, bool resident, std::string& key, std::vector<char>& code, std::string& error);
 // Compile if needed one of the plan's kernels (ponni_plan_s::kernels) and load
 // it on the current device; the main one first.
-int fused_prepare(ponni_plan_s& p, bool io32, bool split, std::string& error);
-// Does a batch run on the small-batch kernel (once the main one is loaded)?
-bool fused_wants_split(ponni_plan_s const& p, int64_t batch);
+int fused_prepare(ponni_plan_s& p, bool io32, FusedForm form, std::string& error);
+// The form of the plan's kernel that a call runs on once it is loaded (the
+// main one takes any call).
+FusedForm fused_wanted_form(ponni_plan_s const& p, void const* x, int64_t ld_in, int64_t batch, bool io32);
 hipError_t fused_launch(ponni_plan_s const& p, LaunchArgs const& a, bool io32, hipStream_t stream);
 
 }  // namespace ponni_hip

@@ -104,7 +104,8 @@ __device__ inline H<(N + 15) / 16, NT, E> load_rows_h(X const* __restrict__ x, i
 // 16 NT elements apart instead of 4 x that, in four different LDS banks
 // (row-major, all four groups read one bank).  Only whole tiles
 // of a 16-byte aligned x with a row stride of whole 16-byte pieces are
-// requested this way (the caller checks); rows >= N issue nothing.  The
+// requested this way (the caller checks; others by prefetch_rows_any below);
+// rows >= N issue nothing.  The
 // loads are asynchronous: the caller waits (vmcnt) before reading buf.
 typedef __attribute__((address_space(3))) void* lds_ptr;
 
@@ -164,6 +165,57 @@ __device__ inline H<(N + 15) / 16, NT, E> load_rows_lds16(X const* __restrict__ 
   return s;
 }
 
+// Rows at any alignment (an odd batch, a column subview): the 16-byte blocks
+// that hold the row's columns, one more per row than above, requested from
+// the aligned address below the row's first column, and read at the row's
+// own byte offset in them.  (Every block requested holds a column of the
+// row, so it lies in the memory page of that column.)
+template <int NT, class X>
+constexpr int any_pieces() {
+  return 16 * NT * int(sizeof(X)) / 16 + 1;
+}
+template <int N, int NT, class X>
+__device__ inline void prefetch_rows_any(X const* __restrict__ x, int64_t ld, Lane const& L, char* __restrict__ buf) {
+  constexpr int T = (N + 15) / 16;
+  constexpr int PR = any_pieces<NT, X>();
+#pragma unroll
+  for (int i = 0; i < (T * 16 * PR + 63) / 64; i++) {
+    int const piece = 64 * i + L.lane;
+    int const slot = piece / PR, k = piece % PR;
+    int const r = (slot & ~15) | ((slot & 3) << 2) | ((slot >> 2) & 3);
+    uint64_t const row = reinterpret_cast<uint64_t>(x + int64_t(r) * ld + L.col0);
+    if (r < N && (k < PR - 1 || (row & 15) != 0))
+      dma16(reinterpret_cast<void const*>((row & ~uint64_t(15)) + 16 * k), buf + 64 * 16 * i);
+  }
+}
+template <int N, int NT, class E, class X>
+__device__ inline H<(N + 15) / 16, NT, E> load_rows_any(X const* __restrict__ x, int64_t ld,
+                                                        char const* __restrict__ buf, Lane const& L) {
+  constexpr int T = (N + 15) / 16;
+  constexpr int PR = any_pieces<NT, X>(), XS = int(sizeof(X));
+  // A row's offset in its first block repeats every 8 rows (or 4, or 2), and
+  // a tile's columns start at a multiple of 16 bytes.
+  char const* at[4];
+#pragma unroll
+  for (int e = 0; e < 4; e++) {
+    unsigned const row = static_cast<unsigned>(reinterpret_cast<uint64_t>(x)) +
+                         static_cast<unsigned>(fresh(4 * L.g + e)) * static_cast<unsigned>(ld) * XS;
+    at[e] = buf + (4 * e + L.g) * (16 * PR) + (row & 15) + XS * L.c;
+  }
+  H<T, NT, E> s;
+#pragma unroll
+  for (int m = 0; m < T; m++)
+#pragma unroll
+    for (int n = 0; n < NT; n++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        int const f = 16 * m + 4 * L.g + e;
+        E const v = static_cast<E>(*reinterpret_cast<X const*>(at[e] + m * 256 * PR + 16 * XS * n));
+        s.v[m][n][e] = (N % 16 == 0 || f < N) ? v : E(0.0f);
+      }
+  return s;
+}
+
 // Waits: every outstanding vector-memory operation of this wave (vmcnt(0)),
 // or every outstanding LDS operation (lgkmcnt(0)).
 __device__ inline void wait_vmem() { __builtin_amdgcn_s_waitcnt(0x0F70); }
@@ -189,15 +241,14 @@ __device__ inline void store_rows_h(H<T, NT, E> const& s, Y* __restrict__ y, int
 // Transposed tile (a dense layer run with its MFMA operands swapped, fused
 // dense_hs<..., TR = true>): lane l, element e <-> feature 16m + c, column
 // col0 + 16n + 4g + e, so each lane's 4 elements are consecutive columns of
-// one output row.  Whole tiles of a y aligned to 4 elements with a row stride
-// of a multiple of 4 elements (vec_ok) store them as one write; otherwise
-// element by element inside the batch.  Rows >= N are not written.
-template <class Y> struct Vec4Of { typedef Y type __attribute__((ext_vector_type(4))); };
+// one output row.  Whole tiles store them as one write (at any alignment,
+// which gfx950 stores as well); the batch's last tile element by element.
+// Rows >= N are not written.
+template <class Y> struct Vec4Of { typedef Y type __attribute__((ext_vector_type(4), aligned(alignof(Y)))); };
 template <int N, int T, int NT, class E, class Y>
-__device__ inline void store_rows_ht(H<T, NT, E> const& s, Y* __restrict__ y, int64_t ld, Lane const& L,
-                                     bool vec_ok) {
+__device__ inline void store_rows_ht(H<T, NT, E> const& s, Y* __restrict__ y, int64_t ld, Lane const& L) {
   using Y4 = typename Vec4Of<Y>::type;
-  bool const full = vec_ok && L.col0 + 16 * NT <= L.batch;
+  bool const full = L.col0 + 16 * NT <= L.batch;
 #pragma unroll
   for (int m = 0; m < T; m++) {
     int const f = 16 * m + L.c;

@@ -232,8 +232,8 @@ __device__ inline H<TO, NT, E> split_get_h(typename Vec<E>::x4 const* __restrict
 
 // Own tiles of the output: row-major tiles, or transposed ones (TR).
 template <int N, int TO, int W, bool TR, int OWN, int NT, class E, class Y>
-__device__ inline void split_store_h(H<OWN, NT, E> const& own, Y* __restrict__ y, int64_t ld, int wave, Lane const& L,
-                                     bool vec_ok) {
+__device__ inline void split_store_h(H<OWN, NT, E> const& own, Y* __restrict__ y, int64_t ld, int wave,
+                                     Lane const& L) {
   using Y4 = typename Vec4Of<Y>::type;
 #pragma unroll
   for (int o = 0; o < OWN; o++) {
@@ -243,7 +243,7 @@ __device__ inline void split_store_h(H<OWN, NT, E> const& own, Y* __restrict__ y
       int const f = 16 * mo + L.c;
       if (N % 16 != 0 && f >= N) continue;
       Y* __restrict__ yr = y + int64_t(f) * ld + L.col0 + 4 * L.g;
-      bool const full = vec_ok && L.col0 + 16 * NT <= L.batch;
+      bool const full = L.col0 + 16 * NT <= L.batch;
 #pragma unroll
       for (int n = 0; n < NT; n++) {
         Y4 const v = __builtin_convertvector(own.v[o][n], Y4);

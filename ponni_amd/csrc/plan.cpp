@@ -1021,7 +1021,7 @@ int upload(ponni_plan_s& p) {
   if (count > 0) HIP_TRY(hipMemcpy(p.d_params, packed, count * param_element_size(p), hipMemcpyHostToDevice));
   if ((p.path == PONNI_PATH_FUSED || p.narrow_jit) && p.kernels[0][0].fn == nullptr) {
     std::string error;
-    int const st = fused_prepare(p, false, false, error);
+    int const st = fused_prepare(p, false, FUSED_MAIN, error);
     if (st != PONNI_OK) return fail(st, error);
   }
   int const st = build_gather(p);
@@ -1463,11 +1463,12 @@ int forward_impl(ponni_plan plan, const void* x, int64_t ld_in, void* y, int64_t
     if (dev != plan->device) return fail(PONNI_ERR_DEVICE, "plan was first used on another device");
   }
   // The kernels of this call that are not loaded yet.  (A captured stream
-  // cannot load a module: a plan whose small-batch kernel is not there yet
-  // then runs its other kernel, which takes any batch.)
-  bool const need_rows = io32 && plan->kernels[1][0].fn == nullptr;
-  bool const need_split = !no_alloc && plan->kernels[io32][1].fn == nullptr && fused_wants_split(*plan, batch);
-  if (need_rows || need_split) {
+  // cannot load a module: a plan whose form for this call is not there yet
+  // then runs its main kernel, which takes any call.)
+  bool const need_rows = io32 && plan->kernels[1][FUSED_MAIN].fn == nullptr;
+  FusedForm const form = no_alloc ? FUSED_MAIN : fused_wanted_form(*plan, x, ld_in, batch, io32);
+  bool const generated = plan->path == PONNI_PATH_FUSED || plan->narrow_jit;
+  if (generated && (need_rows || plan->kernels[io32][form].fn == nullptr)) {
     hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
     bool const can_load =
         hipStreamIsCapturing(stream, &capturing) == hipSuccess && capturing == hipStreamCaptureStatusNone;
@@ -1475,11 +1476,12 @@ int forward_impl(ponni_plan plan, const void* x, int64_t ld_in, void* y, int64_t
       return fail(PONNI_ERR_UNSUPPORTED, "fp32 rows: the kernel is not loaded yet, and the stream is being captured");
     std::string error;
     if (need_rows) {
-      int const st = fused_prepare(*plan, true, false, error);
+      int const st = fused_prepare(*plan, true, FUSED_MAIN, error);
       if (st != PONNI_OK) return fail(st, error);
     }
-    if (need_split && can_load) {
-      int const st = fused_prepare(*plan, io32, true, error);
+    FusedForm const wanted = fused_wanted_form(*plan, x, ld_in, batch, io32);
+    if (plan->kernels[io32][wanted].fn == nullptr && can_load) {
+      int const st = fused_prepare(*plan, io32, wanted, error);
       if (st != PONNI_OK) return fail(st, error);
     }
   }

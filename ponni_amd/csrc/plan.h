@@ -54,12 +54,17 @@ inline void launch_kernel(F kernel, dim3 grid, dim3 block, uint32_t shmem, hipSt
     (void)hipLaunchKernel(fn, grid, block, argv, shmem, stream);
 }
 
+// Forms of a plan's generated kernel: for any call; for small batches
+// (fused_split.h); 16-bit, for input rows that do not start on 16 bytes.
+enum FusedForm { FUSED_MAIN = 0, FUSED_SMALL = 1, FUSED_ANY_ROWS = 2, kFusedForms = 3 };
+
 // A generated kernel on the device.
 struct FusedKernel {
   hipFunction_t fn = nullptr;
   int columns_per_block = 128;
   int waves = 4;         // per workgroup
   int64_t resident = 0;  // a persistent grid's workgroups (0: one per column block)
+  bool rows_in_lds = false;  // its input rows go through LDS a tile ahead
   int wave_columns = 0;  // columns of a tile where tiles go to waves (0: to workgroups)
 };
 
@@ -200,11 +205,10 @@ struct ponni_plan_s {
   // NARROW plans run a generated kernel (narrow_jit.h) unless JIT is off.
   bool narrow_jit = false;
   // FUSED path (and generated NARROW): the plan's generated kernels,
-  // kernels[fp32 rows][small batch].  kernels[0][0], the main one, is loaded when
-  // the plan is put on the device; the small-batch kernels (fused_split.h) and
-  // those of a 16-bit plan on fp32 rows by the first forward that runs on
-  // them.
-  ponni_hip::FusedKernel kernels[2][2];
+  // kernels[fp32 rows][form].  kernels[0][FUSED_MAIN] is loaded when the plan is
+  // put on the device; the other forms, and those of a 16-bit plan on fp32
+  // rows, by the first forward that runs on them.
+  ponni_hip::FusedKernel kernels[2][ponni_hip::kFusedForms];
   int fused_cus = 0;  // compute units of the plan's device
   // Waves per SIMD the main kernel is compiled for, and its form with resident
   // fragments (0: not settled yet).

@@ -126,3 +126,34 @@ def test_tiles_dealt_to_waves(cuda, chain, dtype):
         assert torch.isnan(ys[:, B:].float()).all(), "kernel wrote past the batch"
         want = oracle.forward(layers, xs[:, :B].double().cpu().numpy(), ORACLE_MODE[dtype])
         (check_f32 if dtype == "f32" else check_half)(ys[:, :B].double().cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("chain", ["odd_tiles", "wide", "residual", "few_tiles"])
+def test_half_rows_at_any_alignment_through_lds(cuda, chain, dtype):
+    """Large batches of 16-bit rows that start anywhere (odd strides, column
+    subviews): input through the blocks of 16 bytes around each row, outputs
+    as unaligned vectors, against the oracle on a sample of columns that
+    holds the batch's ends."""
+    import torch
+
+    layers = CHAINS[chain](np.random.default_rng(79))
+    tdt = getattr(torch, TORCH_DT[dtype])
+    m = P.create_inference_model(*layers, dtype=dtype, path="fused")
+    n_in, n_out = m.get_num_inputs(), m.get_num_outputs()
+    B = 150_001
+    pick = np.concatenate([np.arange(70), np.random.default_rng(5).integers(70, B - 70, 1500), np.arange(B - 70, B)])
+    x = np.random.default_rng(4).standard_normal((n_in, B)).astype(np.float32)
+    xq = torch.from_numpy(x).to(tdt)
+    want = oracle.forward(layers, xq[:, pick].double().numpy(), ORACLE_MODE[dtype])
+    for off, pad in [(0, 0), (1, 0), (3, 4), (7, 7), (2, 5), (0, 1)]:
+        print(f"rows at any alignment: chain={chain} dtype={dtype} off={off} pad={pad}", flush=True)
+        xs = torch.zeros((n_in, off + B + pad), dtype=tdt, device="cuda:0")
+        xs[:, off:off + B] = xq.cuda()
+        ys = torch.full((n_out, off + B + pad), float("nan"), dtype=tdt, device="cuda:0")
+        m.forward_batch_parallel(xs[:, off:off + B], ys[:, off:off + B])
+        torch.cuda.synchronize()
+        assert torch.isnan(ys[:, :off].float()).all() and torch.isnan(ys[:, off + B:].float()).all()
+        got = ys[:, off:off + B].double().cpu().numpy()
+        assert np.isfinite(got).all()
+        check_half(got[:, pick], want)
