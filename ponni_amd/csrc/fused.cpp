@@ -523,7 +523,8 @@ std::string fused_source_once(ponni_plan_s const& p, FusedConfig& cfg, bool allo
     << "* __restrict__ y, int64_t ldy, int64_t batch) {\n";
   if (cfg.lds_bytes > 0) {
     o << "  __shared__ " << F4 << " lds_p[" << cfg.lds_bytes / (4 * es) << "];\n";
-    o << "  stage(lds_p, gparams, " << cfg.lds_bytes / es << ");\n";
+    o << "  stage16<" << cfg.lds_bytes / 16 << ", " << cfg.waves << ", 0>(lds_p, gparams);\n";
+    o << "  wait_vmem();\n  __syncthreads();\n";
     o << "  " << F << " const* __restrict__ P0 = reinterpret_cast<" << F << " const*>(lds_p);\n";
   } else {
     o << "  " << F << " const* __restrict__ P0 = gparams;\n";
@@ -546,7 +547,8 @@ std::string fused_source_once(ponni_plan_s const& p, FusedConfig& cfg, bool allo
       if (op.code != OP_DENSE && op.code != OP_PROJ_ADD) continue;
       int const n = (tiles(op.code == OP_DENSE ? op.n_in : op.aux) + 1) / 2 * tiles(op.n_out);
       if (!frag_at.emplace(op.woff, frags).second) continue;
-      copies << "  stage_frags<E>(a_all + " << frags * 64 << ", gparams + " << op.woff << ", " << n << ");\n";
+      copies << "  stage16<" << n * 64 << ", " << cfg.waves << ", " << frags % cfg.waves << ">(a_all + " << frags * 64
+             << ", gparams + " << op.woff << ");\n";
       frags += n;
     }
     o << "  __shared__ Vec<E>::x8 a_all[" << frags * 64 << "];\n" << copies.str() << "  wait_vmem();\n  __syncthreads();\n";
@@ -1082,10 +1084,14 @@ std::string fused_source_once(ponni_plan_s const& p, FusedConfig& cfg, bool allo
   o << "  }\n}\n";
   if (!vec_lds.empty()) {
     head << "  __shared__ " << F4 << " lds_vec[" << vec_total / 4 << "];\n";
-    for (auto const& kv : vec_lds)
-      head << "  stage_vec(lds_vec + " << kv.second.first / 4 << ", gparams + " << kv.first << ", "
-           << kv.second.second / 4 << ");\n";
-    head << "  __syncthreads();\n";
+    int turn = 0;
+    for (auto const& kv : vec_lds) {
+      int const pieces = kv.second.second * es / 16;
+      head << "  stage16<" << pieces << ", " << cfg.waves << ", " << turn << ">(lds_vec + " << kv.second.first / 4
+           << ", gparams + " << kv.first << ");\n";
+      turn = (turn + (pieces + 63) / 64) % cfg.waves;
+    }
+    head << "  wait_vmem();\n  __syncthreads();\n";
     head << "  " << F << " const* __restrict__ VP = reinterpret_cast<" << F << " const*>(lds_vec);\n";
   }
   int exchange_bytes = 0;

@@ -107,28 +107,6 @@ __device__ inline H<(N + 15) / 16, NT, E> load_rows_h(X const* __restrict__ x, i
 // requested this way (the caller checks; others by prefetch_rows_any below);
 // rows >= N issue nothing.  The
 // loads are asynchronous: the caller waits (vmcnt) before reading buf.
-typedef __attribute__((address_space(3))) void* lds_ptr;
-
-// One 16-byte global_load_lds_dwordx4 per lane: lane l's 16 bytes at g land
-// in LDS at lds + 16 l (lds uniform across the wave, passed in M0).  Issued
-// as inline asm so that the compiler's wait insertion does not see an LDS
-// write it cannot place: it cannot tell apart regions of one LDS array
-// addressed at run time (the staging slots), so after the builtin it waits
-// for every outstanding request (vmcnt(0)) before the next read of the
-// array -- the first fragment read of every chunk waited for the requests
-// just made for two chunks ahead.  Every read of data requested here is
-// ordered by the kernel's own explicit waits (a vmcnt that leaves only
-// later requests outstanding, then a barrier where other waves' requests
-// are read); the compiler's own vmcnt values stay correct, because vector
-// memory loads complete in issue order and untracked requests only make
-// them wait longer.  The s_nop is the wait state the hardware needs
-// between the write of M0 and an LDS DMA, which the compiler inserts for
-// its own instructions but not in front of inline asm.
-__device__ inline void dma16(void const* g, void* lds) {
-  unsigned const m0 = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(reinterpret_cast<uint64_t>((lds_ptr)lds)));
-  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "{m0}"(m0) : "memory");
-}
-
 template <int N, int NT, class X>
 __device__ inline void prefetch_rows_lds16(X const* __restrict__ x, int64_t ld, Lane const& L,
                                            X* __restrict__ buf) {
@@ -216,9 +194,7 @@ __device__ inline H<(N + 15) / 16, NT, E> load_rows_any(X const* __restrict__ x,
   return s;
 }
 
-// Waits: every outstanding vector-memory operation of this wave (vmcnt(0)),
-// or every outstanding LDS operation (lgkmcnt(0)).
-__device__ inline void wait_vmem() { __builtin_amdgcn_s_waitcnt(0x0F70); }
+// Every outstanding LDS operation of this wave (lgkmcnt(0)).
 __device__ inline void wait_lds() { __builtin_amdgcn_s_waitcnt(0xC07F); }
 
 template <int N, int T, int NT, class E, class Y>
@@ -483,13 +459,6 @@ __device__ inline H<TO, NT, E> dense_hs(H<TI, NT, E> const& in, Stage<E>& st, La
   return out;
 }
 
-// n fragments into LDS once per workgroup; the caller waits (wait_vmem) and
-// synchronizes before the first read.
-template <class E>
-__device__ inline void stage_frags(typename Vec<E>::x8* __restrict__ lds, float const* __restrict__ src, int n) {
-  for (int f = wave_id(); f < n; f += blockDim.x >> 6) dma16(src + f * 256 + (threadIdx.x & 63) * 4, lds + f * 64);
-}
-
 // The same for plans whose A fragments all stay in LDS (frags: the layer's,
 // 64 lanes each): no chunks, so no waits and no barriers, and the waves of a
 // workgroup run apart.
@@ -566,14 +535,6 @@ template <class E, int NT>
 __device__ inline void tile_round(floatx4 const (&t)[NT], typename Vec<E>::x4 (&o)[NT]) {
 #pragma unroll
   for (int n = 0; n < NT; n++) o[n] = round4<E>(t[n]);
-}
-
-// Stage `bytes` (a multiple of 16) from global memory into LDS, once per
-// workgroup; the caller synchronizes before the first read.
-__device__ inline void stage_bytes(void* __restrict__ lds, void const* __restrict__ src, int bytes) {
-  floatx4* d = reinterpret_cast<floatx4*>(lds);
-  floatx4 const* s4 = reinterpret_cast<floatx4 const*>(src);
-  for (int i = threadIdx.x; i < bytes / 16; i += blockDim.x) d[i] = s4[i];
 }
 
 // Projection add: out = in + round(b + W^T saved) computed in fp32, rounded once.

@@ -695,17 +695,44 @@ __device__ inline S<1, NT> reduce(S<T, NT> const& s, Lane const& L) {
   return out;
 }
 
-// Copy n4 float4s of one per-feature vector into LDS (no barrier).
-__device__ inline void stage_vec(realx4* __restrict__ lds, real const* __restrict__ src, int n4) {
-  realx4 const* s4 = reinterpret_cast<realx4 const*>(src);
-  for (int i = threadIdx.x; i < n4; i += blockDim.x) lds[i] = s4[i];
+typedef __attribute__((address_space(3))) void* lds_ptr;
+
+// One 16-byte global_load_lds_dwordx4 per lane: lane l's 16 bytes at g land
+// in LDS at lds + 16 l (lds uniform across the wave, passed in M0).  Issued
+// as inline asm so that the compiler's wait insertion does not see an LDS
+// write it cannot place: it cannot tell apart regions of one LDS array
+// addressed at run time (the staging slots), so after the builtin it waits
+// for every outstanding request (vmcnt(0)) before the next read of the
+// array -- the first fragment read of every chunk waited for the requests
+// just made for two chunks ahead.  Every read of data requested here is
+// ordered by the kernel's own explicit waits (a vmcnt that leaves only
+// later requests outstanding, then a barrier where other waves' requests
+// are read); the compiler's own vmcnt values stay correct, because vector
+// memory loads complete in issue order and untracked requests only make
+// them wait longer.  The s_nop is the wait state the hardware needs
+// between the write of M0 and an LDS DMA, which the compiler inserts for
+// its own instructions but not in front of inline asm.
+__device__ inline void dma16(void const* g, void* lds) {
+  unsigned const m0 = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(reinterpret_cast<uint64_t>((lds_ptr)lds)));
+  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "{m0}"(m0) : "memory");
 }
 
-// Stage `count` values (a multiple of 4) of packed parameters into LDS.
-__device__ inline void stage(realx4* __restrict__ lds, real const* __restrict__ src, int count) {
-  realx4 const* s4 = reinterpret_cast<realx4 const*>(src);
-  for (int i = threadIdx.x; i < count / 4; i += blockDim.x) lds[i] = s4[i];
-  __syncthreads();
+// Every outstanding vector-memory operation of this wave done (vmcnt(0)).
+__device__ inline void wait_vmem() { __builtin_amdgcn_s_waitcnt(0x0F70); }
+
+// N16 16-byte pieces of packed parameters into LDS once per workgroup, 64
+// pieces a request, the requests dealt to its WAVES waves from wave TURN on.
+// The caller waits (wait_vmem) and synchronizes before the first read, once
+// for all such copies: all of them are in flight together.  (Copied through
+// registers in a loop each, every turn of every loop waited for memory: fp32
+// 16-64-64-64-8, 42 KB, and the 17 vectors of a four-block residual chain.)
+template <int N16, int WAVES, int TURN>
+__device__ inline void stage16(void* lds, void const* src) {
+  int const wave = wave_id(), lane = threadIdx.x & 63;
+#pragma unroll
+  for (int c = 0; c < (N16 + 63) / 64; c++)
+    if (wave == (TURN + c) % WAVES && 64 * c + lane < N16)
+      dma16(static_cast<char const*>(src) + 16 * (64 * c + lane), static_cast<char*>(lds) + 1024 * c);
 }
 
 }  // namespace fused
