@@ -99,11 +99,23 @@ __device__ inline void workgroup_barrier() {
 // rows at any alignment).
 enum InputMode { IN_VEC = 0, IN_DWORD = 1, IN_ELEMENT = 2 };
 
+// tanh of fp32 plans.  The hardware form 1 - 2 / (1 + e^2x) is off by up to an
+// ulp of one, which near zero is not an ulp of the result: there, x p(x^2)
+// with p a Chebyshev fit of tanh(x) / x (1e-9 on |x| <= 0.55).
+__device__ inline float tanh_f32(float x) {
+  float const t = x * x;
+  float q = fmaf(t, -0.00623885f, 0.02104217f);
+  q = fmaf(t, q, -0.05384337f);
+  q = fmaf(t, q, 0.13332468f);
+  q = fmaf(t, q, -0.33333311f);
+  return __builtin_fabsf(x) <= 0.55f ? fmaf(x * t, q, x) : act_tanh_fast(x);
+}
+
 // The epilogue steps that run on the accumulators: each(f) for one of them,
 // false for any other.  fp32 and 16-bit plans take the logistic family's
 // hardware forms, as the generated kernels do (pointwise.h); fp64 keeps
 // libm's, whose code for every accumulator at once is too long.
-template <class C, class Each>
+template <class C, bool Precise, class Each>
 __device__ inline bool usual_step(Step const& st, Each&& each) {
   C const a = C(st.a);
   switch (st.act) {
@@ -113,7 +125,10 @@ __device__ inline bool usual_step(Step const& st, Each&& each) {
   }
   if constexpr (sizeof(C) == 4) {
     switch (st.act) {
-      case ACT_TANH: each([](C v) { return act_tanh_fast(v); }); return true;
+      case ACT_TANH:
+        if constexpr (Precise) each([](C v) { return tanh_f32(v); });
+        else each([](C v) { return act_tanh_fast(v); });
+        return true;
       case ACT_SIGMOID: each([](C v) { return act_sigmoid_fast(v); }); return true;
       case ACT_SILU: each([](C v) { return act_silu_fast(v); }); return true;
       case ACT_GELU_TANH: each([](C v) { return act_gelu_tanh_fast(v); }); return true;
@@ -299,7 +314,7 @@ __global__ __launch_bounds__(256, 2) void layered_dense(DenseArgs a) {
       }
       continue;
     }
-    bool const done = usual_step<C>(st, [&](auto f) {
+    bool const done = usual_step<C, ES == 4>(st, [&](auto f) {
 #pragma unroll
       for (int i = 0; i < MI; i++)
 #pragma unroll
