@@ -1533,12 +1533,12 @@ int fused_prepare(ponni_plan_s& p, bool io32, FusedForm form, std::string& error
   st = load_module(key, code, fused_kernel_name(p) + cfg.suffix(), cfg.waves * 64, m, dev, error);
   if (st != PONNI_OK) return st;
   // The persistent grid's size, looked up once rather than at every launch.
-  if (hipDeviceGetAttribute(&p.fused_cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-      p.fused_cus <= 0) {
+  int cus = 0;
+  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) {
     error = "no compute units";
     return PONNI_ERR_DEVICE;
   }
-  FusedKernel& k = p.kernels[io32][form];
+  FusedKernel k;
   // (a kernel that spills registers already gains nothing from the form for
   // misaligned rows, which needs a few more: fp16 32-128-16 residual, 15
   // spilled, 1,000,003 columns 484 against 490 us)
@@ -1546,10 +1546,16 @@ int fused_prepare(ponni_plan_s& p, bool io32, FusedForm form, std::string& error
   k.columns_per_block = cfg.columns_per_block;
   k.waves = cfg.waves;
   k.wave_columns = cfg.by_wave ? cfg.columns_per_block / cfg.waves : 0;
-  k.resident = 0;
   if (!split && (cfg.lds_bytes > 0 || cfg.vec_bytes > 0 || cfg.params_in_registers || cfg.persistent_loop))
-    k.resident = int64_t(p.fused_cus) * (m->blocks_per_cu > 0 ? m->blocks_per_cu : 1);
+    k.resident = int64_t(cus) * (m->blocks_per_cu > 0 ? m->blocks_per_cu : 1);
   k.fn = m->fn;
+  // Forward passes of other threads may be running on the plan: a form is
+  // published once, its handle last.
+  static std::mutex publishing;
+  std::lock_guard<std::mutex> lock(publishing);
+  FusedKernel& slot = p.kernels[io32][form];
+  if (slot.loaded()) return PONNI_OK;
+  if (main) p.fused_cus = cus;
   if (main && p.path == PONNI_PATH_FUSED) {
     bool const half = p.dtype == PONNI_F16 || p.dtype == PONNI_BF16;
     int widest = 0;
@@ -1566,6 +1572,7 @@ int fused_prepare(ponni_plan_s& p, bool io32, FusedForm form, std::string& error
     p.split_always = half ? fused_nt(p) == 1 && spills >= 100
                           : spills > 0 || (fused_nt(p) == 1 && cfg.waves_per_simd == 1);
   }
+  slot.publish(k);
   return PONNI_OK;
 }
 
@@ -1601,7 +1608,7 @@ FusedForm fused_wanted_form(ponni_plan_s const& p, void const* x, int64_t ld_in,
 
 hipError_t fused_launch(ponni_plan_s const& p, LaunchArgs const& a, bool io32, hipStream_t stream) {
   FusedForm form = fused_wanted_form(p, a.x, a.ld_x, a.batch, io32);
-  if (p.kernels[io32][form].fn == nullptr) form = FUSED_MAIN;
+  if (!p.kernels[io32][form].loaded()) form = FUSED_MAIN;
   FusedKernel const& k = p.kernels[io32][form];
   // (a persistent grid whose tiles go to waves takes every CU it has tiles for)
   int64_t const columns = k.wave_columns > 0 ? k.wave_columns : k.columns_per_block;

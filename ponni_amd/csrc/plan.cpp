@@ -1019,7 +1019,7 @@ int upload(ponni_plan_s& p) {
     p.d_params_bytes = bytes;
   }
   if (count > 0) HIP_TRY(hipMemcpy(p.d_params, packed, count * param_element_size(p), hipMemcpyHostToDevice));
-  if ((p.path == PONNI_PATH_FUSED || p.narrow_jit) && p.kernels[0][0].fn == nullptr) {
+  if ((p.path == PONNI_PATH_FUSED || p.narrow_jit) && !p.kernels[0][FUSED_MAIN].loaded()) {
     std::string error;
     int const st = fused_prepare(p, false, FUSED_MAIN, error);
     if (st != PONNI_OK) return fail(st, error);
@@ -1465,10 +1465,10 @@ int forward_impl(ponni_plan plan, const void* x, int64_t ld_in, void* y, int64_t
   // The kernels of this call that are not loaded yet.  (A captured stream
   // cannot load a module: a plan whose form for this call is not there yet
   // then runs its main kernel, which takes any call.)
-  bool const need_rows = io32 && plan->kernels[1][FUSED_MAIN].fn == nullptr;
+  bool const need_rows = io32 && !plan->kernels[1][FUSED_MAIN].loaded();
   FusedForm const form = no_alloc ? FUSED_MAIN : fused_wanted_form(*plan, x, ld_in, batch, io32);
   bool const generated = plan->path == PONNI_PATH_FUSED || plan->narrow_jit;
-  if (generated && (need_rows || plan->kernels[io32][form].fn == nullptr)) {
+  if (generated && (need_rows || !plan->kernels[io32][form].loaded())) {
     hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
     bool const can_load =
         hipStreamIsCapturing(stream, &capturing) == hipSuccess && capturing == hipStreamCaptureStatusNone;
@@ -1480,7 +1480,7 @@ int forward_impl(ponni_plan plan, const void* x, int64_t ld_in, void* y, int64_t
       if (st != PONNI_OK) return fail(st, error);
     }
     FusedForm const wanted = fused_wanted_form(*plan, x, ld_in, batch, io32);
-    if (plan->kernels[io32][wanted].fn == nullptr && can_load) {
+    if (!plan->kernels[io32][wanted].loaded() && can_load) {
       int const st = fused_prepare(*plan, io32, wanted, error);
       if (st != PONNI_OK) return fail(st, error);
     }

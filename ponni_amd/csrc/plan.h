@@ -66,6 +66,18 @@ struct FusedKernel {
   int64_t resident = 0;  // a persistent grid's workgroups (0: one per column block)
   bool rows_in_lds = false;  // its input rows go through LDS a tile ahead
   int wave_columns = 0;  // columns of a tile where tiles go to waves (0: to workgroups)
+
+  // A form may be loaded by one thread's forward pass while others launch:
+  // the other members hold once loaded() is true.
+  bool loaded() const { return __atomic_load_n(&fn, __ATOMIC_ACQUIRE) != nullptr; }
+  void publish(FusedKernel const& k) {
+    columns_per_block = k.columns_per_block;
+    waves = k.waves;
+    resident = k.resident;
+    rows_in_lds = k.rows_in_lds;
+    wave_columns = k.wave_columns;
+    __atomic_store_n(&fn, k.fn, __ATOMIC_RELEASE);
+  }
 };
 
 // Kinds of packed parameter slots (plan.cpp visit_param_slots).

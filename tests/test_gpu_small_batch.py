@@ -157,3 +157,44 @@ def test_half_rows_at_any_alignment_through_lds(cuda, chain, dtype):
         got = ys[:, off:off + B].double().cpu().numpy()
         assert np.isfinite(got).all()
         check_half(got[:, pick], want)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "f16"])
+def test_forms_first_used_by_several_threads(cuda, dtype):
+    """One plan whose other kernels (small batches, misaligned rows) are first
+    needed by several threads at once, each on a stream of its own: every
+    thread's outputs are those of a plan used by one thread."""
+    import threading
+
+    import torch
+
+    layers = CHAINS["odd_tiles"](np.random.default_rng(80))
+    tdt = getattr(torch, TORCH_DT[dtype])
+    one = P.create_inference_model(*layers, dtype=dtype, path="fused")
+    shared = P.create_inference_model(*layers, dtype=dtype, path="fused")
+    n_in = one.get_num_inputs()
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    xs = [torch.randn((n_in, B), device="cuda", generator=gen).to(tdt) for B in (150_000, 64, 150_001, 515)]
+    want = [one.forward_batch_parallel(x) for x in xs]
+    shared.forward_batch_parallel(xs[0])  # parameters on the device, the main kernel loaded
+    torch.cuda.synchronize()
+    start, errors = threading.Barrier(len(xs)), []
+
+    def work(i):
+        try:
+            with torch.cuda.stream(torch.cuda.Stream()):
+                start.wait(30)
+                for j in [i, *range(len(xs))]:
+                    y = shared.forward_batch_parallel(xs[j])
+                    torch.cuda.current_stream().synchronize()
+                    if not torch.equal(y, want[j]):
+                        errors.append((i, j))
+        except Exception as e:  # noqa: BLE001 (reported by the assertion below)
+            errors.append((i, repr(e)))
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(len(xs))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(60)
+    assert not any(t.is_alive() for t in threads) and not errors, errors
