@@ -78,6 +78,15 @@ def test_plan_info_and_path_selection():
     assert create([P.Matvec(np.ones((300, 8)))], dtype="f64").path == "generic"
 
 
+@pytest.mark.parametrize("w, dtype, path", [
+    ((9, 600, 9), "f32", "layered"), ((40, 700, 30), "f32", "layered"), ((8, 600, 8), "f32", "generic"),
+    ((9, 300, 9), "f64", "layered"), ((9, 1100, 9), "f16", "layered"), ((9, 1100, 9), "bf16", "layered"),
+    ((9, 512, 9), "f32", "fused"), ((8, 600, 9), "f32", "layered")])
+def test_wide_chains_with_few_inputs_take_the_matrix_cores(w, dtype, path):
+    layers = [P.Matvec(np.ones((a, b))) for a, b in zip(w, w[1:])]
+    assert create(layers, dtype=dtype).path == path
+
+
 @pytest.mark.parametrize("seed", range(8))
 def test_scratch_planning_matches_reference_rules(seed):
     rng = np.random.default_rng(seed)
