@@ -613,17 +613,27 @@ std::string fused_source_once(ponni_plan_s const& p, FusedConfig& cfg, bool allo
   o.str("");
   o << "  Lane L;\n  L.lane = threadIdx.x & 63;\n  L.g = L.lane >> 4;\n  L.c = L.lane & 15;\n  L.batch = batch;\n";
   // Persistent kernels with no barrier in the tile loop deal tiles of one wave's
-  // columns to the waves, wave 0 of every workgroup first, so that a batch
-  // spreads over all CUs and SIMDs whatever its size (whole workgroups of 12
-  // waves in turn: fp32 24-96-48-10 graph, 262,144 columns, a last round on 171 of
-  // 256 CUs, 61.5 us; this way 56).  16-bit rows: pairs of waves take
-  // neighbouring tiles, the two halves of a cache line.
+  // columns to the waves.  A layer (one workgroup of every CU) whose waves all
+  // have a tile takes neighbouring ones per workgroup, which keeps rows together
+  // in HBM; in the last layer that is not full, wave 0 of every workgroup
+  // comes first, then wave 1, so that any batch spreads over all CUs and SIMDs
+  // (whole workgroups of 12 waves in turn: fp32 24-96-48-10 graph, 262,144
+  // columns, a last round on 171 of 256 CUs, 61.5 us; this way 55; wave 0 of every
+  // layer's workgroups first put two tiles on some SIMDs and none on others:
+  // fp64 9-25-7 residual chain, three workgroups per CU, 32,768 columns 32.5
+  // against 19.0 us).  16-bit rows: pairs of waves take neighbouring tiles
+  // there, the two halves of a cache line.
   cfg.by_wave = cfg.resident || (!half && !cfg.split && (cfg.lds_bytes > 0 || cfg.params_in_registers));
   int const tile_columns = cfg.by_wave ? 16 * NT : cfg.columns_per_block;
   o << "  int64_t const tiles = (batch + " << tile_columns - 1 << ") / " << tile_columns << ";\n";
-  std::string const first_tile = !cfg.by_wave ? "blockIdx.x"
-                                 : half       ? "(int64_t(wave_id() >> 1) * gridDim.x + blockIdx.x) * 2 + (wave_id() & 1)"
-                                              : "int64_t(wave_id()) * gridDim.x + blockIdx.x";
+  if (cfg.by_wave) {
+    o << "  int const layer = blockIdx.x / " << kChipCus << " * " << kChipCus << ", in_layer = blockIdx.x - layer;\n";
+    o << "  int const width = gridDim.x - layer < " << kChipCus << " ? gridDim.x - layer : " << kChipCus << ";\n";
+    o << "  int const in_full = in_layer * " << cfg.waves << " + wave_id(), in_last = "
+      << (half ? "((wave_id() >> 1) * width + in_layer) * 2 + (wave_id() & 1)" : "wave_id() * width + in_layer") << ";\n";
+    o << "  auto tile_from = [&](int64_t base) {\n    int64_t const first = base + layer * " << cfg.waves
+      << ";\n    return first + (first + width * " << cfg.waves << " <= tiles ? in_full : in_last);\n  };\n";
+  }
   std::string const tile_step = cfg.by_wave ? "int64_t(gridDim.x) * " + std::to_string(cfg.waves) : "gridDim.x";
   auto column_of = [&](std::string const& tile) {
     std::string const c = std::to_string(16 * NT);
@@ -678,7 +688,8 @@ std::string fused_source_once(ponni_plan_s const& p, FusedConfig& cfg, bool allo
     // others (the batch's last tile) load directly.
     if (cfg.any_rows) o << "  constexpr bool xvec = true;\n";
     else o << "  bool const xvec = ((reinterpret_cast<uint64_t>(x) | uint64_t(ldx) * " << io_bytes << ") & 15) == 0;\n";
-    o << "  int64_t const tile0 = " << first_tile << ";\n  L.col0 = " << column_of("tile0") << ";\n";
+    o << "  int64_t const tile0 = " << (cfg.by_wave ? "tile_from(0)" : "blockIdx.x") << ";\n  L.col0 = " << column_of("tile0")
+      << ";\n";
     o << "  if (tile0 < tiles && xvec && L.col0 + " << WCOLS << " <= batch) " << prefetch("L") << "\n";
     // The LDS writes of these loads complete with vmcnt, which the compiler
     // does not track (fused_f16.h dma16): each tile's rows are waited for
@@ -689,7 +700,9 @@ std::string fused_source_once(ponni_plan_s const& p, FusedConfig& cfg, bool allo
   // (the small-batch kernel runs one tile per workgroup: its exchange buffers
   // alternate within a tile only)
   if (cfg.split) o << "  if (int64_t const tile = blockIdx.x; tile < tiles) {\n";
-  else o << "  for (int64_t tile = " << (in_dma ? "tile0" : first_tile) << "; tile < tiles; tile += " << tile_step << ") {\n";
+  else if (cfg.by_wave)
+    o << "  for (int64_t base = 0, tile = tile_from(0); tile < tiles; base += " << tile_step << ", tile = tile_from(base)) {\n";
+  else o << "  for (int64_t tile = blockIdx.x; tile < tiles; tile += " << tile_step << ") {\n";
   o << "    L.col0 = " << column_of("tile") << ";\n";
   // Register-resident parameters may be hoisted out of the tile loop; otherwise
   // pin() hides the pointer's loop invariance so they are re-read per tile.
@@ -705,8 +718,9 @@ std::string fused_source_once(ponni_plan_s const& p, FusedConfig& cfg, bool allo
       << (cfg.any_rows ? "x, ldx, " : "") << "in_buf[wave_id()], L) : load_rows_h<" << cur_n << ", " << NT
       << ", E>(x, ldx, L);\n";
     o << "    wait_lds();\n";
-    o << "    Lane Ln = L;\n    Ln.col0 = " << column_of("tile + " + tile_step) << ";\n";
-    o << "    bool const pre_next = tile + " << tile_step << " < tiles && xvec && Ln.col0 + " << WCOLS << " <= batch;\n";
+    o << "    int64_t const next = " << (cfg.by_wave ? "tile_from(base + " : "tile + (") << tile_step << ");\n";
+    o << "    Lane Ln = L;\n    Ln.col0 = " << column_of("next") << ";\n";
+    o << "    bool const pre_next = next < tiles && xvec && Ln.col0 + " << WCOLS << " <= batch;\n";
     if (hook_dense < 0) o << "    " << prefetch_next << "\n";
   } else if (half) o << "    auto " << cur << " = load_rows_h<" << cur_n << ", " << NT << ", E>(x, ldx, L);\n";
   else o << "    auto " << cur << " = " << (in_k.empty() ? "load_rows<" : "load_rows_k<") << cur_n << ">(x, ldx, L);\n";
@@ -1610,9 +1624,14 @@ hipError_t fused_launch(ponni_plan_s const& p, LaunchArgs const& a, bool io32, h
   FusedForm form = fused_wanted_form(p, a.x, a.ld_x, a.batch, io32);
   if (!p.kernels[io32][form].loaded()) form = FUSED_MAIN;
   FusedKernel const& k = p.kernels[io32][form];
-  // (a persistent grid whose tiles go to waves takes every CU it has tiles for)
   int64_t const columns = k.wave_columns > 0 ? k.wave_columns : k.columns_per_block;
   int64_t grid = (a.batch + columns - 1) / columns;
+  if (k.wave_columns > 0) {
+    // As many workgroups per CU as the tiles need waves (further ones would
+    // only copy the parameters).
+    int64_t const round = int64_t(p.fused_cus) * k.waves;
+    grid = std::min(grid, (grid + round - 1) / round * p.fused_cus);
+  }
   if (k.resident > 0 && grid > k.resident) grid = k.resident;
   void const* params = a.params;
   void const* x = a.x;

@@ -12,6 +12,8 @@ namespace ponni_hip {
 constexpr int64_t kFusedLdsParamBytes = 64 * 1024;
 // LDS of one workgroup on gfx950.
 constexpr int kFusedLdsBytes = 160 * 1024;
+// CUs of an MI355X: workgroups i, i + kChipCus, ... of a launch share one.
+constexpr int kChipCus = 256;
 
 struct FusedConfig {
   int lds_bytes = 0;          // 0: parameters stream from L2

@@ -198,3 +198,36 @@ def test_forms_first_used_by_several_threads(cuda, dtype):
     for t in threads:
         t.join(60)
     assert not any(t.is_alive() for t in threads) and not errors, errors
+
+
+def test_one_tile_per_simd_costs_what_fewer_do(cuda):
+    """Tiles dealt to waves spread over the SIMDs before any takes a second
+    one, at every number of workgroups per CU (three here, where wave 0 of each
+    was dealt to first and a SIMD took two of 32,768 columns' 1,024 tiles: 1.6 times
+    the time of 16,384 columns)."""
+    import torch
+
+    r = np.random.default_rng(81)
+    layers = [P.Matvec(_w(r, 9, 25))]
+    for _ in range(2):
+        layers += [P.Save_State(0, 25), P.LayerNorm(25), P.Matvec(_w(r, 25, 25)), P.Gelu(25, True),
+                   P.Matvec(_w(r, 25, 25)), P.Binop_Add(0, 25)]
+    m = P.create_inference_model(*layers, P.Matvec(_w(r, 25, 7)), dtype="f64", path="fused")
+    A = P._abi
+    A.check(A.lib().ponni_plan_device_params(m._plan, ctypes.byref(ctypes.c_void_p())))  # main kernel only
+    us = {}
+    for B in (16_384, 32_768):
+        x = torch.randn((9, B), dtype=torch.float64, device="cuda:0")
+        y = torch.empty((7, B), dtype=torch.float64, device="cuda:0")
+        runs = []
+        for _ in range(12):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(20):
+                m.forward_raw_no_alloc(x.data_ptr(), B, y.data_ptr(), B, B, torch.cuda.current_stream().cuda_stream)
+            b.record()
+            torch.cuda.synchronize()
+            runs.append(a.elapsed_time(b) * 50)
+        us[B] = min(runs)
+    print(f"one tile per SIMD: {us[32_768]:.1f} us, every other SIMD {us[16_384]:.1f}", flush=True)
+    assert us[32_768] < 1.3 * us[16_384]
