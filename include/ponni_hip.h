@@ -447,6 +447,14 @@ int ponni_plan_compile(ponni_plan plan);
 int ponni_plan_kernel_config(ponni_plan plan, int32_t* threads, int32_t* columns_per_block,
                              int32_t* persistent);
 
+/* The form of a FUSED plan's generated kernel that ponni_forward runs a batch
+ * on, of rows whose starts are multiples of row_alignment bytes (fp32_rows:
+ * ponni_forward_fp32_rows): 0 the main one, 1 the one for small batches, 2 the
+ * one for 16-bit rows that do not start on 16 bytes.  Compiles what the answer
+ * depends on; no device required. */
+int ponni_plan_call_form(ponni_plan plan, int64_t batch, int32_t row_alignment,
+                         int32_t fp32_rows, int32_t* form);
+
 /* Device pointer to the plan's packed parameters in its kernel's layout
  * (uploading them first if they changed; synchronizes the device then):
  * the first argument of the generated kernel. */

@@ -185,6 +185,8 @@ def lib() -> ctypes.CDLL:
     L.ponni_plan_kernel_source.argtypes = [vp, ctypes.c_char_p, i64]
     L.ponni_plan_program_source.restype = i64
     L.ponni_plan_program_source.argtypes = [vp, ctypes.c_char_p, i64]
+    L.ponni_plan_call_form.restype = ctypes.c_int
+    L.ponni_plan_call_form.argtypes = [vp, i64, ctypes.c_int32, ctypes.c_int32, ctypes.POINTER(ctypes.c_int32)]
     L.ponni_plan_compile.restype = ctypes.c_int
     L.ponni_plan_compile.argtypes = [vp]
     L.ponni_plan_kernel_config.restype = ctypes.c_int

@@ -22,6 +22,7 @@
 #include <string>
 #include <vector>
 #include <climits>
+#include <cmath>
 #include <dlfcn.h>
 #include <link.h>
 #include <sys/stat.h>
@@ -1529,15 +1530,90 @@ int load_module(std::string const& key, std::vector<char> const& code, std::stri
 
 }  // namespace
 
-int fused_prepare(ponni_plan_s& p, bool io32, FusedForm form, std::string& error) {
-  bool const split = form == FUSED_SMALL;
-  std::string key;
-  std::vector<char> code;
+namespace {
+
+// A round of the main kernel takes a wave's whole pass however few columns the
+// batch has, and a batch just over a round takes two; the small-batch kernel's
+// time grows with the batch from about a quarter of a round, or by whole
+// workgroups per CU in 16-bit chains that stream their weights.  The slope is
+// split_cost_ratio times a factor for the classes of plans that estimate does
+// not fit.  Base, factors and bounds: from both kernels' times over 304 random
+// plans of every class (widths 24 to 1024, mlp, residual, graph) at 8 to 19
+// batches from 0.1 to 16 rounds each: of the 933 where the rule picks the
+// small-batch kernel it is slower by over 4 % in 2 (worst 1.10); where it picks
+// the main one the small-batch kernel would be 6 % faster on average, most of
+// that in fp32 residual chains of 257 features and more.
+SmallBatchRule small_batch_rule(ponni_plan_s const& p, FusedConfig const& main, std::vector<char> const& code) {
+  SmallBatchRule r;
+  bool const half = p.dtype == PONNI_F16 || p.dtype == PONNI_BF16;
+  bool repeated = false;
+  int contraction = 0;
+  for (Op const& op : p.ops) {
+    if (op.code == OP_DENSE || op.code == OP_PROJ_ADD) contraction = std::max(contraction, tiles(op.n_out));
+    repeated = repeated || (op.code != OP_DENSE && op.code != OP_SAVE && op.code != OP_LOAD);
+  }
+  // (fp32 and 16-bit models of at most two tiles run at the launch floor either way)
+  if (contraction < (p.dtype == PONNI_F64 ? 2 : 3)) return r;
+  int const spills = metadata_int(code, ".vgpr_spill_count");
+  bool const one_tile = fused_nt(p) == 1;
+  double const ratio = split_cost_ratio(p);
+  r.columns = main.by_wave ? 4 * main.columns_per_block / main.waves : main.columns_per_block;
+  r.rounds = main.by_wave ? 1 : 2;  // (tiles dealt to waves share the SIMDs instead of taking a second round)
+  r.base = 0.25;
+  r.slope = ratio;
+  if (half && !main.by_wave && (one_tile || !repeated)) {
+    FusedConfig small;
+    split_shape(p, small);
+    r.step = 16 * small.split_nt;
+    r.base = 0.2;
+    r.slope = ratio * (!one_tile ? 1.25 : !repeated ? 1.2 : spills >= 200 ? 1.5 : 2.0);
+    r.spilled = ratio * 1.9;
+  } else if (p.dtype == PONNI_F32 && one_tile && repeated) {
+    r.slope = 1.5 * ratio;
+  }
+  // Where the main kernel is the slower one at every batch (131,072 columns,
+  // TFLOP/s, main against small-batch): fp32 chains with two column tiles that
+  // spill (12-245-35 residual, 179 registers, 41 against 92; 22-235-2, 13, 75
+  // against 93; none of 40 plans slower), fp32 chains wider than 448 features
+  // with one wave per SIMD (20-464-464-464-60 57 against 106; 13 plans, the
+  // slowest 1.04 times the main kernel's time; narrower ones up to 1.45), and
+  // fp64 chains that spill hundreds (39-225-46 residual, 1371, 4605 against 2415 us).
+  // 16-bit chains that spill run faster on the main kernel (55-448-48 residual,
+  // 339, 65,536 columns, 248 against 605 us).
+  if (p.dtype == PONNI_F32) r.always = one_tile ? main.waves_per_simd == 1 && !repeated && tiles(p.max_width) > 28 : spills >= 8;
+  if (p.dtype == PONNI_F64) r.always = spills >= 600;
+  return r;
+}
+
+}  // namespace
+
+static FusedConfig form_config(bool io32, FusedForm form) {
   FusedConfig cfg;
   cfg.io32 = io32;
-  cfg.split = split;
+  cfg.split = form == FUSED_SMALL;
   cfg.any_rows = form == FUSED_ANY_ROWS;
-  cfg.resident = !split;
+  cfg.resident = !cfg.split;
+  return cfg;
+}
+
+// A compiled form's launch shape (cfg as fused_source left it).
+static FusedKernel fused_kernel(FusedConfig const& cfg, std::vector<char> const& code) {
+  FusedKernel k;
+  k.spills = std::max(metadata_int(code, ".vgpr_spill_count"), 0);
+  // (a kernel that spills registers already gains nothing from the form for
+  // misaligned rows, which needs a few more: fp16 32-128-16 residual, 15
+  // spilled, 1,000,003 columns 484 against 490 us)
+  k.rows_in_lds = cfg.rows_in_lds && k.spills == 0;
+  k.columns_per_block = cfg.columns_per_block;
+  k.waves = cfg.waves;
+  k.wave_columns = cfg.by_wave ? cfg.columns_per_block / cfg.waves : 0;
+  return k;
+}
+
+int fused_prepare(ponni_plan_s& p, bool io32, FusedForm form, std::string& error) {
+  std::string key;
+  std::vector<char> code;
+  FusedConfig cfg = form_config(io32, form);
   bool const main = !io32 && form == FUSED_MAIN;  // (settles the plan's occupancy)
   int st = main ? fused_compile(p, true, key, code, error) : compile_cached(p, cfg, key, code, error);
   if (st != PONNI_OK) return st;
@@ -1552,15 +1628,8 @@ int fused_prepare(ponni_plan_s& p, bool io32, FusedForm form, std::string& error
     error = "no compute units";
     return PONNI_ERR_DEVICE;
   }
-  FusedKernel k;
-  // (a kernel that spills registers already gains nothing from the form for
-  // misaligned rows, which needs a few more: fp16 32-128-16 residual, 15
-  // spilled, 1,000,003 columns 484 against 490 us)
-  k.rows_in_lds = cfg.rows_in_lds && metadata_int(code, ".vgpr_spill_count") <= 0;
-  k.columns_per_block = cfg.columns_per_block;
-  k.waves = cfg.waves;
-  k.wave_columns = cfg.by_wave ? cfg.columns_per_block / cfg.waves : 0;
-  if (!split && (cfg.lds_bytes > 0 || cfg.vec_bytes > 0 || cfg.params_in_registers || cfg.persistent_loop))
+  FusedKernel k = fused_kernel(cfg, code);
+  if (!cfg.split && (cfg.lds_bytes > 0 || cfg.vec_bytes > 0 || cfg.params_in_registers || cfg.persistent_loop))
     k.resident = int64_t(cus) * (m->blocks_per_cu > 0 ? m->blocks_per_cu : 1);
   k.fn = m->fn;
   // Forward passes of other threads may be running on the plan: a form is
@@ -1570,54 +1639,64 @@ int fused_prepare(ponni_plan_s& p, bool io32, FusedForm form, std::string& error
   FusedKernel& slot = p.kernels[io32][form];
   if (slot.loaded()) return PONNI_OK;
   if (main) p.fused_cus = cus;
-  if (main && p.path == PONNI_PATH_FUSED) {
-    bool const half = p.dtype == PONNI_F16 || p.dtype == PONNI_BF16;
-    int widest = 0;
-    for (Op const& op : p.ops)
-      if (op.code == OP_DENSE || op.code == OP_PROJ_ADD) widest = std::max(widest, tiles(op.n_out));
-    // (fp32 and 16-bit models of at most two tiles run at the launch floor either way)
-    p.split_ratio = widest >= (p.dtype == PONNI_F64 ? 2 : 3) ? split_cost_ratio(p) : 0;
-    // The main kernel with spilled states, or with one column tile per wave
-    // and one wave per SIMD, is the slower one at every batch (262,144 columns:
-    // fp32 40-256-20 residual, 151 registers spilled, 2908 against 1435 us;
-    // fp32 24-384-384-12 1519 against 809; fp16 64-1024-1024-64, 259 spilled,
-    // 1028 against 791); 16-bit plans that spill few are not (62: 455 against 489).
-    int const spills = metadata_int(code, ".vgpr_spill_count");
-    p.split_always = half ? fused_nt(p) == 1 && spills >= 100
-                          : spills > 0 || (fused_nt(p) == 1 && cfg.waves_per_simd == 1);
-  }
+  if (main && p.path == PONNI_PATH_FUSED) p.small_batch = small_batch_rule(p, cfg, code);
   slot.publish(k);
   return PONNI_OK;
 }
 
-// A round of the main kernel (one workgroup per CU) takes a wave's whole pass
-// however few columns the batch has, and a batch just over a round takes two;
-// the small-batch kernel's time grows with the batch from about a quarter of
-// a round (measured 0.15-0.25 over the models below).  Measured at 10,000 /
-// 21,600 / 32,769 columns, main against small-batch: fp32 32-128-16 residual
-// 82 / 85 / 165 against 43 / 82 / 116 us; fp16 64-256-256-256-64 24 / 25 / 30
-// against 11 / 16 / 25; fp64 16-64-64-64-8 12.6 / 13.2 / 22.4 against 8.4 /
-// 13.2 / 17.4.  Beyond two rounds the main kernel's workgroups balance.
-static bool fused_wants_split(ponni_plan_s const& p, int64_t batch) {
-  if (p.split_ratio <= 0) return false;
-  if (p.split_always) return true;
-  FusedKernel const& main = p.kernels[0][0];
-  // (tiles dealt to waves: one wave per SIMD everywhere is the flat part; more
-  // waves then share the SIMDs instead of taking a second round)
-  int const columns = main.wave_columns > 0 ? 4 * main.wave_columns : main.columns_per_block;
-  double const rounds = double(batch) / (double(p.fused_cus) * columns);
-  return rounds <= (main.wave_columns > 0 ? 1 : 2) && 0.25 + p.split_ratio * rounds < (rounds <= 1 ? 1 : 2);
+// (a small-batch kernel of a 16-bit plan that spills so many registers is the
+// slower one at every batch: bf16 192-781-781-781-23, 203 spilled, 100 against
+// 87 us at 3,276 columns, 403 against 118 at 32,768)
+constexpr int kSmallBatchSpills = 100;
+
+static bool fused_wants_split(ponni_plan_s const& p, int64_t batch, bool io32) {
+  SmallBatchRule const& r = p.small_batch;
+  if (r.slope <= 0) return false;
+  bool const half = p.dtype == PONNI_F16 || p.dtype == PONNI_BF16;
+  int const spills = __atomic_load_n(&p.kernels[io32][FUSED_SMALL].spills, __ATOMIC_RELAXED);
+  if (half && spills >= kSmallBatchSpills) return false;
+  if (r.always) return true;
+  double const cus = p.fused_cus;
+  double const rounds = double(batch) / (cus * r.columns);
+  double const taken = r.step > 0 ? std::ceil(double(batch) / (cus * r.step)) * r.step / r.columns : rounds;
+  return rounds <= r.rounds && r.base + (half && spills > 0 ? r.spilled : r.slope) * taken < (rounds <= 1 ? 1 : 2);
 }
 
 FusedForm fused_wanted_form(ponni_plan_s const& p, void const* x, int64_t ld_in, int64_t batch, bool io32) {
   if (p.path != PONNI_PATH_FUSED) return FUSED_MAIN;
-  if (fused_wants_split(p, batch)) return FUSED_SMALL;
+  if (fused_wants_split(p, batch, io32)) return FUSED_SMALL;
   // Rows that do not start on 16 bytes, where aligned ones go through LDS a
   // tile ahead: element loads instead took half again the time (fp16
   // 64-256-256-256-64, 262,145 columns: 166 us, aligned 110).
   int const es = io32 ? 4 : 2;
   bool const aligned = ((reinterpret_cast<uint64_t>(x) | uint64_t(ld_in) * es) & 15) == 0;
   return p.kernels[io32][FUSED_MAIN].rows_in_lds && !aligned ? FUSED_ANY_ROWS : FUSED_MAIN;
+}
+
+int fused_call_form(ponni_plan_s& p, int64_t batch, int row_alignment, bool io32, FusedForm& form, std::string& error) {
+  form = FUSED_MAIN;
+  if (p.path != PONNI_PATH_FUSED) return PONNI_OK;
+  std::string key;
+  std::vector<char> code;
+  if (!p.kernels[0][FUSED_MAIN].loaded()) {
+    int const st = fused_compile(p, true, key, code, error);
+    if (st != PONNI_OK) return st;
+    FusedConfig cfg = form_config(false, FUSED_MAIN);
+    (void)fused_source(p, cfg);
+    p.small_batch = small_batch_rule(p, cfg, code);
+    if (p.fused_cus == 0) p.fused_cus = kChipCus;
+  }
+  for (FusedForm f : {FUSED_MAIN, FUSED_SMALL}) {
+    FusedKernel& k = p.kernels[io32][f];
+    if (k.loaded() || (f == FUSED_SMALL && !fused_wants_split(p, batch, io32))) continue;
+    FusedConfig cfg = form_config(io32, f);
+    int const st = compile_cached(p, cfg, key, code, error);
+    if (st != PONNI_OK) return st;
+    (void)fused_source(p, cfg);
+    k.describe(fused_kernel(cfg, code));
+  }
+  form = fused_wanted_form(p, reinterpret_cast<void const*>(uint64_t(row_alignment)), 0, batch, io32);
+  return PONNI_OK;
 }
 
 hipError_t fused_launch(ponni_plan_s const& p, LaunchArgs const& a, bool io32, hipStream_t stream) {

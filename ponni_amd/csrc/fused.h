@@ -57,6 +57,9 @@ int fused_prepare(ponni_plan_s& p, bool io32, FusedForm form, std::string& error
 // The form of the plan's kernel that a call runs on once it is loaded (the
 // main one takes any call).
 FusedForm fused_wanted_form(ponni_plan_s const& p, void const* x, int64_t ld_in, int64_t batch, bool io32);
+// The form that such a call runs on (rows that start on multiples of
+// row_alignment bytes), compiling what that depends on; needs no device.
+int fused_call_form(ponni_plan_s& p, int64_t batch, int row_alignment, bool io32, FusedForm& form, std::string& error);
 hipError_t fused_launch(ponni_plan_s const& p, LaunchArgs const& a, bool io32, hipStream_t stream);
 
 }  // namespace ponni_hip

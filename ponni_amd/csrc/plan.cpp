@@ -1709,6 +1709,20 @@ int ponni_plan_kernel_config(ponni_plan plan, int32_t* threads, int32_t* columns
   return PONNI_OK;
 }
 
+int ponni_plan_call_form(ponni_plan plan, int64_t batch, int32_t row_alignment, int32_t fp32_rows, int32_t* form) {
+  if (plan == nullptr || form == nullptr) return fail(PONNI_ERR_INVALID_ARGUMENT, "null argument");
+  if (batch <= 0 || batch > INT32_MAX || row_alignment <= 0) return fail(PONNI_ERR_SHAPE, "no such call");
+  if (plan->path != PONNI_PATH_FUSED) return fail(PONNI_ERR_UNSUPPORTED, "only FUSED plans have forms of their kernel");
+  bool const half = plan->dtype == PONNI_F16 || plan->dtype == PONNI_BF16;
+  if (fp32_rows && !half) return fail(PONNI_ERR_UNSUPPORTED, "fp32 rows: a 16-bit plan");
+  std::string error;
+  FusedForm f = FUSED_MAIN;
+  int const st = fused_call_form(*plan, batch, row_alignment, fp32_rows != 0, f, error);
+  if (st != PONNI_OK) return fail(st, error);
+  *form = f;
+  return PONNI_OK;
+}
+
 int ponni_plan_device_params(ponni_plan plan, const void** params) {
   if (plan == nullptr || params == nullptr) return fail(PONNI_ERR_INVALID_ARGUMENT, "null argument");
   if (plan->device_dirty) {

@@ -66,18 +66,35 @@ struct FusedKernel {
   int64_t resident = 0;  // a persistent grid's workgroups (0: one per column block)
   bool rows_in_lds = false;  // its input rows go through LDS a tile ahead
   int wave_columns = 0;  // columns of a tile where tiles go to waves (0: to workgroups)
+  int spills = 0;        // registers spilled (read by other threads at any time)
 
   // A form may be loaded by one thread's forward pass while others launch:
   // the other members hold once loaded() is true.
   bool loaded() const { return __atomic_load_n(&fn, __ATOMIC_ACQUIRE) != nullptr; }
-  void publish(FusedKernel const& k) {
+  void describe(FusedKernel const& k) {
     columns_per_block = k.columns_per_block;
     waves = k.waves;
     resident = k.resident;
     rows_in_lds = k.rows_in_lds;
     wave_columns = k.wave_columns;
+    __atomic_store_n(&spills, k.spills, __ATOMIC_RELAXED);
+  }
+  void publish(FusedKernel const& k) {
+    describe(k);
     __atomic_store_n(&fn, k.fn, __ATOMIC_RELEASE);
   }
+};
+
+// When a FUSED plan's small-batch kernel runs (fused.cpp fused_wants_split):
+// its time, in main-kernel rounds (one pass of a wave on every SIMD, or of a
+// workgroup on every CU), is base + slope * the rounds that the batch fills.
+struct SmallBatchRule {
+  double base = 0, slope = 0;  // (slope 0: the plan has no such kernel)
+  int columns = 0;             // of a round, per CU
+  int step = 0;                // its columns are taken in steps of so many per CU (0: as they are)
+  int rounds = 0;              // of a batch for which it can be the faster one, at most
+  bool always = false;         // the faster one at every batch
+  double spilled = 0;          // slope where it spills registers itself
 };
 
 // Kinds of packed parameter slots (plan.cpp visit_param_slots).
@@ -226,10 +243,7 @@ struct ponni_plan_s {
   // fragments (0: not settled yet).
   int fused_wps = 0;
   int resident_wps = 0;
-  // The small-batch kernel's time per column over the main one's (0: the plan
-  // has none), and whether it is the faster one at every batch.
-  double split_ratio = 0;
-  bool split_always = false;
+  ponni_hip::SmallBatchRule small_batch;  // settled with the main kernel
 
   // Parameter segments shared with caller-owned arrays (two per layer at
   // most), and the gather map that refreshes the device-shared ones.

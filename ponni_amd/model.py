@@ -269,6 +269,13 @@ class Inference:
         A.check(A.lib().ponni_plan_kernel_config(self._plan, ctypes.byref(t), ctypes.byref(c), ctypes.byref(p)))
         return t.value, c.value, bool(p.value)
 
+    def call_form(self, batch: int, row_alignment: int = 16, fp32_rows: bool = False) -> str:
+        """The form of a FUSED plan's kernel that a forward pass of such a batch
+        runs on (ponni_plan_call_form): "main", "small" or "any_rows"."""
+        f = ctypes.c_int32()
+        A.check(A.lib().ponni_plan_call_form(self._plan, batch, row_alignment, int(fp32_rows), ctypes.byref(f)))
+        return ("main", "small", "any_rows")[f.value]
+
     def compile(self) -> None:
         A.check(A.lib().ponni_plan_compile(self._plan))
 

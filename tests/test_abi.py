@@ -281,6 +281,39 @@ def test_fused_kernels_compile_on_the_host(seed, tmp_path, monkeypatch):
     assert any(f.suffix == ".co" for f in tmp_path.iterdir())
 
 
+def _residual_chain(n, w, out, blocks):
+    layers = [P.Matvec(np.ones((n, w)))]
+    for _ in range(blocks):
+        layers += [P.Save_State(0, w), P.LayerNorm(w), P.Matvec(np.ones((w, w))), P.Bias(np.ones(w)), P.Gelu(w, True),
+                   P.Matvec(np.ones((w, w))), P.Bias(np.ones(w)), P.Binop_Add(0, w)]
+    return layers + [P.Matvec(np.ones((w, out)))]
+
+
+def _mlp_chain(widths, act):
+    layers = []
+    for i, (a, b) in enumerate(zip(widths, widths[1:])):
+        layers += [P.Matvec(np.ones((a, b))), P.Bias(np.ones(b))] + ([act(b)] if i < len(widths) - 2 else [])
+    return layers
+
+
+@pytest.mark.parametrize("chain, dtype, forms", [
+    # kernels with one tile of columns a workgroup, measured the faster ones (us, main against small-batch)
+    ("residual 32 128 16 4", "f32", {10_000: "small", 1_000_000: "main"}),          # 82 against 43
+    ("mlp 64 250 250 250 64", "f16", {21_600: "small", 262_144: "main"}),           # 25 against 14
+    ("mlp 20 464 464 464 60", "f32", {1_000: "small", 1_000_000: "small"}),         # 57 against 106 TFLOP/s
+    # and the slower ones where the main kernel spills registers or is wide
+    ("residual 28 116 2 2", "f32", {910_433: "main"}),                              # 1350 against 1704
+    ("residual 29 144 20 1", "f64", {1_000: "small", 131_072: "main"}),             # 346 against 516
+    ("mlp 192 781 781 781 23", "bf16", {3_276: "main", 32_768: "main"}),            # 87 against 100, 118 against 403
+    ("mlp 28 425 425 425 19", "f32", {131_072: "main"})])                           # 118 against 81 TFLOP/s
+def test_small_batch_kernel_runs_where_it_is_faster(chain, dtype, forms):
+    kind, *n = chain.split()
+    n = [int(v) for v in n]
+    layers = _residual_chain(*n) if kind == "residual" else _mlp_chain(n, P.Silu if dtype == "bf16" else P.Tanh)
+    m = create(layers, dtype=dtype, path="fused")
+    assert {B: m.call_form(B) for B in forms} == forms
+
+
 _COMPILE_C2 = """
 import sys
 if sys.argv[1] == "torch":
