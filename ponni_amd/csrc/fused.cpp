@@ -1561,10 +1561,12 @@ SmallBatchRule small_batch_rule(ponni_plan_s const& p, FusedConfig const& main, 
   r.rounds = main.by_wave ? 1 : 2;  // (tiles dealt to waves share the SIMDs instead of taking a second round)
   r.base = 0.25;
   r.slope = ratio;
+  FusedConfig small;
+  split_shape(p, small);
+  r.block_columns = 16 * small.split_nt;
+  r.block_threads = 64 * small.split_waves;
   if (half && !main.by_wave && (one_tile || !repeated)) {
-    FusedConfig small;
-    split_shape(p, small);
-    r.step = 16 * small.split_nt;
+    r.step = r.block_columns;
     r.base = 0.2;
     r.slope = ratio * (!one_tile ? 1.25 : !repeated ? 1.2 : spills >= 200 ? 1.5 : 2.0);
     r.spilled = ratio * 1.9;
@@ -1655,6 +1657,9 @@ static bool fused_wants_split(ponni_plan_s const& p, int64_t batch, bool io32) {
   bool const half = p.dtype == PONNI_F16 || p.dtype == PONNI_BF16;
   int const spills = __atomic_load_n(&p.kernels[io32][FUSED_SMALL].spills, __ATOMIC_RELAXED);
   if (half && spills >= kSmallBatchSpills) return false;
+  // (a launch takes fewer than 2^32 threads, which one workgroup per
+  // block_columns columns reaches at 2^27 columns or more)
+  if (uint64_t((batch + r.block_columns - 1) / r.block_columns) * unsigned(r.block_threads) > UINT32_MAX) return false;
   if (r.always) return true;
   double const cus = p.fused_cus;
   double const rounds = double(batch) / (cus * r.columns);

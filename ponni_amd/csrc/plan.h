@@ -91,6 +91,7 @@ struct FusedKernel {
 struct SmallBatchRule {
   double base = 0, slope = 0;  // (slope 0: the plan has no such kernel)
   int columns = 0;             // of a round, per CU
+  int block_columns = 16, block_threads = 256;  // its workgroups
   int step = 0;                // its columns are taken in steps of so many per CU (0: as they are)
   int rounds = 0;              // of a batch for which it can be the faster one, at most
   bool always = false;         // the faster one at every batch

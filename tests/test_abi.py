@@ -314,6 +314,16 @@ def test_small_batch_kernel_runs_where_it_is_faster(chain, dtype, forms):
     assert {B: m.call_form(B) for B in forms} == forms
 
 
+@pytest.mark.parametrize("dtype, widths", [("f32", (20, 464, 464, 60)), ("f16", (20, 520, 24))])
+def test_small_batch_kernel_within_a_launch(dtype, widths):
+    """One workgroup of 256 or 512 threads for 16 or 32 columns: a launch holds
+    fewer than 2^32 threads, so larger batches run on the main kernel."""
+    m = create(_mlp_chain(widths, P.Relu), dtype=dtype, path="fused")
+    if dtype == "f32":  # a plan that runs every other batch on the small-batch kernel
+        assert m.call_form(2**28 - 16) == "small"
+    assert [m.call_form(B) for B in (2**28, 2**31 - 1)] == ["main", "main"]
+
+
 _COMPILE_C2 = """
 import sys
 if sys.argv[1] == "torch":
