@@ -766,6 +766,7 @@ std::string fused_source_once(ponni_plan_s const& p, FusedConfig& cfg, bool allo
   size_t next_begin = 0, at = 0;
   int exchange_tiles = 0;
   int parity = 0;
+  bool input_read = false;  // by every wave
   std::string const SW = std::to_string(cfg.waves);
   auto begin_next = [&]() {
     if (next_begin >= contractions.size()) return;
@@ -779,6 +780,10 @@ std::string fused_source_once(ponni_plan_s const& p, FusedConfig& cfg, bool allo
     std::string const buf = "xbuf[" + std::to_string(parity) + "]";
     parity ^= 1;
     o << "    split_put<" << tiles(n) << ", " << SW << ">(" << buf << ", " << own << ", wv, L);\n";
+    // (y may be x: every wave has the input before any of them stores; a wave
+    // without a tile of this layer has not waited for it)
+    if (!input_read) o << "    wait_vmem();\n";
+    input_read = true;
     begin_next();
     o << "    exchange_barrier();\n";
     o << "    auto " << nv << " = " << (half ? "split_get_h<" : "split_get<") << tiles(n) << (half ? ", E" : "") << ", "
@@ -880,6 +885,7 @@ std::string fused_source_once(ponni_plan_s const& p, FusedConfig& cfg, bool allo
         o << (dense_hook.empty() ? "    });\n" : dense_hook);
         dense_hook.clear();
         if (cfg.split && &op == &p.ops.back()) {
+          if (!input_read) o << "    wait_vmem();\n    exchange_barrier();\n";
           if (half)
             o << "    split_store_h<" << n << ", " << tiles(n) << ", " << SW << ", " << (pad_ok ? "false" : "true") << ">("
               << own << ", y, ldy, wv, L);\n";

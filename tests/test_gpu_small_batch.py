@@ -231,3 +231,29 @@ def test_one_tile_per_simd_costs_what_fewer_do(cuda):
         us[B] = min(runs)
     print(f"one tile per SIMD: {us[32_768]:.1f} us, every other SIMD {us[16_384]:.1f}", flush=True)
     assert us[32_768] < 1.3 * us[16_384]
+
+
+@pytest.mark.parametrize("dtype", ["f32", "f16", "f64"])
+@pytest.mark.parametrize("chain", ["one", "three_tiles"])
+def test_small_batch_kernel_in_place(cuda, chain, dtype):
+    """y on x's own rows: every wave of a workgroup reads the columns that they
+    all store.  One contraction (no exchange between the reads and the
+    stores), and a first layer of three tiles, which leaves one of the four
+    waves without one."""
+    import torch
+
+    r = np.random.default_rng(82)
+    layers = {"one": lambda: [P.Matvec(_w(r, 100, 90)), P.Tanh(90)],
+              "three_tiles": lambda: [P.Save_State(0, 48), P.Matvec(_w(r, 48, 48)), P.Relu(48),
+                                      P.Binop_Projection_Add(0, _w(r, 48, 48), r.uniform(-0.1, 0.1, 48))]}[chain]()
+    m = P.create_inference_model(*layers, dtype=dtype, path="fused")
+    n_in, n_out = m.get_num_inputs(), m.get_num_outputs()
+    for B in (16, 515, 4_096):
+        assert m.call_form(B) == "small"
+        print(f"in place: chain={chain} dtype={dtype} B={B}", flush=True)
+        x = torch.randn((n_in, B), device="cuda:0", generator=torch.Generator("cuda:0").manual_seed(B))
+        x = x.to(getattr(torch, TORCH_DT[dtype]))
+        want = m.forward_batch_parallel(x)
+        m.forward_batch_parallel(x, x[:n_out])
+        torch.cuda.synchronize()
+        assert torch.equal(x[:n_out], want)
