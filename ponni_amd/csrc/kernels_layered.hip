@@ -396,13 +396,24 @@ hipError_t launch(DenseArgs const& a, hipStream_t stream) {
   return hipGetLastError();
 }
 
+// Do the op's input and output rows share memory?
+bool overlap(DenseArgs const& a, size_t es) {
+  auto const x = reinterpret_cast<uint64_t>(a.x), y = reinterpret_cast<uint64_t>(a.y);
+  uint64_t const x_end = x + (uint64_t(a.n_in - 1) * a.ldx + a.batch) * es;
+  uint64_t const y_end = y + (uint64_t(a.n_out - 1) * a.ldy + a.batch) * es;
+  return x < y_end && y < x_end;
+}
+
 // The large tile where it fills the 256 CUs, two workgroups each; otherwise
-// the small one, four times as many workgroups.
+// the small one, four times as many workgroups.  An op whose output takes its
+// input's place (a chain of one, called in place) has all its outputs in one
+// workgroup's tile if either tile holds them: it reads its columns before it stores.
 template <class S, int MI, int NJ, int MS, int NS>
 hipError_t launch_sized(DenseArgs const& a, hipStream_t stream) {
   int64_t const large = (a.batch + 32 * NJ - 1) / (32 * NJ) * ((a.n_out + 32 * MI - 1) / (32 * MI));
   bool const fits = a.n_out <= 32 * MS;  // (the large tile would be half empty)
-  return large >= 512 && !fits ? launch<S, MI, NJ>(a, stream) : launch<S, MS, NS>(a, stream);
+  bool const whole = !fits && a.n_out <= 32 * MI && overlap(a, sizeof(S));
+  return (large >= 512 && !fits) || whole ? launch<S, MI, NJ>(a, stream) : launch<S, MS, NS>(a, stream);
 }
 
 }  // namespace

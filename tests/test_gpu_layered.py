@@ -12,7 +12,7 @@ import pytest
 import oracle
 import ponni_amd as P
 from ponni_amd import graph as G
-from tests.test_gpu_parity import ORACLE_MODE, check_f32, check_half, check_non_finite, gpu_run
+from tests.test_gpu_parity import ORACLE_MODE, TORCH_DT, check_f32, check_half, check_non_finite, gpu_run
 from tests.test_graph import lowered_with_params
 
 pytestmark = pytest.mark.gpu
@@ -78,3 +78,22 @@ def test_layered_infinite_inputs(cuda, n_in, dtype):
         want = oracle.forward(layers, xg, ORACLE_MODE[dtype])
         assert np.isfinite(want[:, 0:400:2]).mean() > 0.5
         check_non_finite(got, want, dtype)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "f16", "f64"])
+@pytest.mark.parametrize("n_out", [64, 65, 128])
+def test_layered_one_layer_in_place(cuda, n_out, dtype):
+    """A chain of one layer whose outputs take its inputs' rows: the outputs of a
+    column, read by every workgroup that computes one of them, stay in one."""
+    import torch
+
+    r = np.random.default_rng(n_out)
+    m = P.create_inference_model(P.Matvec(_w(r, 200, n_out)), P.Relu(n_out), dtype=dtype, path="layered")
+    for B in (130, 2_000):
+        print(f"layered in place: n_out={n_out} dtype={dtype} B={B}", flush=True)
+        x = torch.randn((200, B), device="cuda:0", generator=torch.Generator("cuda:0").manual_seed(B))
+        x = x.to(getattr(torch, TORCH_DT[dtype]))
+        want = m.forward_batch_parallel(x)
+        m.forward_batch_parallel(x, x[:n_out])
+        torch.cuda.synchronize()
+        assert torch.equal(x[:n_out], want)
