@@ -99,22 +99,55 @@ __device__ inline void workgroup_barrier() {
 // rows at any alignment).
 enum InputMode { IN_VEC = 0, IN_DWORD = 1, IN_ELEMENT = 2 };
 
-// tanh of fp32 plans.  The hardware form 1 - 2 / (1 + e^2x) is off by up to an
-// ulp of one, which near zero is not an ulp of the result: there, x p(x^2)
-// with p a Chebyshev fit of tanh(x) / x (1e-9 on |x| <= 0.55).
-__device__ inline float tanh_f32(float x) {
-  float const t = x * x;
-  float q = fmaf(t, -0.00623885f, 0.02104217f);
-  q = fmaf(t, q, -0.05384337f);
-  q = fmaf(t, q, 0.13332468f);
-  q = fmaf(t, q, -0.33333311f);
-  return __builtin_fabsf(x) <= 0.55f ? fmaf(x * t, q, x) : act_tanh_fast(x);
+// The usual activations of fp32 plans on the accumulators.  The hardware forms
+// of the generated kernels (pointwise.h) are off by up to an ulp of one near
+// zero (tanh) and by |x| / 2 ulp (sigmoid and SiLU of negative x), which libm's
+// (GENERIC's) are not: largest relative errors, libm / hardware forms / these,
+// tanh on -2..-0.55 1.5e-7 / 3.5e-7 / 2.0e-7, sigmoid on -40..-12 1.8e-7 /
+// 1.9e-6 / 2.0e-7.  64-1024-1024-64 tanh, 65,536 columns: 1302 us with the
+// hardware forms, 1307 with these, 1325 with libm's; 40-700-30 sigmoid 129, 132, 170.
+// e^v: 2^(v log2 e) with the rounding error of the product carried along.
+__device__ inline float exp_f32(float v) {
+  constexpr float kLog2eRest = 1.9259630e-8f, kLn2 = 0.69314718f;
+  float const t = v * kLog2e;
+  float const rest = fmaf(v, kLog2eRest, fmaf(v, kLog2e, -t));
+  float const e = __builtin_amdgcn_exp2f(t);
+  return __builtin_fabsf(t) < 128.0f ? fmaf(e, rest * kLn2, e) : e;
 }
+// x / (1 + e): the hardware's reciprocal and one correction of the quotient.
+__device__ inline float over_one_plus(float x, float e) {
+  float const d = 1.0f + e, r = __builtin_amdgcn_rcpf(d), q = x * r;
+  return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-d, q, x), r, q), d, x);
+}
+__device__ inline float sigmoid_f32(float x) { return over_one_plus(1.0f, exp_f32(-x)); }
+__device__ inline float silu_f32(float x) { return over_one_plus(x, exp_f32(-x)); }
+// ponni_Gelu.h:48-53: x sigmoid(2u), u = sqrt(2/pi) (x + 0.044715 x^3)
+__device__ inline float gelu_tanh_f32(float x) {
+  constexpr float c = -2.0f * 0.79788456080286535588f;
+  return over_one_plus(x, exp_f32(x * fmaf(0.044715f * c, x * x, c)));
+}
+// 1 - 2 e / (1 + e) of |x|, e = e^(-2|x|); near zero, where that cancels, x p(x^2)
+// with p a Chebyshev fit of tanh(x) / x (4.5e-9 on |x| <= 0.55).
+__device__ inline float tanh_f32(float x) {
+  float const s = x * x;
+  float q = fmaf(s, -0.00623885f, 0.02104217f);
+  q = fmaf(s, q, -0.05384337f);
+  q = fmaf(s, q, 0.13332468f);
+  q = fmaf(s, q, -0.33333311f);
+  float const a = __builtin_fabsf(x);
+  float const e = __builtin_amdgcn_exp2f(-2.0f * kLog2e * a);
+  float const r = a <= 0.55f ? fmaf(a * s, q, a) : 1.0f + over_one_plus(-2.0f * e, e);
+  return __builtin_copysignf(r, x);
+}
+// 16-bit plans: the hardware form, and x itself where that is closer than the
+// type resolves (below 2^-7 tanh(x) is x to 2e-5; the form's error there is an
+// ulp of fp32's one, more than an ulp of a small fp16 result).  fp16
+// 24-1100-200, 40,000 columns: 84 us without, 87 with.
+__device__ inline float tanh_half(float x) { return __builtin_fabsf(x) < 0.0078125f ? x : act_tanh_fast(x); }
 
 // The epilogue steps that run on the accumulators: each(f) for one of them,
-// false for any other.  fp32 and 16-bit plans take the logistic family's
-// hardware forms, as the generated kernels do (pointwise.h); fp64 keeps
-// libm's, whose code for every accumulator at once is too long.
+// false for any other.  fp64 keeps libm's, whose code for every accumulator at
+// once is too long.
 template <class C, bool Precise, class Each>
 __device__ inline bool usual_step(Step const& st, Each&& each) {
   C const a = C(st.a);
@@ -125,13 +158,10 @@ __device__ inline bool usual_step(Step const& st, Each&& each) {
   }
   if constexpr (sizeof(C) == 4) {
     switch (st.act) {
-      case ACT_TANH:
-        if constexpr (Precise) each([](C v) { return tanh_f32(v); });
-        else each([](C v) { return act_tanh_fast(v); });
-        return true;
-      case ACT_SIGMOID: each([](C v) { return act_sigmoid_fast(v); }); return true;
-      case ACT_SILU: each([](C v) { return act_silu_fast(v); }); return true;
-      case ACT_GELU_TANH: each([](C v) { return act_gelu_tanh_fast(v); }); return true;
+      case ACT_TANH: each([](C v) { return Precise ? tanh_f32(v) : tanh_half(v); }); return true;
+      case ACT_SIGMOID: each([](C v) { return Precise ? sigmoid_f32(v) : act_sigmoid_fast(v); }); return true;
+      case ACT_SILU: each([](C v) { return Precise ? silu_f32(v) : act_silu_fast(v); }); return true;
+      case ACT_GELU_TANH: each([](C v) { return Precise ? gelu_tanh_f32(v) : act_gelu_tanh_fast(v); }); return true;
       default: break;
     }
   }

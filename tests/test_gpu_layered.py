@@ -97,3 +97,48 @@ def test_layered_one_layer_in_place(cuda, n_out, dtype):
         m.forward_batch_parallel(x, x[:n_out])
         torch.cuda.synchronize()
         assert torch.equal(x[:n_out], want)
+
+
+# (largest relative error in fp32 ulps of 2^-24: 1 + e and the quotient round to
+# 1, 2^x is off by 1 or 2 and, carried along, its argument by a half, and tanh's last
+# addition rounds to a half of at least 0.5; the hardware forms alone: 5.8, 31, 63)
+FP32_BOUNDS = [("tanh", 1e-6, 0.55, 2), ("tanh", -2.0, -0.55, 4.5), ("tanh", -8.0, -2.0, 2), ("sigmoid", -40.0, -6.0, 5),
+               ("silu", -80.0, -40.0, 6), ("sigmoid", -3.0, 9.0, 5), ("silu", -6.0, 9.0, 6), ("gelu", -0.5, 6.0, 6)]
+
+
+def _activation_error(cuda, dtype, act, lo, hi):
+    """y, the exact value and x of one activation on both signs or as given,
+    through an identity layer (exact in any order of its sum)."""
+    import torch
+
+    n = 64
+    layer = {"tanh": P.Tanh(n), "sigmoid": P.Sigmoid(n), "silu": P.Silu(n), "gelu": P.Gelu(n, True)}[act]
+    m = P.create_inference_model(P.Matvec(np.eye(n)), layer, dtype=dtype, path="layered")
+    gen = torch.Generator("cuda:0").manual_seed(5)
+    x = torch.rand((n, 20_000), device="cuda:0", dtype=torch.float64, generator=gen) * (hi - lo) + lo
+    x = x.to(getattr(torch, TORCH_DT[dtype]))
+    y = m.forward_batch_parallel(x).double()
+    v = x.double()
+    u = 2 * np.sqrt(2 / np.pi) * (v + 0.044715 * v**3)
+    want = {"tanh": torch.tanh, "sigmoid": lambda v: 1 / (1 + torch.exp(-v)), "silu": lambda v: v / (1 + torch.exp(-v)),
+            "gelu": lambda v: v / (1 + torch.exp(-u))}[act](v)
+    return y, want
+
+
+@pytest.mark.parametrize("act, lo, hi, ulps", FP32_BOUNDS)
+def test_layered_fp32_activations(cuda, act, lo, hi, ulps):
+    y, want = _activation_error(cuda, "f32", act, lo, hi)
+    assert float(((y - want).abs() / want.abs()).max()) * 2**24 <= ulps
+
+
+@pytest.mark.parametrize("dtype, digits, smallest", [("f16", 10, -14), ("bf16", 7, -126)])
+@pytest.mark.parametrize("lo, hi", [(1e-7, 1e-5), (1e-5, 1e-4), (1e-4, 1e-3), (1e-3, 0.1), (-2.0, 2.0)])
+def test_layered_half_tanh_near_zero(cuda, lo, hi, dtype, digits, smallest):
+    """Half an ulp of the type, and a sixteenth for fp32's own error (x for
+    tanh(x) below 2^-7: a third of x^2, 1/25 of an fp16 ulp; above, an fp32 ulp of
+    one: 1/30 of one).  The hardware form alone was off by 2 ulps at 1e-4."""
+    import torch
+
+    y, want = _activation_error(cuda, dtype, "tanh", lo, hi)
+    ulp = torch.exp2(torch.floor(torch.log2(want.abs())).clamp_min(smallest) - digits)
+    assert float(((y - want).abs() / ulp).max()) <= 0.5 + 1 / 16
