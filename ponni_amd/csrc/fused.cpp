@@ -1525,6 +1525,8 @@ int load_module(std::string const& key, std::vector<char> const& code, std::stri
     if (e == hipSuccess) e = hipModuleGetFunction(&m->fn, m->module, name.c_str());
     if (e == hipSuccess) e = hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&m->blocks_per_cu, m->fn, threads, 0);
     if (e != hipSuccess) {
+      (void)hipGetLastError();  // (reported here, not by the next launch)
+      if (m->module != nullptr) (void)hipModuleUnload(m->module);
       error = std::string("loading the fused kernel failed: ") + hipGetErrorString(e);
       return PONNI_ERR_DEVICE;
     }
@@ -1675,13 +1677,14 @@ static bool fused_wants_split(ponni_plan_s const& p, int64_t batch, bool io32) {
 
 FusedForm fused_wanted_form(ponni_plan_s const& p, void const* x, int64_t ld_in, int64_t batch, bool io32) {
   if (p.path != PONNI_PATH_FUSED) return FUSED_MAIN;
-  if (fused_wants_split(p, batch, io32)) return FUSED_SMALL;
+  FusedKernel const* const forms = p.kernels[io32];
+  if (fused_wants_split(p, batch, io32) && !forms[FUSED_SMALL].unavailable()) return FUSED_SMALL;
   // Rows that do not start on 16 bytes, where aligned ones go through LDS a
   // tile ahead: element loads instead took half again the time (fp16
   // 64-256-256-256-64, 262,145 columns: 166 us, aligned 110).
   int const es = io32 ? 4 : 2;
   bool const aligned = ((reinterpret_cast<uint64_t>(x) | uint64_t(ld_in) * es) & 15) == 0;
-  return p.kernels[io32][FUSED_MAIN].rows_in_lds && !aligned ? FUSED_ANY_ROWS : FUSED_MAIN;
+  return forms[FUSED_MAIN].rows_in_lds && !aligned && !forms[FUSED_ANY_ROWS].unavailable() ? FUSED_ANY_ROWS : FUSED_MAIN;
 }
 
 int fused_call_form(ponni_plan_s& p, int64_t batch, int row_alignment, bool io32, FusedForm& form, std::string& error) {
@@ -1697,16 +1700,26 @@ int fused_call_form(ponni_plan_s& p, int64_t batch, int row_alignment, bool io32
     p.small_batch = small_batch_rule(p, cfg, code);
     if (p.fused_cus == 0) p.fused_cus = kChipCus;
   }
-  for (FusedForm f : {FUSED_MAIN, FUSED_SMALL}) {
+  auto compile_form = [&](FusedForm f) -> int {
     FusedKernel& k = p.kernels[io32][f];
-    if (k.loaded() || (f == FUSED_SMALL && !fused_wants_split(p, batch, io32))) continue;
+    if (k.loaded() || k.unavailable()) return PONNI_OK;
     FusedConfig cfg = form_config(io32, f);
     int const st = compile_cached(p, cfg, key, code, error);
     if (st != PONNI_OK) return st;
     (void)fused_source(p, cfg);
     k.describe(fused_kernel(cfg, code));
+    return PONNI_OK;
+  };
+  int const st = compile_form(FUSED_MAIN);
+  if (st != PONNI_OK) return st;
+  auto wanted = [&] {
+    return fused_wanted_form(p, reinterpret_cast<void const*>(uint64_t(row_alignment)), 0, batch, io32);
+  };
+  // (one that does not compile gives way to the main one, as in ponni_forward)
+  for (form = wanted(); form != FUSED_MAIN; form = wanted()) {
+    if (compile_form(form) != PONNI_OK) p.kernels[io32][form].give_up();
+    else if (wanted() == form) break;
   }
-  form = fused_wanted_form(p, reinterpret_cast<void const*>(uint64_t(row_alignment)), 0, batch, io32);
   return PONNI_OK;
 }
 

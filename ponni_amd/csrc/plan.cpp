@@ -1468,9 +1468,11 @@ int forward_impl(ponni_plan plan, const void* x, int64_t ld_in, void* y, int64_t
     if (dev != plan->device) return fail(PONNI_ERR_DEVICE, "plan was first used on another device");
   }
   // The kernels of this call that are not loaded yet.  (A captured stream
-  // cannot load a module: a plan whose form for this call is not there yet
-  // then runs its main kernel, which takes any call.)
+  // cannot load a module: a plan whose form for this call is not there yet, or
+  // cannot be built, then runs its main kernel, which takes any call.)
   bool const need_rows = io32 && !plan->kernels[1][FUSED_MAIN].loaded();
+  if (need_rows && plan->kernels[1][FUSED_MAIN].unavailable())
+    return fail(PONNI_ERR_UNSUPPORTED, "fp32 rows: the kernel could not be built");
   FusedForm const form = no_alloc ? FUSED_MAIN : fused_wanted_form(*plan, x, ld_in, batch, io32);
   bool const generated = plan->path == PONNI_PATH_FUSED || plan->narrow_jit;
   if (generated && (need_rows || !plan->kernels[io32][form].loaded())) {
@@ -1480,15 +1482,13 @@ int forward_impl(ponni_plan plan, const void* x, int64_t ld_in, void* y, int64_t
     if (need_rows && !can_load)
       return fail(PONNI_ERR_UNSUPPORTED, "fp32 rows: the kernel is not loaded yet, and the stream is being captured");
     std::string error;
-    if (need_rows) {
-      int const st = fused_prepare(*plan, true, FUSED_MAIN, error);
-      if (st != PONNI_OK) return fail(st, error);
+    if (need_rows && fused_prepare(*plan, true, FUSED_MAIN, error) != PONNI_OK) {
+      plan->kernels[1][FUSED_MAIN].give_up();
+      return fail(PONNI_ERR_UNSUPPORTED, "fp32 rows: " + error);
     }
     FusedForm const wanted = fused_wanted_form(*plan, x, ld_in, batch, io32);
-    if (!plan->kernels[io32][wanted].loaded() && can_load) {
-      int const st = fused_prepare(*plan, io32, wanted, error);
-      if (st != PONNI_OK) return fail(st, error);
-    }
+    if (!plan->kernels[io32][wanted].loaded() && can_load && fused_prepare(*plan, io32, wanted, error) != PONNI_OK)
+      plan->kernels[io32][wanted].give_up();
   }
   void* scratch[3] = {};  // tmp1, tmp2, the saved-slot area
   int64_t scratch_ld = 0;

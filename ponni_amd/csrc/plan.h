@@ -67,10 +67,15 @@ struct FusedKernel {
   bool rows_in_lds = false;  // its input rows go through LDS a tile ahead
   int wave_columns = 0;  // columns of a tile where tiles go to waves (0: to workgroups)
   int spills = 0;        // registers spilled (read by other threads at any time)
+  bool failed = false;
 
   // A form may be loaded by one thread's forward pass while others launch:
   // the other members hold once loaded() is true.
   bool loaded() const { return __atomic_load_n(&fn, __ATOMIC_ACQUIRE) != nullptr; }
+  // A form that could not be built or loaded is not tried again: its calls run
+  // on the main kernel.
+  bool unavailable() const { return __atomic_load_n(&failed, __ATOMIC_RELAXED); }
+  void give_up() { __atomic_store_n(&failed, true, __ATOMIC_RELAXED); }
   void describe(FusedKernel const& k) {
     columns_per_block = k.columns_per_block;
     waves = k.waves;

@@ -257,3 +257,54 @@ def test_small_batch_kernel_in_place(cuda, chain, dtype):
         m.forward_batch_parallel(x, x[:n_out])
         torch.cuda.synchronize()
         assert torch.equal(x[:n_out], want)
+
+
+_COMPILE_FORMS = """
+import sys
+import torch  # (its code generator, as in the process that uses the cache)
+import numpy as np
+import ponni_amd as P
+r = np.random.default_rng(1)
+m = P.create_inference_model(P.Matvec(r.uniform(-1, 1, (37, 75))), P.Tanh(75), P.Matvec(r.uniform(-1, 1, (75, 11))),
+                             dtype="f16", path="fused")
+print(m.call_form(64), m.call_form(300_001, 2), m.call_form(300_000, fp32_rows=True))
+"""
+
+
+def test_a_form_that_cannot_be_loaded_gives_way(cuda, tmp_path, monkeypatch):
+    """A code cache whose objects for the small-batch and misaligned-row forms
+    hold another kernel (here the main one's): those calls run on the main
+    kernel, every time; fp32 rows are refused and infer_batch_half2's caller
+    converts, as for a plan without that kernel."""
+    import os
+    import shutil
+    import subprocess
+    import sys
+
+    import torch
+
+    monkeypatch.setenv("PONNI_JIT_CACHE", str(tmp_path))
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    out = subprocess.run([sys.executable, "-c", _COMPILE_FORMS], cwd=root, capture_output=True, text=True, timeout=100,
+                         env={**os.environ, "HIP_VISIBLE_DEVICES": "-1"})
+    assert out.stdout.split() == ["small", "any_rows", "main"], out.stdout + out.stderr
+    objects = {f: f.read_bytes() for f in tmp_path.iterdir() if f.suffix == ".co"}
+    others = [f for f, code in objects.items() if any(s in code for s in (b"_split", b"_any", b"_io32"))]
+    main = next(f for f in objects if f not in others)
+    assert len(others) >= 3
+    for f in others:
+        shutil.copyfile(main, f)
+    r = np.random.default_rng(1)
+    layers = [P.Matvec(r.uniform(-1, 1, (37, 75))), P.Tanh(75), P.Matvec(r.uniform(-1, 1, (75, 11)))]
+    m = P.create_inference_model(*layers, dtype="f16", path="fused")
+    for B in (64, 300_001, 64):
+        x = torch.randn((37, B), device="cuda:0", generator=torch.Generator("cuda:0").manual_seed(B)).half()
+        y = m.forward_batch_parallel(x)
+        torch.cuda.synchronize()
+        assert torch.cuda.current_stream().query()
+        check_half(y[:, :64].double().cpu().numpy(),
+                   oracle.forward(layers, x[:, :64].double().cpu().numpy(), oracle.MODE_F16_OPERANDS))
+        assert m.call_form(B, 2 if B % 8 else 16) == "main"
+    x = torch.randn((37, 4096), device="cuda:0")
+    for _ in range(2):
+        assert not m.forward_fp32_rows(x, torch.empty((11, 4096), device="cuda:0"))
