@@ -353,8 +353,9 @@ int ponni_forward(ponni_plan plan, const void* x, int64_t ld_in, void* y,
  * what converting the arrays around ponni_forward gives, without the passes
  * over memory (the generated infer_batch_half2 on Scalar views,
  * kokkos_nn/emitter.py:1551-1573).  FUSED and generated NARROW plans; others,
- * and a plan whose kernel for it would have to be loaded while the stream is
- * captured, give PONNI_ERR_UNSUPPORTED.  x and y must not overlap. */
+ * and a plan whose kernel for it cannot be built or would have to be loaded
+ * while the stream is captured, give PONNI_ERR_UNSUPPORTED.  x and y must not
+ * overlap. */
 int ponni_forward_fp32_rows(ponni_plan plan, const float* x, int64_t ld_in, float* y,
                             int64_t ld_out, int64_t batch, hipStream_t stream);
 
@@ -424,13 +425,18 @@ int64_t ponni_plan_kernel_source(ponni_plan plan, char* buf, int64_t len);
  * or -1 (other dtypes). */
 int64_t ponni_plan_program_source(ponni_plan plan, char* buf, int64_t len);
 
-/* Compile a FUSED plan's kernel with hipRTC now (no device needed; the result
- * is cached in-process and under $PONNI_JIT_CACHE or ~/.cache/ponni_hip) so the
- * first ponni_forward does not pay for it.  A no-op for the other paths.
- * A FUSED plan's second kernel, for batches too small to fill the chip with
- * the first, is compiled (and cached alike) by the first ponni_forward of
- * such a batch on a stream that is not being captured; until then, and in
- * ponni_forward_no_alloc, every batch runs on the first kernel.
+/* Compile a FUSED plan's main kernel with hipRTC now (no device needed; the
+ * result is cached in-process and under $PONNI_JIT_CACHE or ~/.cache/ponni_hip)
+ * so the first ponni_forward does not pay for it.  A no-op for the other paths.
+ * The plan's other forms of it -- for batches too small to fill the chip, for
+ * 16-bit rows that do not start on 16 bytes, and each of these and the main one
+ * for ponni_forward_fp32_rows -- are compiled (and cached alike) and loaded by
+ * the first ponni_forward that runs on them, on a stream that is not being
+ * captured; ponni_plan_call_form compiles the one for a given call ahead of
+ * it.  Where a form is not loaded (in ponni_forward_no_alloc and captured calls
+ * with no ordinary call of the kind before them) or cannot be built, calls
+ * run on the main kernel, which takes any of them, and
+ * ponni_forward_fp32_rows gives PONNI_ERR_UNSUPPORTED.
  * Stands in for the compile step of building a reference model, which
  * happens when the application is compiled. */
 int ponni_plan_compile(ponni_plan plan);
@@ -450,8 +456,8 @@ int ponni_plan_kernel_config(ponni_plan plan, int32_t* threads, int32_t* columns
 /* The form of a FUSED plan's generated kernel that ponni_forward runs a batch
  * on, of rows whose starts are multiples of row_alignment bytes (fp32_rows:
  * ponni_forward_fp32_rows): 0 the main one, 1 the one for small batches, 2 the
- * one for 16-bit rows that do not start on 16 bytes.  Compiles what the answer
- * depends on; no device required. */
+ * one for 16-bit rows that do not start on 16 bytes.  Compiles that form, and
+ * what the answer depends on; no device required. */
 int ponni_plan_call_form(ponni_plan plan, int64_t batch, int32_t row_alignment,
                          int32_t fp32_rows, int32_t* form);
 
