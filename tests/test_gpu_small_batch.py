@@ -78,6 +78,7 @@ def test_small_batch_and_main_kernels(cuda, chain, dtype):
     A.check(A.lib().ponni_plan_device_params(main._plan, ctypes.byref(ctypes.c_void_p())))
     n_in, n_out = small.get_num_inputs(), small.get_num_outputs()
     for B, pad in [(1, 0), (16, 3), (33, 0), (64, 8), (515, 0)]:
+        assert small.call_form(B) == "small"
         x = np.random.default_rng(B).standard_normal((n_in, B))
         xs = torch.zeros((n_in, B + pad), dtype=tdt, device="cuda:0")
         xs[:, :B] = torch.from_numpy(x).to(tdt)
@@ -153,6 +154,8 @@ def test_half_rows_at_any_alignment_through_lds(cuda, chain, dtype):
         ys = torch.full((n_out, off + B + pad), float("nan"), dtype=tdt, device="cuda:0")
         m.forward_batch_parallel(xs[:, off:off + B], ys[:, off:off + B])
         torch.cuda.synchronize()
+        aligned = ((xs.data_ptr() + 2 * off) | (2 * xs.stride(0))) % 16 == 0
+        assert m.call_form(B, 16 if aligned else 2) == ("main" if aligned else "any_rows")
         assert torch.isnan(ys[:, :off].float()).all() and torch.isnan(ys[:, off + B:].float()).all()
         got = ys[:, off:off + B].double().cpu().numpy()
         assert np.isfinite(got).all()
@@ -308,3 +311,24 @@ def test_a_form_that_cannot_be_loaded_gives_way(cuda, tmp_path, monkeypatch):
     x = torch.randn((37, 4096), device="cuda:0")
     for _ in range(2):
         assert not m.forward_fp32_rows(x, torch.empty((11, 4096), device="cuda:0"))
+
+
+@pytest.mark.parametrize("chain", ["wide", "spilling"])
+def test_small_batch_kernel_at_large_batches(cuda, chain):
+    """Plans that run the small-batch kernel at every batch (fp32, wider than 448
+    features, or spilling on the main kernel), with thousands of workgroups and
+    a ragged last one: sampled columns, both ends among them, against the oracle."""
+    import torch
+
+    r = np.random.default_rng(83)
+    layers = _mlp(r, [20, 464, 464, 60], P.Relu) if chain == "wide" else _residual(r, 12, 245, 35, 2)
+    m = P.create_inference_model(*layers, dtype="f32", path="fused")
+    B = 150_001
+    assert m.call_form(B) == "small"
+    pick = np.concatenate([np.arange(40), np.random.default_rng(6).integers(40, B - 40, 400), np.arange(B - 40, B)])
+    x = torch.randn((m.get_num_inputs(), B), device="cuda:0", generator=torch.Generator("cuda:0").manual_seed(7))
+    ys = torch.full((m.get_num_outputs(), B + 3), float("nan"), device="cuda:0")
+    m.forward_batch_parallel(x, ys[:, :B])
+    torch.cuda.synchronize()
+    assert torch.isnan(ys[:, B:]).all() and torch.isfinite(ys[:, :B]).all()
+    check_f32(ys[:, pick].double().cpu().numpy(), oracle.forward(layers, x[:, pick].double().cpu().numpy()))
