@@ -509,6 +509,7 @@ std::string fused_source_once(ponni_plan_s const& p, FusedConfig& cfg, bool allo
 
   if (dbl) o << "#define PONNI_REAL double\n";
   if (NT != 2) o << "#define PONNI_NT " << NT << "\n";
+  if (!half && !cfg.split && NT == 1) o << "#define PONNI_GELU_TERMS\n";
   // One column tile per wave at two waves per SIMD: A fragments read two
   // steps ahead (fused_f16.h kFragPipe; 64x512x512x64 3.28 against 3.38 ms,
   // 320 / 384 features 5-7 % faster; at one wave per SIMD, and with two

@@ -292,11 +292,19 @@ __device__ inline float act_tanh_fast(float x) {
 // u = sqrt(2/pi) (x + 0.044715 x^3).  The exponent -2u log2 e as x (c + 0.044715 c x^2):
 // 5 VALU operations and the two transcendentals, 3 fewer than term by term,
 // which is what bounds 16-bit models with GELU (fp32 models: it adds to the
-// MFMA time).
+// MFMA time).  fp32 kernels with one column tile per wave, which stream their
+// weights through the compiler's own schedule, keep the terms (PONNI_GELU_TERMS,
+// fused.cpp): 25-308-14 residual chain of three blocks, 131,072 columns, 1685 us
+// with them, 2909 with the polynomial; 61-338-34 4970 against 5238.
 __device__ inline float act_gelu_tanh_fast(float x) {
+#ifdef PONNI_GELU_TERMS
+  float const u = 0.79788456080286535588f * (x + 0.044715f * (x * x * x));
+  return x * fast_sigmoid(2.0f * u);
+#else
   constexpr float c = -2.0f * 0.79788456080286535588f * kLog2e;
   float const p = fmaf(0.044715f * c, x * x, c);
   return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x * p));
+#endif
 }
 
 }  // namespace ponni_hip

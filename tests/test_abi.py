@@ -324,6 +324,14 @@ def test_small_batch_kernel_within_a_launch(dtype, widths):
     assert [m.call_form(B) for B in (2**28, 2**31 - 1)] == ["main", "main"]
 
 
+def test_gelu_by_terms_in_wide_fp32_kernels():
+    """fp32 kernels with one column tile per wave keep GELU's exponent term by
+    term: the polynomial cost some of them 1.7 times the time."""
+    wide, tiles, half = (create(_residual_chain(25, w, 14, 1), dtype=d, path="fused").kernel_source()
+                         for w, d in ((308, "f32"), (128, "f32"), (308, "f16")))
+    assert "#define PONNI_GELU_TERMS" in wide and "PONNI_GELU_TERMS" not in tiles + half
+
+
 _COMPILE_C2 = """
 import sys
 if sys.argv[1] == "torch":
