@@ -307,7 +307,12 @@ std::string fused_source_once(ponni_plan_s const& p, FusedConfig& cfg, bool allo
 // (fp16 64-256-256-256-64, 21,600 columns: 15.5 against 22.6 us), unless they
 // hold operations that every wave repeats (256-wide with LayerNorm: 47.6 us
 // with one tile, 47.8 with two, and 26.4 against 31.1 at 10,000); beyond 512
-// features with eight waves (1024: 86 against 141 us).
+// features with eight waves (1024: 86 against 141 us).  Where the line lies, one
+// against two column tiles, fp16 40-w-w-w-24 tanh, us at 4,096 / 21,600 columns:
+// w = 144 4.5 / 11.4 against 5.4 / 8.7, 176 4.9 / 13.0 against 5.8 / 9.9, 192 4.8 /
+// 13.3 against 5.9 / 9.5, 256 6.7 / 20.6 against 7.3 / 13.4: two are better from
+// about 10,000 columns on at every width, where up to 176 features the main
+// kernel, its fragments resident, is the one that runs (bf16 12-159-159-159-23 10 us).
 void split_shape(ponni_plan_s const& p, FusedConfig& cfg) {
   bool const half = p.dtype == PONNI_F16 || p.dtype == PONNI_BF16;
   bool repeated = false;

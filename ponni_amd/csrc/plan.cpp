@@ -1173,7 +1173,10 @@ int ponni_plan_create(const ponni_layer_desc* layers, int32_t num_layers, int32_
     // (each side beyond 8 features: measured GENERIC against LAYERED at 100 /
     // 65,536 columns, us, tanh between the layers: fp32 9-600-9 1478 / 2352
     // against 28 / 104, 63-600-63 7858 / 14361 against 27 / 140; fp64 9-300-9
-    // 917 / 1334 against 27 / 206; fp16 9-1100-9 2695 / 4064 against 21 / 94)
+    // 917 / 1334 against 27 / 206; fp16 9-1100-9 2695 / 4064 against 21 / 94.
+    // 8 features and fewer keep GENERIC, which measured slower there as well:
+    // fp32 8-600-8 1367 / 2119 against 25 / 102, 1-600-1 746 / 809 against
+    // 28 / 100; fp64 1-300-1 494 / 552 against 27 / 201)
     layered_pays = layered_pays || (is_dense(layers[i].kind) && std::min(layers[i].n_in, layers[i].n_out) > 8 &&
                                     int64_t(layers[i].n_in) * layers[i].n_out >= 2048);
   int chosen = path;
