@@ -194,6 +194,8 @@ def test_half2_on_fp32_rows_is_the_converted_call(cuda, shape):
         x = xs[:, off:off + B]
         ys = torch.full((gm.num_outputs, B + pad + off), float("nan"), device="cuda:0")
         y = ys[:, off:off + B]
+        assert plan.forward_fp32_rows(x, y)  # (not left to the conversion)
+        y.fill_(float("nan"))
         gm.infer_batch_half2(x, y)
         want = plan.forward_batch_parallel(x.to(torch.float16).contiguous()).float()
         torch.cuda.synchronize()
