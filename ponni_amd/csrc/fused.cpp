@@ -1585,10 +1585,10 @@ SmallBatchRule small_batch_rule(ponni_plan_s const& p, FusedConfig const& main, 
     r.step = r.block_columns;
     r.base = 0.2;
     r.slope = ratio * (!one_tile ? 1.25 : !repeated ? 1.2 : spills >= 200 ? 1.5 : 2.0);
-    r.spilled = ratio * 1.9;
   } else if (p.dtype == PONNI_F32 && one_tile && repeated) {
     r.slope = 1.5 * ratio;
   }
+  r.spilled = std::max(r.slope, 1.9 * ratio);
   // Where the main kernel is the slower one at every batch (131,072 columns,
   // TFLOP/s, main against small-batch): fp32 chains with two column tiles that
   // spill (12-245-35 residual, 179 registers, 41 against 92; 22-235-2, 13, 75

@@ -100,7 +100,7 @@ struct SmallBatchRule {
   int step = 0;                // its columns are taken in steps of so many per CU (0: as they are)
   int rounds = 0;              // of a batch for which it can be the faster one, at most
   bool always = false;         // the faster one at every batch
-  double spilled = 0;          // slope where it spills registers itself
+  double spilled = 0;          // slope of a 16-bit plan where it spills registers itself
 };
 
 // Kinds of packed parameter slots (plan.cpp visit_param_slots).
