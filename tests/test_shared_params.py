@@ -82,7 +82,8 @@ def test_share_rejections():
 
 
 CASES = [("generic", "f32", "c2"), ("narrow", "f32", "c1"), ("mfma", "f32", "c2"), ("fused", "f32", "c2"),
-         ("fused", "f16", "c2"), ("fused", "bf16", "c2"), ("fused", "f64", "c2"), ("generic", "f16", "c2")]
+         ("fused", "f16", "c2"), ("fused", "bf16", "c2"), ("fused", "f64", "c2"), ("generic", "f16", "c2"),
+         ("layered", "f32", "c2"), ("layered", "f16", "c2"), ("layered", "f64", "c2")]
 TORCH_DT = {"f32": "float32", "f16": "float16", "bf16": "bfloat16", "f64": "float64"}
 MODE = {"f32": oracle.MODE_F32, "f64": oracle.MODE_F64, "f16": oracle.MODE_F16_OPERANDS,
         "bf16": oracle.MODE_BF16_OPERANDS}

@@ -51,6 +51,31 @@ def test_no_alloc_matches_forward(cuda, path, layers):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["f32", "f16"])
+def test_no_alloc_layered_at_the_end_of_the_scratch(cuda, dtype):
+    """The largest batch whose state buffers fit the fixed scratch, not a
+    multiple of 16 columns: LAYERED's buffers, whose rows are otherwise whole
+    16-byte pieces, take the batch as their stride there."""
+    import torch
+
+    r = np.random.default_rng(5)
+    layers = [P.Matvec(r.uniform(-0.2, 0.2, (9, 1100))), P.Tanh(1100), P.Matvec(r.uniform(-0.05, 0.05, (1100, 9)))]
+    m = P.create_inference_model(*layers, dtype=dtype, path="layered")
+    es = 4 if dtype == "f32" else 2
+    B = (64 << 20) // (es * 1100)
+    assert B % 16 and es * 1100 * ((B + 15) // 16 * 16) > 64 << 20
+    x = torch.randn((9, B), device="cuda:0").to(torch.float32 if dtype == "f32" else torch.float16)
+    want = m.forward_batch_parallel(x)
+    y = torch.full_like(want, float("nan"))
+    stream = torch.cuda.current_stream().cuda_stream
+    A.check(call(A.lib().ponni_forward_no_alloc, m, x, y, B, stream))
+    torch.cuda.synchronize()
+    assert torch.equal(y, want)
+    big = torch.zeros((9, B + 1), device="cuda:0", dtype=x.dtype)
+    assert call(A.lib().ponni_forward_no_alloc, m, big, torch.empty_like(big), B + 1, stream) == A.PONNI_ERR_SHAPE
+
+
+@pytest.mark.gpu
 def test_no_alloc_rejects_a_batch_beyond_the_fixed_scratch(cuda):
     import torch
 
