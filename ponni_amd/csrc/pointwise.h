@@ -292,7 +292,9 @@ __device__ inline float act_tanh_fast(float x) {
 // u = sqrt(2/pi) (x + 0.044715 x^3).  The exponent -2u log2 e as x (c + 0.044715 c x^2):
 // 5 VALU operations and the two transcendentals, 3 fewer than term by term,
 // which is what bounds 16-bit models with GELU (fp32 models: it adds to the
-// MFMA time).  fp32 kernels with one column tile per wave, which stream their
+// MFMA time).  Its largest relative error is that of the terms or less on every
+// range of x (1.2e-5 against 1.4e-5 on -10..-6, 2.7e-7 against 3.3e-7 on
+// -1..-0.1, 1.7e-7 both about zero); results differ by single roundings.  fp32 kernels with one column tile per wave, which stream their
 // weights through the compiler's own schedule, keep the terms (PONNI_GELU_TERMS,
 // fused.cpp): 25-308-14 residual chain of three blocks, 131,072 columns, 1685 us
 // with them, 2909 with the polynomial; 61-338-34 4970 against 5238.
